@@ -43,6 +43,23 @@ enum : uint32_t {
   TAG_RESAMPLE = 0x14,
 };
 
+__host__ __device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);  // one instruction; left to itself, two
+#else
+  return a ^ b ^ c;
+#endif
+}
+
+// One round of Philox4x32-10; ten rounds, the key raised by the Weyl
+// constants between them, give philox4x32_10.
+__host__ __device__ __forceinline__ void philox_round(uint4 &c, uint32_t k0, uint32_t k1) {
+  const uint64_t p0 = (uint64_t)kPhiloxM0 * c.x;
+  const uint64_t p1 = (uint64_t)kPhiloxM1 * c.z;
+  c = make_uint4(xor3((uint32_t)(p1 >> 32), c.y, k0), (uint32_t)p1,
+                 xor3((uint32_t)(p0 >> 32), c.w, k1), (uint32_t)p0);
+}
+
 __host__ __device__ __forceinline__ uint4 philox4x32_10(uint4 c, uint32_t k0, uint32_t k1) {
 #pragma unroll
   for (int r = 0; r < 10; ++r) {
@@ -50,10 +67,7 @@ __host__ __device__ __forceinline__ uint4 philox4x32_10(uint4 c, uint32_t k0, ui
       k0 += kPhiloxW0;
       k1 += kPhiloxW1;
     }
-    const uint64_t p0 = (uint64_t)kPhiloxM0 * c.x;
-    const uint64_t p1 = (uint64_t)kPhiloxM1 * c.z;
-    c = make_uint4((uint32_t)(p1 >> 32) ^ c.y ^ k0, (uint32_t)p1,
-                   (uint32_t)(p0 >> 32) ^ c.w ^ k1, (uint32_t)p0);
+    philox_round(c, k0, k1);
   }
   return c;
 }
@@ -66,15 +80,20 @@ __host__ __device__ __forceinline__ uint32_t pick(const uint4 &v, uint32_t i) {
 // u = m * 2^e with m in [sqrt(1/2), sqrt(2)); ln(1+f), f = m - 1, is
 // f + f^2 * P(f) with P a degree-6 least-squares fit (relative error
 // <= 2.2e-7 over the interval).  Each step is exact or one correctly rounded
-// fp32 operation, so host and device results agree bit for bit.
+// fp32 operation, so host and device results agree bit for bit.  The bits of
+// w that make u, converted in place, are 2^32 u exactly; taking the bits of
+// 2^32 sqrt(1/2) off leaves e above the 23 mantissa bits and the offset of m
+// from sqrt(1/2) in them, so m and e cost five integer operations.
 __host__ __device__ __forceinline__ float neg_ln_u(uint32_t w) {
-  const float u = (float)((w >> 9) * 2u + 1u) * 0x1p-24f;
-  int e;
-  float m = frexpf(u, &e);
-  if (m < 0x1.6a09e6p-1f) {
-    m = m + m;
-    e = e - 1;
-  }
+  constexpr uint32_t kSqrtHalf = 0x3F3504F3u;
+  const float v = (float)((w & 0xFFFFFE00u) | 0x100u);
+  uint32_t ix;
+  __builtin_memcpy(&ix, &v, 4);
+  ix -= kSqrtHalf + (32u << 23);
+  const int e = (int)ix >> 23;
+  const uint32_t mb = (ix & 0x007FFFFFu) + kSqrtHalf;
+  float m;
+  __builtin_memcpy(&m, &mb, 4);
   const float f = m - 1.0f;
   float p = -0x1.9190e0p-4f;
   p = fmaf(p, f, 0x1.4953eep-3f);

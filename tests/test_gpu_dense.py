@@ -44,6 +44,26 @@ def test_dense_integer_instances_match_oracle_bit_for_bit(ctx, n, R, S, refresh)
     assert out["best_energy"] == be[i] and (out["best_state"] == bs[i]).all()
 
 
+@pytest.mark.parametrize("n", [1, 16, 17, 64, 65, 128, 129, 257, 385, 512, 513, 640, 769, 1024])
+def test_dense_blocks_and_tiles(ctx, n):
+    """Sizes at the edges of a block (16 spins), of a turn of the waves (64)
+    and of the padded tile counts (multiples of 128), with one sweep per
+    segment as well, a second instance and 64 + 1 replicas: bit for bit."""
+    R, S = 65, 3
+    qs = np.stack([_int_instance(n, 31), _int_instance(n, 32)])
+    ts = _tscale(S, 0.05, 1.0)
+    print(f"[gpu] dense blocks n={n}", flush=True)
+    b = onesolver_amd.DenseBatch(ctx, qs)
+    for refresh in (0, 1):
+        out = b.anneal(R, ts, seed=19, instance=6, refresh_interval=refresh, final_states=True)
+        for i in range(2):
+            fin, bs, be = oracle.sweep_dense(qs[i], n, ts, R, seed=19, instance=6 + i)
+            assert (out["final_states"][i] == fin).all()
+            assert (out["best_states"][i] == bs).all()
+            assert np.array_equal(out["best_energies"][i], be)
+    b.close()
+
+
 def test_dense_sk_real_valued(ctx):
     n, R, S = 256, 512, 200
     q32, _ = instances.sk_qubo(n, seed=1, instance=0)
