@@ -10,36 +10,11 @@
 #include "os_ctx.h"
 #include "os_dense.h"
 #include "os_kernels.h"
+#include "os_mpnn.h"
 
 namespace os {
 
-void mp_launch_features(hipStream_t st, int B, int n, int Np, const double *q, double *rowstat,
-                        double *scale, uint16_t *A, float *X0, uint16_t *XT0);
-void mp_launch_agg(hipStream_t st, int B, int Np, const uint16_t *A, const uint16_t *XT, float *Y,
-                   bool accumulate);
-void mp_launch_node_fwd(hipStream_t st, int B, int Np, const float *Hin, const float *M,
-                        const float *wl, float *Z, float *H, uint16_t *HT);
-void mp_launch_node_bwd(hipStream_t st, int B, int Np, const float *dH, const float *Z,
-                        const float *wl, float *dZ, float *dHprev, uint16_t *dMsgT);
-void mp_launch_head(hipStream_t st, int B, int n, int Np, const float *H3, const float *wo,
-                    const uint8_t *labels, float inv_count, float *p, double *lossterm,
-                    float *dlogit, float *dH3);
-void mp_launch_wgrad(hipStream_t st, int rows, int W, const float *X, const float *G,
-                     float *partial, float *grad_w, float *grad_b);
-void mp_launch_loss_sum(hipStream_t st, size_t count, const double *terms, double *out);
-void mp_launch_adam(hipStream_t st, int P, const float *grad, const uint8_t *kind, float *w,
-                    float *m, float *v, float *wc, float lr, float b1, float b2, float eps,
-                    int step);
-void mp_launch_csr_features(hipStream_t st, int I, int max_n, const CsrInst *inst,
-                            const int32_t *row_ptr, const double *val, const double *diag,
-                            const int32_t *scale_rows, double *scale, float *X0);
-void mp_launch_csr_agg(hipStream_t st, int I, int max_n, const CsrInst *inst,
-                       const int32_t *row_ptr, const int32_t *col, const double *val,
-                       const double *scale, const float *Hin, float *M);
 CsrView csr_view(os_csr_batch *b, Ctx **ctx);
-void mp_launch_compute_copy(hipStream_t st, int P, const uint8_t *kind, const float *w,
-                            float *wc);
-
 namespace {
 
 constexpr int kF0 = 4, kHid = 64, kLayers = 3;
@@ -73,15 +48,18 @@ struct Mpnn {
   int step = 0;
   DevBuf w, wc, grad, m, v, kind;
   int B = 0, Np = 0;
-  DevBuf rowstat, scale, A, X0, XT0, HT[kLayers], M[kLayers], Z[kLayers], H[kLayers];
-  DevBuf p, lossterm, dlogit, dH, dHprev, dZ, dMsgT, partial, lossout, labels;
+  DevBuf rowstat, scale, A, X0, XT0, HT[kLayers - 1], M[kLayers], Z[kLayers], H[kLayers - 1];
+  DevBuf p, dlogit, lossblock, dH[2], dMsgT[2], partial, head_partial, lossout, labels;
   DevBuf srows;  // sparse batches: the rows of each instance's scale
   ~Mpnn() {
-    for (auto *b : {&w, &wc, &grad, &m, &v, &kind, &rowstat, &scale, &A, &X0, &XT0, &p, &lossterm,
-                    &dlogit, &dH, &dHprev, &dZ, &dMsgT, &partial, &lossout, &labels, &srows})
+    for (auto *b : {&w, &wc, &grad, &m, &v, &kind, &rowstat, &scale, &A, &X0, &XT0, &p, &dlogit,
+                    &lossblock, &dH[0], &dH[1], &dMsgT[0], &dMsgT[1], &partial, &head_partial,
+                    &lossout, &labels, &srows})
       b->release();
-    for (int l = 0; l < kLayers; ++l)
-      for (auto *b : {&HT[l], &M[l], &Z[l], &H[l]}) b->release();
+    for (auto &b : M) b.release();
+    for (auto &b : Z) b.release();
+    for (auto &b : H) b.release();
+    for (auto &b : HT) b.release();
   }
 
   void shape(int b, int np) {
@@ -91,27 +69,31 @@ struct Mpnn {
     A.ensure(sizeof(uint16_t) * rows * np);
     X0.ensure(sizeof(float) * rows * 64);
     XT0.ensure(sizeof(uint16_t) * rows * 64);
-    for (int l = 0; l < kLayers; ++l) {
-      HT[l].ensure(sizeof(uint16_t) * rows * 64);
-      M[l].ensure(sizeof(float) * rows * 64);
-      Z[l].ensure(sizeof(float) * rows * 64);
-      H[l].ensure(sizeof(float) * rows * 64);
-    }
+    for (auto &x : HT) x.ensure(sizeof(uint16_t) * rows * 64);
+    for (auto &x : M) x.ensure(sizeof(float) * rows * 64);
+    for (auto &x : Z) x.ensure(sizeof(float) * rows * 64);
+    for (auto &x : H) x.ensure(sizeof(float) * rows * 64);
     p.ensure(sizeof(float) * rows);
-    lossterm.ensure(sizeof(double) * rows);
     dlogit.ensure(sizeof(float) * rows);
-    dH.ensure(sizeof(float) * rows * 64);
-    dHprev.ensure(sizeof(float) * rows * 64);
-    dZ.ensure(sizeof(float) * rows * 64);
-    dMsgT.ensure(sizeof(uint16_t) * rows * 64);
-    partial.ensure(sizeof(float) * (rows / 64) * 65 * 64);
+    lossblock.ensure(sizeof(double) * (rows / 64));
     lossout.ensure(sizeof(double));
     B = b;
     Np = np;
   }
 
+  MpHead head(const uint8_t *dev_labels, float inv_count) const {
+    MpHead h;
+    h.wo = wc.as<float>() + kWo;
+    h.labels = dev_labels;
+    h.inv_count = inv_count;
+    h.p = p.as<float>();
+    h.dlogit = dlogit.as<float>();
+    h.lossblock = lossblock.as<double>();
+    return h;
+  }
+
   // forward pass over instances [first, first+count) of d; with labels, the
-  // loss terms, dlogit and dH3 as well
+  // loss terms and dlogit as well
   void forward(const Dense &d, int first, int count, const uint8_t *dev_labels) {
     const int n = d.n, np = (n + 63) / 64 * 64;
     shape(count, np);
@@ -119,17 +101,16 @@ struct Mpnn {
     const double *q = d.q64.as<double>() + (size_t)first * n * n;
     mp_launch_features(st, count, n, np, q, rowstat.as<double>(), scale.as<double>(),
                        A.as<uint16_t>(), X0.as<float>(), XT0.as<uint16_t>());
+    const MpHead h = head(dev_labels, 1.0f / ((float)count * (float)n));
     for (int l = 0; l < kLayers; ++l) {
-      const float *hin = l == 0 ? X0.as<float>() : H[l - 1].as<float>();
-      const uint16_t *hint = l == 0 ? XT0.as<uint16_t>() : HT[l - 1].as<uint16_t>();
-      mp_launch_agg(st, count, np, A.as<uint16_t>(), hint, M[l].as<float>(), false);
-      mp_launch_node_fwd(st, count, np, hin, M[l].as<float>(), wc.as<float>() + l * kLayerStride,
-                         Z[l].as<float>(), H[l].as<float>(),
-                         l + 1 < kLayers ? HT[l].as<uint16_t>() : nullptr);
+      const bool last = l + 1 == kLayers;
+      mp_launch_layer_fwd(st, count, n, np, A.as<uint16_t>(),
+                          l == 0 ? XT0.as<uint16_t>() : HT[l - 1].as<uint16_t>(),
+                          l == 0 ? X0.as<float>() : H[l - 1].as<float>(), M[l].as<float>(),
+                          wc.as<float>() + l * kLayerStride, Z[l].as<float>(),
+                          last ? nullptr : H[l].as<float>(),
+                          last ? nullptr : HT[l].as<uint16_t>(), last ? &h : nullptr);
     }
-    mp_launch_head(st, count, n, np, H[kLayers - 1].as<float>(), wc.as<float>() + kWo, dev_labels,
-                   1.0f / ((float)count * (float)n), p.as<float>(), lossterm.as<double>(),
-                   dlogit.as<float>(), dH.as<float>());
   }
 
   // forward pass over a sparse batch (marginals in p, one row per spin);
@@ -139,12 +120,11 @@ struct Mpnn {
     hipStream_t st = ctx->stream;
     scale.ensure(sizeof(double) * std::max(v.num_instances, 1));
     X0.ensure(sizeof(float) * rows * 64);
-    for (int l = 0; l < kLayers; ++l) {
-      M[l].ensure(sizeof(float) * rows * 64);
-      Z[l].ensure(sizeof(float) * rows * 64);
-      H[l].ensure(sizeof(float) * rows * 64);
-    }
+    for (auto &x : M) x.ensure(sizeof(float) * rows * 64);
+    for (auto &x : Z) x.ensure(sizeof(float) * rows * 64);
+    for (auto &x : H) x.ensure(sizeof(float) * rows * 64);
     p.ensure(sizeof(float) * rows);
+    const MpHead h = head(nullptr, 0.0f);
     // padding rows: zero features and messages, so every row the node
     // kernels read is defined
     OS_HIP_CHECK(hipMemsetAsync(X0.ptr, 0, sizeof(float) * rows * 64, st));
@@ -156,13 +136,11 @@ struct Mpnn {
       const float *hin = l == 0 ? X0.as<float>() : H[l - 1].as<float>();
       mp_launch_csr_agg(st, v.num_instances, v.max_n, v.inst, v.row_ptr, v.col, v.val,
                         scale.as<double>(), hin, M[l].as<float>());
-      mp_launch_node_fwd(st, 1, (int)rows, hin, M[l].as<float>(),
-                         wc.as<float>() + l * kLayerStride, Z[l].as<float>(), H[l].as<float>(),
-                         nullptr);
+      const bool last = l + 1 == kLayers;
+      mp_launch_layer_fwd(st, 1, (int)rows, (int)rows, nullptr, nullptr, hin, M[l].as<float>(),
+                          wc.as<float>() + l * kLayerStride, Z[l].as<float>(),
+                          last ? nullptr : H[l].as<float>(), nullptr, last ? &h : nullptr);
     }
-    mp_launch_head(st, 1, (int)rows, (int)rows, H[kLayers - 1].as<float>(),
-                   wc.as<float>() + kWo, nullptr, 0.0f, p.as<float>(), nullptr, nullptr,
-                   nullptr);
     // the next dense forward re-shapes its buffers from scratch
     B = 0;
     Np = 0;
@@ -172,28 +150,31 @@ struct Mpnn {
   // labels must have run
   void backward() {
     hipStream_t st = ctx->stream;
-    const int rows = B * Np;
-    float *g = grad.as<float>();
-    mp_launch_wgrad(st, rows, 1, H[kLayers - 1].as<float>(), dlogit.as<float>(),
-                    partial.as<float>(), g + kWo, g + kBo);
-    for (int l = kLayers - 1; l >= 0; --l) {
-      const float *wl = wc.as<float>() + l * kLayerStride;
-      mp_launch_node_bwd(st, B, Np, dH.as<float>(), Z[l].as<float>(), wl, dZ.as<float>(),
-                         l > 0 ? dHprev.as<float>() : nullptr, dMsgT.as<uint16_t>());
-      const float *hin = l == 0 ? X0.as<float>() : H[l - 1].as<float>();
-      mp_launch_wgrad(st, rows, 64, hin, dZ.as<float>(), partial.as<float>(),
-                      g + l * kLayerStride, g + l * kLayerStride + 8192);
-      mp_launch_wgrad(st, rows, 64, M[l].as<float>(), dZ.as<float>(), partial.as<float>(),
-                      g + l * kLayerStride + 4096, nullptr);
-      if (l > 0) {
-        mp_launch_agg(st, B, Np, A.as<uint16_t>(), dMsgT.as<uint16_t>(), dHprev.as<float>(), true);
-        std::swap(dH, dHprev);
-      }
+    const size_t rows = (size_t)B * Np, groups = rows / 64;
+    for (int k = 0; k < 2; ++k) {
+      dH[k].ensure(sizeof(float) * rows * 64);
+      dMsgT[k].ensure(sizeof(uint16_t) * rows * 64);
     }
+    partial.ensure(sizeof(float) * kLayers * groups * kLayerStride);
+    head_partial.ensure(sizeof(float) * groups * 65);
+    const MpHead h = head(labels.as<uint8_t>(), 0.0f);
+    for (int l = kLayers - 1; l >= 0; --l) {
+      const int in = l & 1, out = in ^ 1;  // the layer above wrote the buffers of its `out`
+      mp_launch_layer_bwd(st, B, Np, A.as<uint16_t>(), dMsgT[in].as<uint16_t>(),
+                          dH[in].as<float>(), l + 1 == kLayers ? &h : nullptr, Z[l].as<float>(),
+                          wc.as<float>() + l * kLayerStride,
+                          l == 0 ? X0.as<float>() : H[l - 1].as<float>(), M[l].as<float>(),
+                          l > 0 ? dH[out].as<float>() : nullptr, dMsgT[out].as<uint16_t>(),
+                          partial.as<float>() + (size_t)l * groups * kLayerStride,
+                          head_partial.as<float>());
+    }
+    mp_launch_grad_sum(st, kLayers, (int)groups, partial.as<float>(), head_partial.as<float>(),
+                       grad.as<float>());
   }
 
   double loss_value(int count, int n) {
-    mp_launch_loss_sum(ctx->stream, (size_t)B * Np, lossterm.as<double>(), lossout.as<double>());
+    mp_launch_loss_sum(ctx->stream, (size_t)B * Np / 64, lossblock.as<double>(),
+                       lossout.as<double>());
     double s = 0.0;
     OS_HIP_CHECK(hipMemcpyAsync(&s, lossout.ptr, sizeof(double), hipMemcpyDeviceToHost,
                                 ctx->stream));

@@ -14,9 +14,13 @@
 //
 // Activations of a minibatch of B instances live in [B][Np][64] fp32 arrays
 // (row = spin) and, as MFMA B operands, in [B][64][Np] bf16 (feature-major).
-// Weight gradients are reduced deterministically: fixed 64-row chunks, then
-// the chunk partials in order.
-#include "os_kernels.h"
+// A layer is one launch in each direction, a work-group 64 rows of one
+// instance: the aggregation's 64 x 64 tile goes through LDS straight into the
+// node update (forward) or the activation's gradient (backward), and the
+// backward launch also makes the rows' share of the weight gradients.  Those
+// are reduced deterministically: rows of a work-group in order, then the
+// work-groups in a fixed tree.
+#include "os_mpnn.h"
 
 namespace os {
 
@@ -40,54 +44,79 @@ __device__ __forceinline__ float bf16_round(float f) {
 
 // ---- features --------------------------------------------------------------
 
-// rowstat[b][i] = (sum_{j != i} Q_ij^2, sum_{j != i} Q_ij) of instance q[b]
+// rowstat[b][i] = (sum_{j != i} Q_ij^2, sum_{j != i} Q_ij) of instance q[b]:
+// one wave per row, so the FP64 matrices are read once in 512-byte requests
+// (one thread per row, 8 KB apart, took 146 us for 16 x n=1024; 33 us now).
 __global__ __launch_bounds__(256) void mp_rowstat_kernel(int B, int n, const double *__restrict__ q,
                                                          double *__restrict__ rowstat) {
-  const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
+  const size_t t = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (t >= (size_t)B * n) return;
-  const int b = (int)(t / n), i = (int)(t % n);
-  const double *row = q + ((size_t)b * n + i) * n;
+  const int i = (int)(t % n), lane = threadIdx.x & 63;
+  const double *row = q + t * n;
   double s2 = 0.0, s1 = 0.0;
-  for (int j = 0; j < n; ++j) {
-    if (j == i) continue;
-    const double v = row[j];
-    s2 += v * v;
+#pragma unroll 4
+  for (int j = lane; j < n; j += 64) {
+    const double v = j == i ? 0.0 : row[j];
+    s2 = fma(v, v, s2);
     s1 += v;
   }
-  rowstat[2 * t] = s2;
-  rowstat[2 * t + 1] = s1;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    s2 += __shfl_xor(s2, o);
+    s1 += __shfl_xor(s1, o);
+  }
+  if (lane == 0) {
+    rowstat[2 * t] = s2;
+    rowstat[2 * t + 1] = s1;
+  }
 }
 
-__global__ void mp_scale_kernel(int B, int n, const double *__restrict__ rowstat,
-                                double *__restrict__ scale) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= B) return;
+__global__ __launch_bounds__(256) void mp_scale_kernel(int n, const double *__restrict__ rowstat,
+                                                       double *__restrict__ scale) {
+  __shared__ double part[256];
+  const int b = blockIdx.x;
   double s = 0.0;
-  for (int i = 0; i < n; ++i) s += rowstat[2 * ((size_t)b * n + i)];
-  s = sqrt(s / n);
-  scale[b] = s > 0.0 ? s : 1.0;
+  for (int i = threadIdx.x; i < n; i += 256) s += rowstat[2 * ((size_t)b * n + i)];
+  part[threadIdx.x] = s;
+  __syncthreads();
+  for (int h = 128; h > 0; h >>= 1) {
+    if ((int)threadIdx.x < h) part[threadIdx.x] += part[threadIdx.x + h];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    s = sqrt(part[0] / n);
+    scale[b] = s > 0.0 ? s : 1.0;
+  }
 }
 
-// A[b][i][j] (bf16) and the features X0[b][i][:], XT0[b][:][i] (bf16)
+// A[b][i][j] (bf16) and the features X0[b][i][:], XT0[b][:][i] (bf16).  A
+// work-group is one row.  The quotient by the scale is formed from its
+// reciprocal with one correction by the remainder: three products instead of
+// a division's sequence per coupling.
 __global__ __launch_bounds__(256) void mp_fill_kernel(int n, int Np, const double *__restrict__ q,
                                                       const double *__restrict__ rowstat,
                                                       const double *__restrict__ scale,
                                                       uint16_t *__restrict__ A,
                                                       float *__restrict__ X0,
                                                       uint16_t *__restrict__ XT0) {
-  const int b = blockIdx.y;
-  const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (t >= (size_t)Np * Np) return;
-  const int i = (int)(t / Np), j = (int)(t % Np);
-  const double sc = scale[b];
-  const double *qb = q + (size_t)b * n * n;
-  float a = 0.0f;
-  if (i < n && j < n && i != j) a = (float)(qb[(size_t)i * n + j] / sc);
-  A[(size_t)b * Np * Np + t] = to_bf16(a);
+  const int b = blockIdx.y, i = blockIdx.x;
+  const double sc = scale[b], rc = 1.0 / sc;
+  const double *row = q + ((size_t)b * n + i) * n;
+  uint16_t *a = A + ((size_t)b * Np + i) * Np;
+  for (int j = threadIdx.x; j < Np; j += 256) {
+    float v = 0.0f;
+    if (i < n && j < n && i != j) {
+      const double x = row[j], t = x * rc;
+      v = (float)fma(fma(-t, sc, x), rc, t);
+      if (!isfinite(v)) v = (float)(x / sc);  // the remainder of an infinity is NaN
+    }
+    a[j] = to_bf16(v);
+  }
+  const int j = threadIdx.x;
   if (j < 64) {
     float f = 0.0f;
     if (i < n) {
-      if (j == 0) f = (float)(qb[(size_t)i * n + i] / sc);
+      if (j == 0) f = (float)(row[i] / sc);
       else if (j == 1) f = (float)(rowstat[2 * ((size_t)b * n + i) + 1] / sc);
       else if (j == 2) f = i == 0 ? 1.0f : 0.0f;
       else if (j == 3) f = 1.0f;
@@ -191,130 +220,223 @@ void mp_launch_csr_agg(hipStream_t st, int I, int max_n, const CsrInst *inst,
   OS_HIP_CHECK(hipGetLastError());
 }
 
-// ---- neighbour aggregation: Y[b] (+)= A[b] . X[b], X given feature-major bf16
-template <bool kAcc>
-__global__ __launch_bounds__(256) void mp_agg_kernel(int Np, const uint16_t *__restrict__ A,
-                                                     const uint16_t *__restrict__ XT,
-                                                     float *__restrict__ Y) {
-  const int b = blockIdx.y;
+// ---- layers ------------------------------------------------------------------
+namespace {
+
+constexpr int kRows = 64;  // rows of a work-group
+constexpr int kLd = 68;    // row stride of the LDS tiles: 16-byte rows, no bank conflicts
+constexpr int kUnroll = 4;  // aggregation: k steps (of 16) requested at once, twice
+
+typedef float Tile[kRows][kLd];
+
+__device__ __forceinline__ void load_tile(Tile &dst, const float *__restrict__ src) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int idx = threadIdx.x + 256 * k;
+    *reinterpret_cast<float4 *>(&dst[idx >> 4][4 * (idx & 15)]) =
+        reinterpret_cast<const float4 *>(src)[idx];
+  }
+}
+
+// Rows r0.. of A . X (A row-major, X feature-major, both bf16, fp32 sums) into
+// y: wave w makes rows 32 (w/2).. x features 32 (w%2)...  Four k steps are in
+// flight while four are multiplied; requested one by one, each step waited
+// for L2 (19 us a layer at 16 x n=1024, of which now 8).
+__device__ __forceinline__ void agg_tile(int Np, const uint16_t *__restrict__ A,
+                                         const uint16_t *__restrict__ XT, int r0, Tile &y) {
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int lc = lane & 31, kh = lane >> 5;
-  const int r0 = blockIdx.x * 64 + 32 * (w >> 1);
-  const int f0 = 32 * (w & 1);
-  const uint4 *arow = reinterpret_cast<const uint4 *>(A + ((size_t)b * Np + r0 + lc) * Np) + kh;
-  const uint4 *xrow = reinterpret_cast<const uint4 *>(XT + ((size_t)b * 64 + f0 + lc) * Np) + kh;
+  const int rw = 32 * (w >> 1), f0 = 32 * (w & 1);
+  const uint4 *arow = reinterpret_cast<const uint4 *>(A + (size_t)(r0 + rw + lc) * Np) + kh;
+  const uint4 *xrow = reinterpret_cast<const uint4 *>(XT + (size_t)(f0 + lc) * Np) + kh;
   mp_f32x16 acc;
 #pragma unroll
   for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
-  const int steps = Np / 16;
-  for (int s = 0; s < steps; ++s) {
-    const uint4 a = arow[2 * s];
-    const uint4 x = xrow[2 * s];
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(mp_bf16x8, a),
-                                                  __builtin_bit_cast(mp_bf16x8, x), acc, 0, 0,
-                                                  0);
+  const int steps = Np / 16;  // a multiple of kUnroll: Np is one of 64
+  uint4 a[kUnroll], x[kUnroll];
+#pragma unroll
+  for (int u = 0; u < kUnroll; ++u) {
+    a[u] = arow[2 * u];
+    x[u] = xrow[2 * u];
+  }
+  for (int s = kUnroll; s <= steps; s += kUnroll) {
+    uint4 a1[kUnroll], x1[kUnroll];
+    const int sn = min(s, steps - kUnroll);  // past the end: the last steps again, unused
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      a1[u] = arow[2 * (sn + u)];
+      x1[u] = xrow[2 * (sn + u)];
+    }
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u)
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(mp_bf16x8, a[u]),
+                                                    __builtin_bit_cast(mp_bf16x8, x[u]), acc, 0,
+                                                    0, 0);
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      a[u] = a1[u];
+      x[u] = x1[u];
+    }
   }
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int row = r0 + 8 * (i >> 2) + 4 * kh + (i & 3);
-    float *y = Y + ((size_t)b * Np + row) * 64 + f0 + lc;
-    if (kAcc)
-      *y += acc[i];
-    else
-      *y = acc[i];
+  for (int i = 0; i < 16; ++i) y[rw + 8 * (i >> 2) + 4 * kh + (i & 3)][f0 + lc] = acc[i];
+}
+
+// c[i][j] += sum_k x[tr + 16 i][k] w[k][4 to + j] in order of k, for this
+// thread's 4 x 4 part (tr = tid % 16, to = tid / 16): eight 16-byte reads for
+// 64 products.
+__device__ __forceinline__ void rows_times(const Tile &x, const Tile &w, int tr, int to,
+                                           float (&c)[4][4]) {
+  for (int k = 0; k < 64; k += 4) {
+    float xv[4][4], wv[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      *reinterpret_cast<float4 *>(xv[i]) = *reinterpret_cast<const float4 *>(&x[tr + 16 * i][k]);
+      *reinterpret_cast<float4 *>(wv[i]) = *reinterpret_cast<const float4 *>(&w[k + i][4 * to]);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) c[i][j] = fmaf(xv[i][u], wv[u][j], c[i][j]);
   }
 }
 
-// ---- node update -----------------------------------------------------------
-constexpr int kRowsPerGroup = 16;
+// c[i][j] += sum_k x[tr + 16 i][k] w[4 to + j][k] in order of k.
+__device__ __forceinline__ void rows_times_t(const Tile &x, const Tile &w, int tr, int to,
+                                             float (&c)[4][4]) {
+  for (int k = 0; k < 64; k += 4) {
+    float xv[4][4], wv[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      *reinterpret_cast<float4 *>(xv[i]) = *reinterpret_cast<const float4 *>(&x[tr + 16 * i][k]);
+      *reinterpret_cast<float4 *>(wv[i]) = *reinterpret_cast<const float4 *>(&w[4 * to + i][k]);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) c[i][j] = fmaf(xv[i][u], wv[j][u], c[i][j]);
+  }
+}
 
-// Z = Hin Ws + M Wm + b, H = relu(Z), HT = bf16(H) feature-major (optional)
-__global__ __launch_bounds__(256) void mp_node_fwd_kernel(
-    int Np, const float *__restrict__ Hin, const float *__restrict__ M,
-    const float *__restrict__ wl, float *__restrict__ Z, float *__restrict__ H,
-    uint16_t *__restrict__ HT) {
-  __shared__ float ws[64][64], wm[64][64], bias[64];
-  __shared__ float xs[kRowsPerGroup][64], ms[kRowsPerGroup][64];
-  const int b = blockIdx.y;
-  const int tid = threadIdx.x;
-  for (int k = tid; k < 4096; k += 256) {
-    ws[k >> 6][k & 63] = wl[k];
-    wm[k >> 6][k & 63] = wl[4096 + k];
+// out[a][o] = sum_r x[r][a] g[r][o] in order of r (a = 4 (tid / 16).., o = 4 (tid % 16)..).
+__device__ __forceinline__ void cols_times(const Tile &x, const Tile &g, float *__restrict__ out) {
+  const int ta = threadIdx.x >> 4, to = threadIdx.x & 15;
+  float c[4][4] = {};
+#pragma unroll 4
+  for (int r = 0; r < kRows; ++r) {
+    float xv[4], gv[4];
+    *reinterpret_cast<float4 *>(xv) = *reinterpret_cast<const float4 *>(&x[r][4 * ta]);
+    *reinterpret_cast<float4 *>(gv) = *reinterpret_cast<const float4 *>(&g[r][4 * to]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) c[i][j] = fmaf(xv[i], gv[j], c[i][j]);
   }
-  if (tid < 64) bias[tid] = wl[8192 + tid];
-  const size_t row0 = (size_t)b * Np + (size_t)blockIdx.x * kRowsPerGroup;
-  for (int k = tid; k < kRowsPerGroup * 64; k += 256) {
-    xs[k >> 6][k & 63] = Hin[row0 * 64 + k];
-    ms[k >> 6][k & 63] = M[row0 * 64 + k];
-  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    *reinterpret_cast<float4 *>(out + (4 * ta + i) * 64 + 4 * to) =
+        make_float4(c[i][0], c[i][1], c[i][2], c[i][3]);
+}
+
+// bf16 of a thread's 4 x 4 part (rows tr + 16 i, features 4 to + j) into the
+// feature-major array xt at row r0 of its instance, through LDS so that the
+// stores are 16 bytes.  t: 64 x 72 bf16 of LDS nobody reads any more.
+__device__ __forceinline__ void store_feature_major(const float (&c)[4][4], int tr, int to,
+                                                    uint16_t (*t)[72], int Np, int r0,
+                                                    uint16_t *__restrict__ xt) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) t[4 * to + j][tr + 16 * i] = to_bf16(c[i][j]);
   __syncthreads();
-  const int o = tid & 63;
-  for (int r = tid >> 6; r < kRowsPerGroup; r += 4) {
-    float z = bias[o];
-    for (int a = 0; a < 64; ++a) z = fmaf(xs[r][a], ws[a][o], z);
-    for (int a = 0; a < 64; ++a) z = fmaf(ms[r][a], wm[a][o], z);
-    const size_t row = row0 + r;
-    Z[row * 64 + o] = z;
-    const float h = fmaxf(z, 0.0f);
-    H[row * 64 + o] = h;
-    if (HT) {
-      const int i = (int)(row - (size_t)b * Np);
-      HT[((size_t)b * 64 + o) * Np + i] = to_bf16(h);
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int idx = threadIdx.x + 256 * k;
+    *reinterpret_cast<uint4 *>(xt + (size_t)(idx >> 3) * Np + r0 + 8 * (idx & 7)) =
+        *reinterpret_cast<const uint4 *>(&t[idx >> 3][8 * (idx & 7)]);
+  }
+}
+
+}  // namespace
+
+// Forward: M = A r(Hin) (kAgg: from XT, also stored; otherwise M is given),
+// Z = Hin Ws + M Wm + b, H = relu(Z), HT = bf16(H) feature-major.  kHead: the
+// last layer -- instead of H and HT the head: logit = bo + H wo, p =
+// sigmoid(logit) and, with labels, dlogit and the work-group's sum of BCE
+// terms.  Canonical labels: y_i = x_i xor (1 - x_0) (spin 0 is pinned to 1).
+template <bool kAgg, bool kHead>
+__global__ __launch_bounds__(256) void mp_layer_fwd_kernel(
+    int n, int Np, const uint16_t *__restrict__ A, const uint16_t *__restrict__ XT,
+    const float *__restrict__ Hin, float *__restrict__ M, const float *__restrict__ wl,
+    float *__restrict__ Z, float *__restrict__ H, uint16_t *__restrict__ HT,
+    const float *__restrict__ wo, const uint8_t *__restrict__ labels, float inv_count,
+    float *__restrict__ p, float *__restrict__ dlogit, double *__restrict__ lossblock) {
+  __shared__ __align__(16) Tile ws, wm, xs, ms;
+  const int b = blockIdx.y, r0 = blockIdx.x * kRows;
+  const size_t row0 = (size_t)b * Np + r0;
+  load_tile(ws, wl);
+  load_tile(wm, wl + 4096);
+  load_tile(xs, Hin + row0 * 64);
+  if (kAgg)
+    agg_tile(Np, A + (size_t)b * Np * Np, XT + (size_t)b * 64 * Np, r0, ms);
+  else
+    load_tile(ms, M + row0 * 64);
+  __syncthreads();
+  if (kAgg) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int idx = threadIdx.x + 256 * k;
+      reinterpret_cast<float4 *>(M + row0 * 64)[idx] =
+          *reinterpret_cast<const float4 *>(&ms[idx >> 4][4 * (idx & 15)]);
     }
   }
-}
-
-// dZ = dH * (Z > 0); dHprev = dZ Ws^T; dMsgT = bf16(dZ Wm^T) feature-major
-__global__ __launch_bounds__(256) void mp_node_bwd_kernel(
-    int Np, const float *__restrict__ dH, const float *__restrict__ Z,
-    const float *__restrict__ wl, float *__restrict__ dZ, float *__restrict__ dHprev,
-    uint16_t *__restrict__ dMsgT) {
-  __shared__ float ws[64][65], wm[64][65];
-  __shared__ float dz[kRowsPerGroup][64];
-  const int b = blockIdx.y;
-  const int tid = threadIdx.x;
-  for (int k = tid; k < 4096; k += 256) {
-    ws[k >> 6][k & 63] = wl[k];
-    wm[k >> 6][k & 63] = wl[4096 + k];
+  const int tr = threadIdx.x & 15, to = threadIdx.x >> 4;
+  float z[4][4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const float bias = wl[8192 + 4 * to + j];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) z[i][j] = bias;
   }
-  const size_t row0 = (size_t)b * Np + (size_t)blockIdx.x * kRowsPerGroup;
-  for (int k = tid; k < kRowsPerGroup * 64; k += 256) {
-    const size_t at = row0 * 64 + k;
-    const float g = Z[at] > 0.0f ? dH[at] : 0.0f;
-    dz[k >> 6][k & 63] = g;
-    dZ[at] = g;
+  rows_times(xs, ws, tr, to, z);
+  rows_times(ms, wm, tr, to, z);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const size_t at = (row0 + tr + 16 * i) * 64 + 4 * to;
+    *reinterpret_cast<float4 *>(Z + at) = make_float4(z[i][0], z[i][1], z[i][2], z[i][3]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) z[i][j] = fmaxf(z[i][j], 0.0f);
+    if (!kHead)
+      *reinterpret_cast<float4 *>(H + at) = make_float4(z[i][0], z[i][1], z[i][2], z[i][3]);
   }
+  __syncthreads();  // the tiles are read
+  if (!kHead) {
+    if (HT)
+      store_feature_major(z, tr, to, reinterpret_cast<uint16_t(*)[72]>(&ws[0][0]), Np, r0,
+                          HT + (size_t)b * 64 * Np);
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    *reinterpret_cast<float4 *>(&xs[tr + 16 * i][4 * to]) =
+        make_float4(z[i][0], z[i][1], z[i][2], z[i][3]);
   __syncthreads();
-  if (!dHprev) return;
-  const int a = tid & 63;
-  for (int r = tid >> 6; r < kRowsPerGroup; r += 4) {
-    float s1 = 0.0f, s2 = 0.0f;
-    for (int o = 0; o < 64; ++o) {
-      s1 = fmaf(dz[r][o], ws[a][o], s1);
-      s2 = fmaf(dz[r][o], wm[a][o], s2);
-    }
-    const size_t row = row0 + r;
-    dHprev[row * 64 + a] = s1;
-    const int i = (int)(row - (size_t)b * Np);
-    dMsgT[((size_t)b * 64 + a) * Np + i] = to_bf16(s2);
-  }
-}
-
-// ---- head ------------------------------------------------------------------
-// logit = bo + H3 wo; p = sigmoid; with labels: BCE terms, dlogit and dH3.
-// Canonical labels: y_i = x_i xor (1 - x_0) (spin 0 is pinned to 1).
-__global__ __launch_bounds__(256) void mp_head_kernel(
-    int B, int n, int Np, const float *__restrict__ H3, const float *__restrict__ wo,
-    const uint8_t *__restrict__ labels, float inv_count, float *__restrict__ p,
-    double *__restrict__ lossterm, float *__restrict__ dlogit, float *__restrict__ dH3) {
-  const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (t >= (size_t)B * Np) return;
-  const int b = (int)(t / Np), i = (int)(t % Np);
-  const float *h = H3 + t * 64;
+  if (threadIdx.x >= 64) return;
+  const int r = threadIdx.x, i = r0 + r;
   float l = wo[64];
-  for (int a = 0; a < 64; ++a) l = fmaf(h[a], wo[a], l);
+  for (int a = 0; a < 64; a += 4) {
+    const float4 h = *reinterpret_cast<const float4 *>(&xs[r][a]);
+    l = fmaf(h.x, wo[a], l);
+    l = fmaf(h.y, wo[a + 1], l);
+    l = fmaf(h.z, wo[a + 2], l);
+    l = fmaf(h.w, wo[a + 3], l);
+  }
   const float pr = 1.0f / (1.0f + expf(-l));
-  if (p) p[t] = pr;
+  p[row0 + r] = pr;
   if (!labels) return;
   float g = 0.0f;
   double term = 0.0;
@@ -325,53 +447,117 @@ __global__ __launch_bounds__(256) void mp_head_kernel(
     term = (ld > 0.0 ? ld : 0.0) - ld * (double)y + log1p(exp(-fabs(ld)));
     g = (pr - y) * inv_count;
   }
-  lossterm[t] = term;
-  dlogit[t] = g;
-  for (int a = 0; a < 64; ++a) dH3[t * 64 + a] = g * wo[a];
+  dlogit[row0 + r] = g;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) term += __shfl_xor(term, o);
+  if (r == 0) lossblock[(size_t)b * gridDim.x + blockIdx.x] = term;
 }
 
-// ---- weight gradients --------------------------------------------------------
-// partial[c][a][o] = sum over rows [64c, 64c+64) of X[row][a] * G[row][o]
-// (a = 64: the constant 1, i.e. the bias gradient); W = width of G (64 or 1)
-__global__ __launch_bounds__(256) void mp_wgrad_partial_kernel(int W, const float *__restrict__ X,
-                                                               const float *__restrict__ G,
-                                                               float *__restrict__ partial) {
-  __shared__ float xs[64][65];
-  __shared__ float gs[64][64];
-  const int c = blockIdx.x;
+// Backward: dH is dlogit wo^T (kTop: the last layer) or dHin + A dMsg (the
+// layer above's share through its own rows and through its messages);
+// dZ = dH * (Z > 0); with kPrev dHprev = dZ Ws^T and dMsgT = bf16(dZ Wm^T)
+// feature-major for the layer below.  The 64 rows' weight gradients
+// (Hin^T dZ, M^T dZ, sum dZ, in the layout of the parameters) go to
+// partial[work-group], with kTop those of the head (relu(Z)^T dlogit, sum
+// dlogit) to head_partial[work-group].
+template <bool kTop, bool kPrev>
+__global__ __launch_bounds__(256) void mp_layer_bwd_kernel(
+    int Np, const uint16_t *__restrict__ A, const uint16_t *__restrict__ dMsgTin,
+    const float *__restrict__ dHin, const float *__restrict__ dlogit,
+    const float *__restrict__ wo, const float *__restrict__ Z, const float *__restrict__ wl,
+    const float *__restrict__ Hin, const float *__restrict__ M, float *__restrict__ dHprev,
+    uint16_t *__restrict__ dMsgT, float *__restrict__ partial, float *__restrict__ head_partial) {
+  __shared__ __align__(16) Tile dz, hs, ms;
+  const int b = blockIdx.y, r0 = blockIdx.x * kRows;
+  const size_t row0 = (size_t)b * Np + r0;
+  const size_t wg = (size_t)b * gridDim.x + blockIdx.x;
   const int tid = threadIdx.x;
-  const size_t row0 = (size_t)c * 64;
-  for (int k = tid; k < 64 * 64; k += 256) xs[k >> 6][k & 63] = X[row0 * 64 + k];
-  for (int k = tid; k < 64 * W; k += 256) gs[k / W][k % W] = G[row0 * W + k];
-  __syncthreads();
-  float *out = partial + (size_t)c * 65 * W;
-  for (int idx = tid; idx < 65 * W; idx += 256) {
-    const int a = idx / W, o = idx % W;
-    float s = 0.0f;
-    if (a < 64)
-      for (int r = 0; r < 64; ++r) s = fmaf(xs[r][a], gs[r][o], s);
-    else
-      for (int r = 0; r < 64; ++r) s += gs[r][o];
-    out[idx] = s;
+  if (kTop) {
+    load_tile(hs, Z + row0 * 64);
+    __syncthreads();
+    if (tid < 65) {
+      float s = 0.0f;
+      for (int r = 0; r < kRows; ++r) {
+        const float g = dlogit[row0 + r];
+        s = tid < 64 ? fmaf(fmaxf(hs[r][tid], 0.0f), g, s) : s + g;
+      }
+      head_partial[wg * 65 + tid] = s;
+    }
+    for (int k = tid; k < kRows * 64; k += 256) {
+      const int r = k >> 6, o = k & 63;
+      dz[r][o] = hs[r][o] > 0.0f ? dlogit[row0 + r] * wo[o] : 0.0f;
+    }
+    __syncthreads();  // hs is read
+  } else {
+    agg_tile(Np, A + (size_t)b * Np * Np, dMsgTin + (size_t)b * 64 * Np, r0, dz);
+    __syncthreads();
+    for (int k = tid; k < kRows * 64; k += 256) {
+      const int r = k >> 6, o = k & 63;
+      dz[r][o] = Z[row0 * 64 + k] > 0.0f ? dHin[row0 * 64 + k] + dz[r][o] : 0.0f;
+    }
   }
+  load_tile(hs, Hin + row0 * 64);
+  load_tile(ms, M + row0 * 64);
+  __syncthreads();
+  float *out = partial + wg * 8256;
+  cols_times(hs, dz, out);
+  cols_times(ms, dz, out + 4096);
+  if (tid < 64) {
+    float s = 0.0f;
+    for (int r = 0; r < kRows; ++r) s += dz[r][tid];
+    out[8192 + tid] = s;
+  }
+  if (!kPrev) return;
+  __syncthreads();  // hs and ms are read: they take the weights
+  load_tile(hs, wl);
+  load_tile(ms, wl + 4096);
+  __syncthreads();
+  const int tr = tid & 15, to = tid >> 4;
+  float c[4][4] = {};
+  rows_times_t(dz, hs, tr, to, c);
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    *reinterpret_cast<float4 *>(dHprev + (row0 + tr + 16 * i) * 64 + 4 * to) =
+        make_float4(c[i][0], c[i][1], c[i][2], c[i][3]);
+  float e[4][4] = {};
+  rows_times_t(dz, ms, tr, to, e);
+  __syncthreads();
+  store_feature_major(e, tr, to, reinterpret_cast<uint16_t(*)[72]>(&hs[0][0]), Np, r0,
+                      dMsgT + (size_t)b * 64 * Np);
 }
 
-// grad_w[a][o] = sum_c partial[c][a][o] (a < 64), grad_b[o] = sum_c partial[c][64][o]
-__global__ __launch_bounds__(256) void mp_wgrad_sum_kernel(int W, int chunks,
-                                                           const float *__restrict__ partial,
-                                                           float *__restrict__ grad_w,
-                                                           float *__restrict__ grad_b) {
-  const int idx = blockIdx.x * 256 + threadIdx.x;
-  if (idx >= 65 * W) return;
+// grad[k] = sum of the work-groups' shares: partial[layer][group][8256] for
+// the layers' parameters, head_partial[group][65] behind them.  Eight waves
+// share 64 parameters: wave w adds groups w, w + 8, ..., then the eight sums
+// are added in wave order (one thread per parameter adding all 256 in turn
+// took 58 us a matrix at 16 x n=1024; all parameters now take 12 us).
+__global__ __launch_bounds__(512) void mp_grad_sum_kernel(int layers, int groups,
+                                                          const float *__restrict__ partial,
+                                                          const float *__restrict__ head_partial,
+                                                          float *__restrict__ grad) {
+  __shared__ float sums[8][64];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int k = blockIdx.x * 64 + lane;  // 8256 is a multiple of 64: one layer per block
+  const int layer = blockIdx.x * 64 / 8256;
   float s = 0.0f;
-  for (int c = 0; c < chunks; ++c) s += partial[(size_t)c * 65 * W + idx];
-  if (idx < 64 * W)
-    grad_w[idx] = s;
-  else if (grad_b)
-    grad_b[idx - 64 * W] = s;
+  if (layer < layers) {
+    const float *src = partial + (size_t)layer * groups * 8256 + (k - layer * 8256);
+#pragma unroll 8
+    for (int g = w; g < groups; g += 8) s += src[(size_t)g * 8256];
+  } else if (k - layers * 8256 < 65) {
+    const float *src = head_partial + (k - layers * 8256);
+#pragma unroll 8
+    for (int g = w; g < groups; g += 8) s += src[(size_t)g * 65];
+  }
+  sums[w][lane] = s;
+  __syncthreads();
+  if (w != 0 || k >= layers * 8256 + 65) return;
+#pragma unroll
+  for (int q = 1; q < 8; ++q) s += sums[q][lane];
+  grad[k] = s;
 }
 
-// sum of the loss terms in a fixed order (one work-group)
+// sum of the work-groups' loss terms in a fixed order (one work-group)
 __global__ __launch_bounds__(256) void mp_loss_sum_kernel(size_t count,
                                                           const double *__restrict__ terms,
                                                           double *__restrict__ out) {
@@ -425,52 +611,55 @@ __global__ __launch_bounds__(256) void mp_compute_copy_kernel(int P,
 
 void mp_launch_features(hipStream_t st, int B, int n, int Np, const double *q, double *rowstat,
                         double *scale, uint16_t *A, float *X0, uint16_t *XT0) {
-  mp_rowstat_kernel<<<(unsigned)(((size_t)B * n + 255) / 256), 256, 0, st>>>(B, n, q, rowstat);
+  mp_rowstat_kernel<<<(unsigned)(((size_t)B * n + 3) / 4), 256, 0, st>>>(B, n, q, rowstat);
   OS_HIP_CHECK(hipGetLastError());
-  mp_scale_kernel<<<(B + 63) / 64, 64, 0, st>>>(B, n, rowstat, scale);
+  mp_scale_kernel<<<B, 256, 0, st>>>(n, rowstat, scale);
   OS_HIP_CHECK(hipGetLastError());
-  mp_fill_kernel<<<dim3((unsigned)(((size_t)Np * Np + 255) / 256), B), 256, 0, st>>>(
-      n, Np, q, rowstat, scale, A, X0, XT0);
-  OS_HIP_CHECK(hipGetLastError());
-}
-
-void mp_launch_agg(hipStream_t st, int B, int Np, const uint16_t *A, const uint16_t *XT, float *Y,
-                   bool accumulate) {
-  const dim3 grid(Np / 64, B);
-  if (accumulate)
-    mp_agg_kernel<true><<<grid, 256, 0, st>>>(Np, A, XT, Y);
-  else
-    mp_agg_kernel<false><<<grid, 256, 0, st>>>(Np, A, XT, Y);
+  mp_fill_kernel<<<dim3(Np, B), 256, 0, st>>>(n, Np, q, rowstat, scale, A, X0, XT0);
   OS_HIP_CHECK(hipGetLastError());
 }
 
-void mp_launch_node_fwd(hipStream_t st, int B, int Np, const float *Hin, const float *M,
-                        const float *wl, float *Z, float *H, uint16_t *HT) {
-  mp_node_fwd_kernel<<<dim3(Np / kRowsPerGroup, B), 256, 0, st>>>(Np, Hin, M, wl, Z, H, HT);
+void mp_launch_layer_fwd(hipStream_t st, int B, int n, int Np, const uint16_t *A,
+                         const uint16_t *XT, const float *Hin, float *M, const float *wl,
+                         float *Z, float *H, uint16_t *HT, const MpHead *head) {
+  const dim3 grid(Np / kRows, B);
+  const MpHead h = head ? *head : MpHead{};
+#define OS_FWD(AGG, HEAD)                                                                        \
+  mp_layer_fwd_kernel<AGG, HEAD><<<grid, 256, 0, st>>>(n, Np, A, XT, Hin, M, wl, Z, H, HT, h.wo, \
+                                                       h.labels, h.inv_count, h.p, h.dlogit,     \
+                                                       h.lossblock)
+  if (A) {
+    if (head) OS_FWD(true, true);
+    else OS_FWD(true, false);
+  } else {
+    if (head) OS_FWD(false, true);
+    else OS_FWD(false, false);
+  }
+#undef OS_FWD
   OS_HIP_CHECK(hipGetLastError());
 }
 
-void mp_launch_node_bwd(hipStream_t st, int B, int Np, const float *dH, const float *Z,
-                        const float *wl, float *dZ, float *dHprev, uint16_t *dMsgT) {
-  mp_node_bwd_kernel<<<dim3(Np / kRowsPerGroup, B), 256, 0, st>>>(Np, dH, Z, wl, dZ, dHprev,
-                                                                  dMsgT);
+void mp_launch_layer_bwd(hipStream_t st, int B, int Np, const uint16_t *A,
+                         const uint16_t *dMsgTin, const float *dHin, const MpHead *head,
+                         const float *Z, const float *wl, const float *Hin, const float *M,
+                         float *dHprev, uint16_t *dMsgT, float *partial, float *head_partial) {
+  const dim3 grid(Np / kRows, B);
+  const MpHead h = head ? *head : MpHead{};
+#define OS_BWD(TOP, PREV)                                                                       \
+  mp_layer_bwd_kernel<TOP, PREV><<<grid, 256, 0, st>>>(Np, A, dMsgTin, dHin, h.dlogit, h.wo, Z, \
+                                                       wl, Hin, M, dHprev, dMsgT, partial,      \
+                                                       head_partial)
+  if (head) OS_BWD(true, true);
+  else if (dHprev) OS_BWD(false, true);
+  else OS_BWD(false, false);
+#undef OS_BWD
   OS_HIP_CHECK(hipGetLastError());
 }
 
-void mp_launch_head(hipStream_t st, int B, int n, int Np, const float *H3, const float *wo,
-                    const uint8_t *labels, float inv_count, float *p, double *lossterm,
-                    float *dlogit, float *dH3) {
-  mp_head_kernel<<<(unsigned)(((size_t)B * Np + 255) / 256), 256, 0, st>>>(
-      B, n, Np, H3, wo, labels, inv_count, p, lossterm, dlogit, dH3);
-  OS_HIP_CHECK(hipGetLastError());
-}
-
-void mp_launch_wgrad(hipStream_t st, int rows, int W, const float *X, const float *G,
-                     float *partial, float *grad_w, float *grad_b) {
-  const int chunks = rows / 64;
-  mp_wgrad_partial_kernel<<<chunks, 256, 0, st>>>(W, X, G, partial);
-  OS_HIP_CHECK(hipGetLastError());
-  mp_wgrad_sum_kernel<<<(65 * W + 255) / 256, 256, 0, st>>>(W, chunks, partial, grad_w, grad_b);
+void mp_launch_grad_sum(hipStream_t st, int layers, int groups, const float *partial,
+                        const float *head_partial, float *grad) {
+  mp_grad_sum_kernel<<<(layers * 8256 + 65 + 63) / 64, 512, 0, st>>>(layers, groups, partial,
+                                                                     head_partial, grad);
   OS_HIP_CHECK(hipGetLastError());
 }
 

@@ -56,6 +56,29 @@ def test_mpnn_gradient_matches_oracle(ctx):
     d.close()
 
 
+@pytest.mark.parametrize("n,I", [(2, 1), (63, 2), (65, 2), (130, 5)])
+def test_mpnn_row_tiles_match_oracle(ctx, n, I):
+    """Sizes at the edges of the 64-row tiles (one tile, a ragged last one,
+    three) and work-group counts that are no multiple of eight: loss, gradient
+    and marginals, with the tolerances of the tests above."""
+    d, qs = _data(ctx, I=I, n=n, seed=21)
+    labels = np.random.default_rng(n).integers(0, 2, (I, n), dtype=np.uint8)
+    net = onesolver_amd.WarmStartNet(ctx, seed=3)
+    flat = _params(8)
+    net.set_params(flat)
+    flat32 = flat.astype(np.float32).astype(np.float64)
+    print(f"[gpu] mpnn tiles {I} x n={n}", flush=True)
+    loss, g = net.loss_grad(d, labels)
+    ol, og = mpnn.loss_grad(flat32, list(qs), list(mpnn.canonical(labels)), rounding="bf16")
+    assert abs(loss - ol) < 1e-4 * abs(ol)
+    assert np.linalg.norm(g - og) < 1e-2 * np.linalg.norm(og)
+    p = net.predict(d)
+    for i in range(I):
+        assert np.max(np.abs(p[i] - mpnn.forward(flat32, qs[i], rounding="bf16"))) < 5e-3
+    net.close()
+    d.close()
+
+
 def test_mpnn_predict_matches_oracle(ctx):
     d, qs = _data(ctx, I=2, n=100, seed=2)
     net = onesolver_amd.WarmStartNet(ctx, seed=1)
