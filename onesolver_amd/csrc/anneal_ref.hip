@@ -10,6 +10,7 @@
 //   - an accepted flip updates all fields with row s of Q (coalesced,
 //     Q is symmetric), E += dE;
 //   - best state copied whenever E < E_best (annealing.hpp:115-121).
+// ref_anneal_kernel (n > 1024) takes these steps one by one.
 #include "os_kernels.h"
 
 namespace os {
@@ -91,19 +92,34 @@ __global__ __launch_bounds__(64) void ref_anneal_kernel(int n, const double *__r
   if (lane == 0) best_run[replica] = e_best;
 }
 
-// n <= 64: the same chain with the replica in registers, kLook attempts per
-// step by speculation.  Lane j holds h_j; the state and best state are
-// wave-uniform 64-bit masks; Q is staged in LDS.  The draws of an attempt
-// do not depend on the state, so lane 2^m - 1 + p (m < kLook, p < 2^m)
-// evaluates attempt t + m as if attempts t .. t+m-1 had been accepted where
-// bit i of p is set: it replays their field updates on h at its own site, in
-// the chain's order and with the chain's fma, and takes the acceptance test.
-// A ballot of the 63 answers, walked from m = 0 along the decisions made,
-// gives the chain's kLook decisions; they are then applied in order.  Every
-// FP64 operation that reaches the state, energy or best state is the one of
-// ref_anneal_kernel, so the chains are the same.
-constexpr int kRefSmallN = 64;
-constexpr int kLook = 6;
+// n <= 1024: the same chain, 64 attempts at a time.  The draws of an attempt do
+// not depend on the state, so lane m draws attempt t + m (site, u, threshold)
+// and keeps its site's field and spin.  All 64 acceptance tests are taken at
+// once; the first accepted attempt (ballot) is the next flip of the chain --
+// everything before it is a rejection -- and updates the fields and spins the
+// later lanes keep, with the chain's own fma; then the tests of the lanes
+// behind it are taken again.  So a rejection costs a 64th of a step and an
+// acceptance some forty instructions.  The n fields themselves take the
+// window's accepted rows of Q at its end, in order, several requested at once.  The couplings between the window's sites come from
+// Q staged in LDS (kQLds, n <= 64) or are gathered into LDS at its start.
+// The state and the best state are bit words, word w in lane w.
+//
+// The test exp(-dE / b) > u is decided by dE against -b ln u, made once per
+// lane and window, where they differ by more than 1e-13 (b + |b ln u|), far
+// above the rounding of either side; otherwise, and for b or u outside the
+// ordinary, the expression itself is evaluated.  Every FP64 operation that
+// reaches the state, energy or best state is the one of ref_anneal_kernel, so
+// the chains are the same.
+//
+// A chain is serial, one wave per try: what bounds it is the instructions per
+// acceptance and, for n > 64, the rows of Q read from L2 (8 n bytes per
+// acceptance).  Measured on one MI355X: n = 28, 1024 tries x 1000 attempts
+// 248 -> 55 us (speculating on all outcomes of six attempts before); n = 512,
+// 460 tries x 1000 attempts 1636 -> 425 us (ref_anneal_kernel before: every
+// acceptance waited for its row).
+// Above 1024 spins 32 fields, as many diagonal entries and two rows of a lane
+// no longer fit 256 registers; ref_anneal_kernel takes over there.
+constexpr int kRefWindowN = 1024;
 
 __device__ __forceinline__ double readlane_f64(double v, int l) {
   const uint64_t b = (uint64_t)__double_as_longlong(v);
@@ -112,134 +128,187 @@ __device__ __forceinline__ double readlane_f64(double v, int l) {
   return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
 
-__global__ __launch_bounds__(64) void ref_anneal_small_kernel(int n, const double *__restrict__ q,
-                                                              const double *__restrict__ beta,
-                                                              uint64_t total_attempts, int spb,
-                                                              uint32_t k0, uint32_t k1,
-                                                              uint32_t *__restrict__ best_bits,
-                                                              int W,
-                                                              double *__restrict__ best_run) {
-  extern __shared__ __align__(16) double qs[];  // n x n
+// NC: fields per lane (j = lane + 64 c), n <= 64 NC.
+template <int NC, bool kQLds>
+__global__ __launch_bounds__(64) void ref_anneal_window_kernel(
+    int n, const double *__restrict__ q, const double *__restrict__ beta,
+    uint64_t total_attempts, int spb, uint32_t k0, uint32_t k1,
+    uint32_t *__restrict__ best_bits, int W, double *__restrict__ best_run) {
+  extern __shared__ __align__(16) double sm[];
+  double *qs = sm;           // kQLds: Q, n x n
+  double *pair = sm;         // otherwise: couplings of the window's sites, 64 x 64,
+  double *hl = sm + 64 * 64;  // and the fields, n
   const uint32_t replica = blockIdx.x;
   const int lane = threadIdx.x;
-  for (int i = lane; i < n * n; i += 64) qs[i] = q[i];
-  const bool live = lane < n;
-  uint32_t b0 = 0;
-  {
-    const uint4 o = philox4x32_10(make_uint4(0u, replica, 0u, TAG_REF_INIT), k0, k1);
-    if (live) b0 = (pick(o, (lane >> 5) & 3) >> (lane & 31)) & 1u;
+  if (kQLds) {
+    for (int i = lane; i < n * n; i += 64) qs[i] = q[i];
+    __syncthreads();
   }
-  uint64_t x = __ballot(b0 != 0u);
-  uint64_t best = x;
-  __syncthreads();
-  const double qjj = live ? qs[lane * n + lane] : 0.0;
-  double h = qjj;
-  for (int l = 0; l < n; ++l)
-    if ((x >> l) & 1u) {
-      const double v = live ? qs[l * n + lane] : 0.0;
-      if (live && lane != l) h += v;
+  // h[j] = fma(Q[s][j], d, h[j]) for j != s, row after row of the list that
+  // next(s, d) walks (false behind its end, with any valid s); kBatch rows are
+  // requested together, so that a batch and not every row waits for L2.  A
+  // lane's fields past n take copies of column n - 1 and are never read.
+  constexpr int kBatch = NC <= 8 ? 8 : 64 / NC;
+  double qd[NC], h[NC];
+  int col[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) col[c] = min(lane + 64 * c, n - 1);
+  auto add_rows = [&](auto next) {
+    for (bool more = true; more;) {
+      int sr[kBatch];
+      bool on[kBatch];
+      double d[kBatch], r[kBatch][NC];
+#pragma unroll
+      for (int k = 0; k < kBatch; ++k) {
+        on[k] = next(sr[k], d[k]);
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+          r[k][c] = kQLds ? qs[sr[k] * n + col[c]] : (q + (size_t)sr[k] * n)[(uint32_t)col[c]];
+      }
+      more = on[kBatch - 1];
+#pragma unroll
+      for (int k = 0; k < kBatch; ++k) {
+        if (!on[k]) break;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          const double v = fma(r[k][c], d[k], h[c]);
+          h[c] = lane + 64 * c != sr[k] ? v : h[c];
+        }
+      }
     }
+  };
+  // start state: word `lane` of the state
+  uint32_t word = 0u;
+  {
+    const uint4 o =
+        philox4x32_10(make_uint4((uint32_t)(lane >> 2), replica, 0u, TAG_REF_INIT), k0, k1);
+    const int valid = n - 32 * lane;
+    const uint32_t v = pick(o, (uint32_t)lane & 3u);
+    word = valid >= 32 ? v : valid <= 0 ? 0u : (v & ((1u << valid) - 1u));
+  }
+  uint32_t best = word;
+  // fields: diagonal, then + row l for every set l in ascending order
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    qd[c] = q[(size_t)col[c] * n + col[c]];
+    h[c] = qd[c];
+  }
+  {
+    int w = -1;
+    uint32_t bits = 0u;
+    add_rows([&](int &l, double &d) {  // fma(row, 1, h) is h + row
+      l = 0;
+      d = 1.0;
+      while (bits == 0u) {
+        if (++w >= W) return false;
+        bits = (uint32_t)__builtin_amdgcn_readlane((int)word, w);
+      }
+      l = 32 * w + __builtin_ctz(bits);
+      bits &= bits - 1u;
+      return true;
+    });
+  }
   double part = 0.0;
-  if (live && ((x >> lane) & 1u)) part += 0.5 * (h + qjj);
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int j = lane + 64 * c;
+    const uint32_t xw =
+        (uint32_t)__builtin_amdgcn_ds_bpermute((j >> 5) << 2, (int)word);
+    if (j < n && ((xw >> (j & 31)) & 1u)) part += 0.5 * (h[c] + qd[c]);
+  }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) part += __shfl_xor(part, off, 64);
   double e_cur = part;
   double e_best = part;
 
-  // this lane's candidate: attempt offset m_l, assumed decisions p_l (lane
-  // 63 evaluates nothing); its draw is computed one step ahead
-  const int m_l = 31 - __clz(lane + 1);
-  const uint32_t p_l = (uint32_t)(lane + 1 - (1 << m_l));
-  const int m_c = min(m_l, kLook - 1);
-  auto draw = [&](uint64_t t) {
-    const uint64_t tm = t + (uint64_t)m_c;
-    return philox4x32_10(make_uint4((uint32_t)tm, replica, (uint32_t)(tm >> 32), TAG_REF_STEP),
-                         k0, k1);
-  };
-  uint4 o = draw(0);
-  int bi = 0, bc = 0;  // beta index of attempt t and its remainder: t = bi * spb + bc
-  for (uint64_t t = 0; t < total_attempts; t += kLook) {
-    const int kk = (int)min((uint64_t)kLook, total_attempts - t);
-    const int s_l = (int)__umulhi(o.x, (uint32_t)n);
-    const double u_l = (double)o.y * 0x1p-32;
-    o = draw(t + kLook);
-    // sites and temperatures of the kLook attempts (uniform)
-    int sm[kLook];
-    double bm[kLook];
-    int ci = bi, cc = bc, bi_next = bi, bc_next = bc;
+  uint32_t bi = 0, bc = 0;  // attempt t is number bc of beta[bi]
+  for (uint64_t t = 0; t < total_attempts; t += 64) {
+    const int kk = (int)min((uint64_t)64, total_attempts - t);
+    const uint64_t tm = t + (uint64_t)lane;
+    const uint4 o =
+        philox4x32_10(make_uint4((uint32_t)tm, replica, (uint32_t)(tm >> 32), TAG_REF_STEP), k0,
+                      k1);
+    const int s = (int)__umulhi(o.x, (uint32_t)n);
+    const double u = (double)o.y * 0x1p-32;
+    const double b = lane < kk ? beta[bi + (bc + (uint32_t)lane) / (uint32_t)spb] : 1.0;
+    bi += (bc + 64u) / (uint32_t)spb;
+    bc = (bc + 64u) % (uint32_t)spb;
+    const double thr = -b * log(u);
+    const double tol = 1e-13 * (b + fabs(thr));
+    const bool plain = b > 0.0 && b < 1e300 && u > 0.0;
+    // dE < lo: accepted for sure (lo >= 0, so dE < 0 is among them); dE > hi:
+    // rejected for sure; in between, NaN included: the expression decides
+    const double lo = plain ? fmax(thr - tol, 0.0) : 0.0, hi = plain ? thr + tol : INFINITY;
+    // this lane's field and spin
+    double hm;
+    if (NC == 1) {
+      const uint64_t hb = (uint64_t)__double_as_longlong(h[0]);
+      const uint32_t h0 = (uint32_t)__builtin_amdgcn_ds_bpermute(s << 2, (int)(uint32_t)hb);
+      const uint32_t h1 =
+          (uint32_t)__builtin_amdgcn_ds_bpermute(s << 2, (int)(uint32_t)(hb >> 32));
+      hm = __longlong_as_double((long long)(((uint64_t)h1 << 32) | h0));
+    } else {
 #pragma unroll
-    for (int m = 0; m < kLook; ++m) {
-      sm[m] = __builtin_amdgcn_readlane(s_l, (1 << m) - 1);
-      bm[m] = m < kk ? beta[ci] : 1.0;
-      if (++cc == spb) {
-        cc = 0;
-        ++ci;
-      }
-      if (m == kk - 1) {
-        bi_next = ci;
-        bc_next = cc;
-      }
+      for (int c = 0; c < NC; ++c)
+        if (lane + 64 * c < n) hl[lane + 64 * c] = h[c];
+      __syncthreads();
+      hm = hl[s];
     }
-    // rows of Q at the kLook sites, for the updates applied below
-    double qrow[kLook];
+    uint32_t xb =
+        ((uint32_t)__builtin_amdgcn_ds_bpermute((s >> 5) << 2, (int)word) >> (s & 31)) & 1u;
+    if (!kQLds) {
+      // pair[m][lane] = Q[s_m][s_lane] (read by the lanes behind m)
+#pragma unroll 1
+      for (int m0 = 0; m0 < 64; m0 += 16) {
+        double v[16];
 #pragma unroll
-    for (int m = 0; m < kLook; ++m) qrow[m] = live ? qs[sm[m] * n + lane] : 0.0;
-    // this lane's field h_{s_l} at time t (from lane s_l) and temperature
-    const uint64_t hb = (uint64_t)__double_as_longlong(h);
-    const uint32_t hlo = (uint32_t)__builtin_amdgcn_ds_bpermute(s_l << 2, (int)(uint32_t)hb);
-    const uint32_t hhi =
-        (uint32_t)__builtin_amdgcn_ds_bpermute(s_l << 2, (int)(uint32_t)(hb >> 32));
-    double h_l = __longlong_as_double((long long)(((uint64_t)hhi << 32) | hlo));
-    double b_l = bm[0];
-#pragma unroll
-    for (int m = 1; m < kLook; ++m) b_l = m_c == m ? bm[m] : b_l;
-    // replay the assumed decisions of attempts t .. t + m_l - 1 (selects,
-    // not branches: the fma is the chain's whether or not it is kept)
-    uint64_t fm = 0;  // spins flipped on the assumed path
-#pragma unroll
-    for (int i = 0; i < kLook - 1; ++i) {
-      const int si = sm[i];
-      const double qv = qs[si * n + s_l];
-      const bool on = i < m_l && ((p_l >> i) & 1u);
-      const bool xi = ((x ^ fm) >> si) & 1u;
-      const double hn = fma(qv, xi ? -1.0 : 1.0, h_l);
-      h_l = on && si != s_l ? hn : h_l;
-      fm ^= on ? 1ull << si : 0ull;
-    }
-    const bool xl = ((x ^ fm) >> s_l) & 1u;
-    const double de = xl ? -h_l : h_l;
-    const bool acc = m_l < kk && ((de < 0.0) || (exp(-de / b_l) > u_l));
-    const uint64_t A = __ballot(acc);
-    // the chain's decisions, applied in order
-    uint32_t p = 0;
-#pragma unroll
-    for (int m = 0; m < kLook; ++m) {
-      if (m < kk) {
-        const int L = (1 << m) - 1 + (int)p;
-        if ((A >> L) & 1u) {
-          const int s = sm[m];
-          const double d = ((x >> s) & 1u) ? -1.0 : 1.0;
-          const double hn = fma(qrow[m], d, h);
-          h = live && lane != s ? hn : h;
-          x ^= 1ull << s;
-          e_cur += readlane_f64(de, L);
-          p |= 1u << m;
+        for (int k = 0; k < 16; ++k) {
+          v[k] = (q + (size_t)__builtin_amdgcn_readlane(s, m0 + k) * n)[(uint32_t)s];
         }
-        if (e_cur < e_best) {
-          e_best = e_cur;
-          best = x;
-        }
+#pragma unroll
+        for (int k = 0; k < 16; ++k) pair[(m0 + k) * 64 + lane] = v[k];
       }
+      __syncthreads();
     }
-    bi = bi_next;
-    bc = bc_next;
+    uint64_t live = kk == 64 ? ~0ull : (1ull << kk) - 1ull;  // attempts not yet decided
+    uint64_t taken = 0ull, down = 0ull;                      // accepted; those flipping 1 -> 0
+    double de = xb ? -hm : hm;
+    for (;;) {
+      const uint64_t cand = __ballot(!(de > hi)) & live;
+      if (cand == 0ull) break;
+      const int m = __builtin_ctzll(cand);
+      live &= (~1ull) << m;
+      if (!((__ballot(de < lo) >> m) & 1ull))
+        if (!((__ballot(exp(-de / b) > u) >> m) & 1ull)) continue;
+      const int sm_ = __builtin_amdgcn_readlane(s, m);
+      const uint32_t xm = (uint32_t)__builtin_amdgcn_readlane((int)xb, m);
+      const double dem = readlane_f64(de, m);
+      const double pv = kQLds ? qs[sm_ * n + s] : pair[m * 64 + lane];
+      const double hn = fma(pv, xm ? -1.0 : 1.0, hm);
+      const bool same = s == sm_;
+      hm = same ? hm : hn;
+      xb ^= same ? 1u : 0u;
+      de = xb ? -hm : hm;
+      word ^= lane == (sm_ >> 5) ? 1u << (sm_ & 31) : 0u;
+      e_cur += dem;
+      taken |= 1ull << m;
+      down |= (uint64_t)xm << m;
+      const bool better = e_cur < e_best;
+      e_best = better ? e_cur : e_best;
+      best = better ? word : best;
+    }
+    // the window's accepted rows into the fields, in order
+    add_rows([&](int &l, double &d) {
+      const bool on = taken != 0ull;
+      const int m = on ? __builtin_ctzll(taken) : 0;
+      taken &= taken - 1ull;
+      l = __builtin_amdgcn_readlane(s, m);
+      d = (down >> m) & 1ull ? -1.0 : 1.0;
+      return on;
+    });
   }
-  if (lane == 0) {
-    uint32_t *dst = best_bits + (size_t)replica * W;
-    dst[0] = (uint32_t)best;
-    if (W > 1) dst[1] = (uint32_t)(best >> 32);
-    best_run[replica] = e_best;
-  }
+  if (lane < W) best_bits[(size_t)replica * W + lane] = best;
+  if (lane == 0) best_run[replica] = e_best;
 }
 
 int ref_lds_limit() { return 4096; }
@@ -255,9 +324,18 @@ void launch_ref_anneal(hipStream_t st, int n, const double *q, const double *bet
   const uint64_t total = (uint64_t)num_iter * (uint64_t)spb;
   const int W = (n + 31) / 32;
   const size_t lds = (ref_lds_bytes(n) + 15) & ~(size_t)15;
-  if (n <= kRefSmallN) {
-    ref_anneal_small_kernel<<<num_tries, 64, sizeof(double) * (size_t)n * n, st>>>(
-        n, q, beta, total, spb, k0, k1, best_bits, W, best_run);
+  if (n <= kRefWindowN) {
+    // fields per lane: the next power of two of n / 64
+    const size_t wlds = sizeof(double) * (n <= 64 ? (size_t)n * n : (size_t)64 * 64 + n);
+#define OS_WINDOW(NC, QL)                                                           \
+  ref_anneal_window_kernel<NC, QL><<<num_tries, 64, wlds, st>>>(n, q, beta, total,   \
+                                                                spb, k0, k1, best_bits, W, best_run)
+    if (n <= 64) OS_WINDOW(1, true);
+    else if (n <= 128) OS_WINDOW(2, false);
+    else if (n <= 256) OS_WINDOW(4, false);
+    else if (n <= 512) OS_WINDOW(8, false);
+    else OS_WINDOW(16, false);
+#undef OS_WINDOW
   } else if (n <= ref_lds_limit()) {
     ref_anneal_kernel<true><<<num_tries, 64, lds, st>>>(n, q, beta, total, spb, k0, k1, nullptr,
                                                          best_bits, W, best_run);

@@ -46,7 +46,7 @@ __device__ __forceinline__ float bf16_round(float f) {
 
 // rowstat[b][i] = (sum_{j != i} Q_ij^2, sum_{j != i} Q_ij) of instance q[b]:
 // one wave per row, so the FP64 matrices are read once in 512-byte requests
-// (one thread per row, 8 KB apart, took 146 us for 16 x n=1024; 33 us now).
+// (one thread per row, 8 KB apart, took 146 us for 16 x n=1024; 21 us now).
 __global__ __launch_bounds__(256) void mp_rowstat_kernel(int B, int n, const double *__restrict__ q,
                                                          double *__restrict__ rowstat) {
   const size_t t = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -241,7 +241,8 @@ __device__ __forceinline__ void load_tile(Tile &dst, const float *__restrict__ s
 // Rows r0.. of A . X (A row-major, X feature-major, both bf16, fp32 sums) into
 // y: wave w makes rows 32 (w/2).. x features 32 (w%2)...  Four k steps are in
 // flight while four are multiplied; requested one by one, each step waited
-// for L2 (19 us a layer at 16 x n=1024, of which now 8).
+// for L2 (a layer's aggregation and node update took 19 + 21 us at 16 x n=1024,
+// the one launch takes 27).
 __device__ __forceinline__ void agg_tile(int Np, const uint16_t *__restrict__ A,
                                          const uint16_t *__restrict__ XT, int r0, Tile &y) {
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -530,7 +531,7 @@ __global__ __launch_bounds__(256) void mp_layer_bwd_kernel(
 // the layers' parameters, head_partial[group][65] behind them.  Eight waves
 // share 64 parameters: wave w adds groups w, w + 8, ..., then the eight sums
 // are added in wave order (one thread per parameter adding all 256 in turn
-// took 58 us a matrix at 16 x n=1024; all parameters now take 12 us).
+// took 58 us a matrix at 16 x n=1024; all parameters now take 5.5 us).
 __global__ __launch_bounds__(512) void mp_grad_sum_kernel(int layers, int groups,
                                                           const float *__restrict__ partial,
                                                           const float *__restrict__ head_partial,

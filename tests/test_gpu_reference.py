@@ -79,6 +79,27 @@ def test_reference_anneal_config1_chain_and_hit_rate(ctx):
     assert be >= ground - tol
 
 
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 128, 129, 512, 513, 1025, 2048, 2049])
+def test_reference_anneal_windows_match_oracle_chain(ctx, n):
+    """Sizes at the edges of the fields a lane holds, attempt counts that are
+    no multiple of the 64 taken together, three attempts per beta, and betas
+    for which the test on -b ln u does not hold (0, negative, infinite): the
+    oracle's chains bit for bit (integer Q, so every field is exact)."""
+    rng = np.random.default_rng(n)
+    q = np.triu(rng.integers(-3, 4, (n, n)).astype(np.float64))
+    q = q + np.triu(q, 1).T
+    scale = max(1.0, np.sqrt(n) / 2)
+    beta = np.concatenate([np.geomspace(0.3, 3.0, 40) * scale, [0.0, -1.0, np.inf, 1e-300],
+                           np.geomspace(3.0, 0.5, 21) * scale])
+    print(f"[gpu] reference windows n={n}", flush=True)
+    tries = 70 if n <= 1025 else 20
+    best, be, states, energies = ctx.anneal_reference(q, beta, tries, sweeps_per_beta=3, seed=77)
+    s_or, e_or = oracle.anneal(q, n, beta, tries, sweeps_per_beta=3, seed=77)
+    assert (states == s_or).all()
+    assert np.array_equal(energies, e_or)
+    assert be == e_or.min() and (best == s_or[int(np.argmin(e_or))]).all()
+
+
 def test_reference_anneal_large_n_uses_global_fields(ctx):
     rng = np.random.default_rng(5)
     n = 4100  # above the LDS-resident field limit
