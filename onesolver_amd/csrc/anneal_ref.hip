@@ -115,7 +115,7 @@ __global__ __launch_bounds__(64) void ref_anneal_kernel(int n, const double *__r
 // acceptance and, for n > 64, the rows of Q read from L2 (8 n bytes per
 // acceptance).  Measured on one MI355X: n = 28, 1024 tries x 1000 attempts
 // 248 -> 55 us (speculating on all outcomes of six attempts before); n = 512,
-// 460 tries x 1000 attempts 1636 -> 425 us (ref_anneal_kernel before: every
+// 460 tries x 1000 attempts 1636 -> 428 us (ref_anneal_kernel before: every
 // acceptance waited for its row).
 // Above 1024 spins 32 fields, as many diagonal entries and two rows of a lane
 // no longer fit 256 registers; ref_anneal_kernel takes over there.
