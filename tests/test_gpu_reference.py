@@ -37,6 +37,24 @@ def test_energy_fp64_matches_oracle(ctx, n, count):
     assert np.all(np.abs(got - ref) <= 1e-12 * scale)
 
 
+@pytest.mark.parametrize("n,counts", [(1, (1, 65)), (8, (64, 70000)), (57, (257,)),
+                                      (64, (65600,)), (65, (1, 15, 16, 17, 8193)),
+                                      (66, (31, 33)), (67, (32,)), (68, (16,)), (95, (8, 8192)),
+                                      (96, (17,)), (97, (16,)), (127, (33,)), (128, (8200,)),
+                                      (129, (4097,)), (161, (40,)), (260, (2753,))])
+def test_energy_tiles_match_oracle(ctx, n, counts):
+    """Edges of the energy kernels' tiles (states by 16 and 32, columns by 16
+    and 128, the last 4 and 32 of k) and of their choice.  Whole numbers below
+    2^20: every partial sum is exact, so the energies are equal."""
+    rng = np.random.default_rng(n)
+    q = np.triu(rng.integers(-(1 << 20), 1 << 20, (n, n))).astype(np.float64)
+    q = q + np.triu(q, 1).T
+    for count in counts:
+        print(f"[gpu] energy tiles n={n} count={count}", flush=True)
+        st = rng.integers(0, 2, (count, n)).astype(np.uint8)
+        assert np.array_equal(ctx.energy_fp64(q, st), oracle.energy(q, st)), count
+
+
 @pytest.mark.parametrize("path,ground", _kats())
 def test_reference_anneal_matches_oracle_chain_on_kats(ctx, path, ground):
     q = load_qubo(path)
