@@ -366,7 +366,7 @@ def run_csr_c3(args):
                    "instances": 512, "replicas": R, "sweeps": S, "sum_n": int(ns.sum()),
                    "site_order": args.c3_order, "launch_shape": list(shape()),
                    "launch_shape_fields": ["waves per group", "groups",
-                                           "sites per step" if order else "row prefetch"]},
+                                           "sites per step" if order else "kernel (1: row prefetch, 2: scheduled)"]},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": PEAK_HBM_GBS, "unit": "GB/s",
                      "frac": achieved / PEAK_HBM_GBS,
                      "traffic": (TRAFFIC_CSR_C3_COLOUR if order else TRAFFIC_CSR_C3)

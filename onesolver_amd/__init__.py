@@ -681,7 +681,8 @@ class CsrBatch:
 
     def launch_shape(self):
         """(waves per work-group, resident work-groups, 1 if the
-        row-prefetching kernel runs else 0); zeros before the first run."""
+        row-prefetching kernel runs, 2 if the one that updates uncoupled sites
+        together, else 0); zeros before the first run."""
         w, g, r = ctypes.c_int32(0), ctypes.c_int32(0), ctypes.c_int32(0)
         _check(_csr_lib().os_csr_batch_launch_shape(self._h, ctypes.byref(w), ctypes.byref(g),
                                                     ctypes.byref(r)))

@@ -602,6 +602,257 @@ __global__ __launch_bounds__(64 * kW) void csr_sweep_col_kernel(
   }
 }
 
+// Scheduled variant of the index-order sweep.  The update of site j reads its
+// neighbours l < j as this sweep left them and its neighbours l > j as the last
+// one did, so sites that are not coupled may be updated together as long as
+// every coupled pair keeps its order: the host packs the sites of an instance
+// into steps of at most G (each site in the first step with room after all of
+// its lower-index neighbours, and no site before one that reads it from
+// below), and a wave runs a step for each of its 64/G replicas at once.  Draws,
+// field order and dE of a site are those of csr_sweep_kernel, and the running
+// energy adds the accepted dE in index order at the end of the sweep, so states
+// and energies are the same bit for bit.
+//
+// The serial chain of sites bounds the other kernels whenever there are fewer
+// than some four waves of 64 replicas for each CU; here a wave has 64/G
+// replicas and 1/G of the steps.
+//
+// Measured: 32 instances of 64 .. 1024 spins, degrees 3 .. 8, 128 replicas, 192
+// sweeps 67.3 -> 5.8 ms, the largest instance's chain of 1020 sites (340 ns
+// each) now ~70 steps.  The other kernels remain for batches with enough
+// replicas to fill the chip at 64 a wave, where each site's row is read once
+// for all of them, and for states too large for these LDS arrays: the tuner
+// times all of them on the batch (n = 500, degree 5, 32 sweeps: 64 instances x
+// 1024 replicas 6.6 ms prefetching, 4.4 scheduled; 256 x 1024 stays with the
+// prefetching kernel, 12.6 ms).
+//
+// LDS of a wave, replica by replica: td[j], the threshold of site j until its
+// update and its accepted dE (or 0) afterwards; xb[j], one byte a spin (an
+// address, a read, a conversion and an FMA per coupling, without the bit's own
+// two instructions).
+namespace {
+
+__host__ __device__ inline int sched_tstride(int n) { return ((n + 16) & ~15) + 4; }
+__host__ __device__ inline int sched_bstride(int words) { return words * 32 + 16; }
+
+// Order of this wave's LDS accesses as written (the LDS serves a wave's accesses
+// in order; only the compiler has to keep it).
+__device__ __forceinline__ void lds_order() {
+  __builtin_amdgcn_wave_barrier();
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+
+// Spins 32 wd .. 32 wd + 31 between bytes and a word.
+__device__ __forceinline__ void put_word(uint8_t *xb, int wd, uint32_t v) {
+  uint32_t *b = reinterpret_cast<uint32_t *>(xb + 32 * wd);
+#pragma unroll
+  for (int m = 0; m < 8; ++m) b[m] = (((v >> (4 * m)) & 15u) * 0x00204081u) & 0x01010101u;
+}
+__device__ __forceinline__ uint32_t get_word(const uint8_t *xb, int wd) {
+  const uint32_t *b = reinterpret_cast<const uint32_t *>(xb + 32 * wd);
+  uint32_t v = 0u;
+#pragma unroll
+  for (int m = 0; m < 8; ++m) v |= ((b[m] * 0x01020408u) >> 24) << (4 * m);
+  return v;
+}
+
+template <int G>
+__device__ __forceinline__ void sched_item(
+    const CsrInst &d, int2 wi, char *lds, int lane, int S, int Rp, uint32_t k0, uint32_t k1,
+    uint32_t base, int init_mode, int tb, int use_tsr, const float *__restrict__ tsr,
+    const int4 *__restrict__ ell_col, const float4 *__restrict__ ell_val,
+    const float *__restrict__ diag, const int32_t *__restrict__ sched,
+    const float *__restrict__ tscale, const uint32_t *__restrict__ init_bits,
+    uint32_t *__restrict__ best_bits, uint32_t *__restrict__ final_bits,
+    double *__restrict__ e_best, double *__restrict__ e_final) {
+  constexpr int RW = 64 / G;  // replicas per wave
+  const int rr = lane / G, s = lane % G;
+  const int n = d.n, words = d.words, chunks = d.width >> 2, steps = d.steps;
+  float *td = reinterpret_cast<float *>(lds) + rr * sched_tstride(n);
+  uint8_t *xb = reinterpret_cast<uint8_t *>(lds) + 4 * RW * sched_tstride(n) +
+                rr * sched_bstride(words);
+  const uint32_t r = (uint32_t)(wi.y * RW + rr);
+  const uint32_t id = (base + (uint32_t)wi.x) << 8;
+  const int4 *ecol = ell_col + (d.ell_off >> 2);
+  const float4 *eval = ell_val + (d.ell_off >> 2);
+  const float *dg = diag + d.spin_off;
+  const int32_t *sc = sched + d.sched_off + s;
+  uint32_t *bb = best_bits + d.state_off + r;
+  for (int wd = s; wd < words; wd += G) {
+    uint32_t v;
+    if (init_mode) {
+      v = init_bits[d.state_off + (size_t)wd * Rp + r];
+    } else {
+      const uint4 o = philox4x32_10(make_uint4((uint32_t)(wd >> 2), r, 0u, id | TAG_SWEEP_INIT),
+                                    k0, k1);
+      v = pick(o, (uint32_t)wd & 3u);
+    }
+    const int valid = n - 32 * wd;
+    if (valid < 32) v = valid <= 0 ? 0u : (v & ((1u << valid) - 1u));
+    put_word(xb, wd, v);
+    bb[(size_t)wd * Rp] = v;
+  }
+  lds_order();
+  // FP64 energy in the oracle's order: G sites' terms at a time, added one
+  // after the other
+  double e = 0.0;
+  for (int j0 = 0; j0 < n; j0 += G) {
+    const int j = min(j0 + s, n - 1);
+    double off = 0.0;
+    for (int c = 0; c < chunks; ++c) {
+      const int4 cc = ecol[(size_t)j * chunks + c];
+      const float4 vv = eval[(size_t)j * chunks + c];
+      off = xb[cc.x] ? off + (double)vv.x : off;
+      off = xb[cc.y] ? off + (double)vv.y : off;
+      off = xb[cc.z] ? off + (double)vv.z : off;
+      off = xb[cc.w] ? off + (double)vv.w : off;
+    }
+    const double term = j0 + s < n && xb[j] ? (double)dg[j] + 0.5 * off : 0.0;
+#pragma unroll
+    for (int k = 0; k < G; ++k) e += __shfl(term, k, G);
+  }
+  double eb = e;
+
+  // a site's row and diagonal travel a step ahead of its update, its index two
+  struct Site {
+    int j;
+    float dj;
+    int4 c0, c1;
+    float4 v0, v1;
+  };
+  auto at = [](const void *p, uint32_t off) { return reinterpret_cast<const char *>(p) + off; };
+  auto fetch = [&](int j) {
+    Site st;
+    const int jr = min(j, n - 1);
+    const uint32_t ro = (uint32_t)jr * (uint32_t)chunks * 16u;  // row's byte offset
+    st.j = j;
+    st.dj = *reinterpret_cast<const float *>(at(dg, (uint32_t)jr * 4u));
+    st.c0 = *reinterpret_cast<const int4 *>(at(ecol, ro));
+    st.v0 = *reinterpret_cast<const float4 *>(at(eval, ro));
+    st.c1 = make_int4(n, n, n, n);
+    st.v1 = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (chunks > 1) {
+      st.c1 = *reinterpret_cast<const int4 *>(at(ecol, ro + 16u));
+      st.v1 = *reinterpret_cast<const float4 *>(at(eval, ro + 16u));
+    }
+    return st;
+  };
+  auto decide = [&](const Site &c) {
+    const float thr = td[c.j];
+    float h = c.dj;
+    const float xj = (float)xb[c.j];
+    // h + w for a set neighbour, h for a clear one: see add_if_set
+    h = fmaf((float)xb[c.c0.x], c.v0.x, h);
+    h = fmaf((float)xb[c.c0.y], c.v0.y, h);
+    h = fmaf((float)xb[c.c0.z], c.v0.z, h);
+    h = fmaf((float)xb[c.c0.w], c.v0.w, h);
+    if (chunks > 1) {
+      h = fmaf((float)xb[c.c1.x], c.v1.x, h);
+      h = fmaf((float)xb[c.c1.y], c.v1.y, h);
+      h = fmaf((float)xb[c.c1.z], c.v1.z, h);
+      h = fmaf((float)xb[c.c1.w], c.v1.w, h);
+    }
+    for (int cc = 2; cc < chunks; ++cc) {
+      const uint32_t ro =
+          ((uint32_t)min(c.j, n - 1) * (uint32_t)chunks + (uint32_t)cc) * 16u;
+      const int4 ci = *reinterpret_cast<const int4 *>(at(ecol, ro));
+      const float4 vi = *reinterpret_cast<const float4 *>(at(eval, ro));
+      h = fmaf((float)xb[ci.x], vi.x, h);
+      h = fmaf((float)xb[ci.y], vi.y, h);
+      h = fmaf((float)xb[ci.z], vi.z, h);
+      h = fmaf((float)xb[ci.w], vi.w, h);
+    }
+    const float de = xj != 0.0f ? -h : h;
+    const bool acc = de < thr && c.j < n;
+    lds_order();
+    td[c.j] = acc ? de : 0.0f;
+    if (acc) xb[c.j] = xj != 0.0f ? 0 : 1;
+    lds_order();
+  };
+  for (int t = 0; t < S; ++t) {
+    const float ts = use_tsr ? tsr[d.rep_off + r] : tscale[tb + t];
+    Site sa = fetch(sc[0]), sb;
+    int jn = sc[G];
+    for (int j4 = 4 * s; j4 < n; j4 += 4 * G) {
+      const uint4 o = philox4x32_10(
+          make_uint4((uint32_t)(j4 >> 2), r, (uint32_t)(tb + t), id | TAG_SWEEP_THR), k0, k1);
+      *reinterpret_cast<float4 *>(td + j4) = make_float4(neg_ln_u(o.x) * ts, neg_ln_u(o.y) * ts,
+                                                         neg_ln_u(o.z) * ts, neg_ln_u(o.w) * ts);
+    }
+    lds_order();
+    const int32_t *sp = sc + 2 * G;
+    for (int k = 0; k < steps; k += 2, sp += 2 * G) {
+      sb = fetch(jn);
+      jn = sp[0];
+      decide(sa);
+      sa = fetch(jn);
+      jn = sp[G];
+      decide(sb);
+    }
+    // the accepted dE, in index order (a rejected site's 0 changes nothing)
+    int j = 0;
+#pragma unroll 4
+    for (; j + 4 <= n; j += 4) {
+      const float4 v = *reinterpret_cast<const float4 *>(td + j);
+      e += (double)v.x;
+      e += (double)v.y;
+      e += (double)v.z;
+      e += (double)v.w;
+    }
+    for (; j < n; ++j) e += (double)td[j];
+    lds_order();
+    if (e < eb) {
+      eb = e;
+      for (int wd = s; wd < words; wd += G) bb[(size_t)wd * Rp] = get_word(xb, wd);
+    }
+  }
+  uint32_t *fb = final_bits + d.state_off + r;
+  for (int wd = s; wd < words; wd += G) fb[(size_t)wd * Rp] = get_word(xb, wd);
+  if (s == 0) {
+    e_best[d.rep_off + r] = eb;
+    e_final[d.rep_off + r] = e;
+  }
+  // the next item's start state overwrites these spins
+  lds_order();
+}
+
+}  // namespace
+
+__global__ __launch_bounds__(64) void csr_sweep_sched_kernel(
+    const CsrInst *__restrict__ inst, const int2 *__restrict__ items,
+    const CsrRun *__restrict__ run, const int4 *__restrict__ ell_col,
+    const float4 *__restrict__ ell_val, const float *__restrict__ diag,
+    const int32_t *__restrict__ sched, const float *__restrict__ tscale,
+    const float *__restrict__ tsr, const uint32_t *__restrict__ init_bits,
+    uint32_t *__restrict__ best_bits, uint32_t *__restrict__ final_bits,
+    double *__restrict__ e_best, double *__restrict__ e_final, int *__restrict__ queue) {
+  extern __shared__ __attribute__((aligned(16))) char slds[];
+  const int lane = threadIdx.x;
+  const int num_items = run->num_items, S = run->num_sweeps, Rp = run->Rp;
+  const uint32_t k0 = run->k0, k1 = run->k1;
+  const uint32_t base = run->instance_base;
+  const int init_mode = run->init_mode, tb = run->sweep_base, use_tsr = run->use_tsr;
+  for (;;) {
+    int it = 0;
+    if (lane == 0) it = atomicAdd(queue, 1);
+    it = __builtin_amdgcn_readfirstlane(it);
+    if (it >= num_items) break;
+    const int2 wi = items[it];
+    const CsrInst d = inst[wi.x];
+    const int g = __builtin_amdgcn_readfirstlane(d.isites);
+#define OS_SCHED_ITEM(GG)                                                                      \
+  sched_item<GG>(d, wi, slds, lane, S, Rp, k0, k1, base, init_mode, tb, use_tsr, tsr, ell_col, \
+                 ell_val, diag, sched, tscale, init_bits, best_bits, final_bits, e_best, e_final)
+    if (g == 4)
+      OS_SCHED_ITEM(4);
+    else if (g == 8)
+      OS_SCHED_ITEM(8);
+    else
+      OS_SCHED_ITEM(16);
+#undef OS_SCHED_ITEM
+  }
+}
+
 // FP64 energy of states given as planes: E = sum_j x_j (Q_jj + sum_{l>j} Q_jl x_l),
 // the reference's energy function (upper triangle incl. diagonal), with the
 // double-precision couplings of the CSR input.  Work-group = item (64
@@ -724,6 +975,33 @@ int csr_lds_bytes(int waves, int max_words) { return waves * max_words * 64 * 4;
 
 void launch_csr_queue_reset(hipStream_t st, int *queue) {
   csr_queue_reset_kernel<<<1, 64, 0, st>>>(queue);
+  OS_HIP_CHECK(hipGetLastError());
+}
+
+int csr_sched_lds_bytes(int n, int G) {
+  const int words = (n + 1 + 31) / 32;
+  return 64 / G * (4 * sched_tstride(n) + sched_bstride(words));
+}
+
+int csr_sched_max_groups_per_cu(int lds) {
+  int blocks = 0;
+  OS_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, csr_sweep_sched_kernel, 64,
+                                                           (size_t)lds));
+  return blocks;
+}
+
+void launch_csr_sched_sweeps(hipStream_t st, int groups, int lds, const CsrInst *inst,
+                             const int2 *items, const CsrRun *run, const int4 *ell_col,
+                             const float4 *ell_val, const float *diag, const int32_t *sched,
+                             const float *tscale, const float *tsr, const uint32_t *init_bits,
+                             uint32_t *best_bits, uint32_t *final_bits, double *e_best,
+                             double *e_final, int *queue) {
+  if (lds > 65536)
+    OS_HIP_CHECK(hipFuncSetAttribute((const void *)csr_sweep_sched_kernel,
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+  csr_sweep_sched_kernel<<<groups, 64, lds, st>>>(inst, items, run, ell_col, ell_val, diag, sched,
+                                                  tscale, tsr, init_bits, best_bits, final_bits,
+                                                  e_best, e_final, queue);
   OS_HIP_CHECK(hipGetLastError());
 }
 

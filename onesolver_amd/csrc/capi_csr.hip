@@ -7,9 +7,10 @@
 // kernel, then recomputes the FP64 energy of every best state; the three
 // launches (counter reset, sweeps, energies) are captured once into a
 // hipGraph and replayed, the run parameters living in device memory.  The
-// launch shape (waves per work-group, resident work-groups and, for the
-// colour-class site order, sites per wave step) is picked by timing short
-// runs of the candidates on the batch itself.  Every instance is coloured
+// launch shape (waves per work-group, resident work-groups, the index order's
+// kernel and sites per wave step) is picked by timing short runs of the
+// candidates on the batch itself; an untuned index-order run keeps 64 replicas
+// a wave.  Every instance is coloured
 // greedily when the batch is created (index order, smallest colour free of
 // lower-index neighbours) for the colour-class site order.
 #include <algorithm>
@@ -55,9 +56,21 @@ struct CsrBatch {
   // replica exchange rounds on the GPU: slots, replicas at slots, scales
   DevBuf pt_slots;
   int num_items = 0;
-  // launch shape chosen by the tuner (0: not tuned); reg: row-prefetching kernel
+  // index order: kernel and launch shape chosen by the tuner (waves 0: not tuned)
+  enum Seq { kPlain = 0, kPrefetch = 1, kSched = 2 };
   int waves = 0, groups = 0;
-  bool reg = false;
+  int seq = kPlain;
+  // scheduled kernel: every instance's schedules at 4, 8 and 16 sites per step,
+  // the policy in use (s_sites; 0: none tried) and its work items ((instance,
+  // group of 64/isites replicas)), built for (items_s_sites, items_s_Rp)
+  struct Sched {
+    int32_t isites, steps;
+    int64_t off;
+  };
+  std::vector<Sched> h_sched[3];
+  DevBuf sched, items_s;
+  int num_items_s = 0, s_sites = 0, items_s_sites = 0, items_s_Rp = 0;
+  int s_lds = 0;  // LDS of a wave: the largest of the batch
   int max_width = 0;
   // colour-class site order: its launch shape (0: not tuned), the policy
   // that gives each instance its sites per step (c_uniform: one value for
@@ -76,8 +89,8 @@ struct CsrBatch {
   hipGraphExec_t gexec = nullptr;
   int g_waves = 0, g_groups = 0, g_Rp = 0, g_mode = 0, g_uniform = 0, g_limit = 0;
   bool g_energy = false;  // the graph ends with the FP64 energies of the best states
-  bool g_reg = false;
-  const void *g_tscale = nullptr, *g_items_c = nullptr;
+  int g_seq = 0, g_s_sites = 0;
+  const void *g_tscale = nullptr, *g_items_c = nullptr, *g_items_s = nullptr;
 
   void drop_graph() {
     if (gexec) (void)hipGraphExecDestroy(gexec);
@@ -90,13 +103,13 @@ struct CsrBatch {
     for (auto *b : {&d_inst, &ell_col, &ell_val, &diag, &diag64, &row_ptr, &col, &val64, &items,
                     &run, &tscale, &init, &best, &fin, &eb, &ef, &e64, &queue, &marg, &corder,
                     &cstart, &items_c, &pell_col, &pell_val, &pdiag, &pop_best, &pop_eb,
-                    &pop_anc, &tsr, &pt_slots})
+                    &pop_anc, &tsr, &pt_slots, &sched, &items_s})
       b->release();
   }
 
-  // mode 0: sequential sweeps with shape (rg, w, g); mode 1: colour classes
+  // mode 0: index-order sweeps with shape (sq, w, g); mode 1: colour classes
   // with w waves and g work-groups over the items in items_c
-  void enqueue(bool rg, int w, int g, bool energy) {
+  void enqueue(int sq, int w, int g, bool energy) {
     hipStream_t st = ctx->stream;
     launch_csr_queue_reset(st, queue.as<int>());
     if (mode == 1)
@@ -108,8 +121,15 @@ struct CsrBatch {
                             best.as<uint32_t>(),
                             fin.as<uint32_t>(), eb.as<double>(), ef.as<double>(),
                             queue.as<int>());
+    else if (sq == kSched)
+      launch_csr_sched_sweeps(st, g, s_lds, d_inst.as<CsrInst>(), items_s.as<int2>(),
+                              run.as<CsrRun>(), ell_col.as<int4>(), ell_val.as<float4>(),
+                              diag.as<float>(), sched.as<int32_t>(), tscale.as<float>(),
+                              tsr.as<float>(), init.as<uint32_t>(), best.as<uint32_t>(),
+                              fin.as<uint32_t>(), eb.as<double>(), ef.as<double>(),
+                              queue.as<int>());
     else
-      launch_csr_sweeps(st, rg, w, g, max_words, d_inst.as<CsrInst>(), items.as<int2>(),
+      launch_csr_sweeps(st, sq == kPrefetch, w, g, max_words, d_inst.as<CsrInst>(), items.as<int2>(),
                         run.as<CsrRun>(), ell_col.as<int4>(), ell_val.as<float4>(),
                         diag.as<float>(), tscale.as<float>(), tsr.as<float>(),
                         init.as<uint32_t>(), best.as<uint32_t>(), fin.as<uint32_t>(),
@@ -256,18 +276,103 @@ void col_items(CsrBatch &b, int uniform, int limit) {
   b.items_c_Rp = b.Rp;
 }
 
+// Schedules of an instance for the scheduled index-order kernel at G = 4, 8 and
+// 16 sites per step: each site goes to the first step with room after every
+// lower-index site that it reads or that reads it.  A schedule that fills less
+// than half of its slots is left out and the next smaller G stands in for it.
+void build_schedules(const CsrInst &d, const int32_t *rp, const int32_t *cl,
+                     std::vector<int32_t> &out, CsrBatch::Sched (&made)[3]) {
+  const int n = d.n;
+  std::vector<int32_t> earliest(n), fill, next, step(n);
+  for (int k = 0; k < 3; ++k) {
+    const int G = 4 << k;
+    std::fill(earliest.begin(), earliest.end(), 0);
+    fill.assign((size_t)n + 1, 0);
+    next.resize((size_t)n + 1);  // union-find: the first step from here with room
+    std::iota(next.begin(), next.end(), 0);
+    int steps = 0;
+    for (int j = 0; j < n; ++j) {
+      int e = earliest[j];
+      for (int q = rp[j]; q < rp[j + 1]; ++q)
+        if (cl[q] < j) e = std::max(e, step[cl[q]] + 1);
+      int f = e;
+      while (next[f] != f) f = next[f] = next[next[f]];
+      step[j] = f;
+      if (++fill[f] == G) next[f] = f + 1;
+      steps = std::max(steps, f + 1);
+      for (int q = rp[j]; q < rp[j + 1]; ++q)
+        if (cl[q] > j) earliest[cl[q]] = std::max(earliest[cl[q]], f + 1);
+    }
+    steps += steps & 1;
+    if (k > 0 && (int64_t)steps * G > 2 * (int64_t)n + 64) {
+      made[k] = made[k - 1];
+      continue;
+    }
+    const size_t at = out.size();
+    out.resize(at + (size_t)(steps + 2) * G, n);  // two idle steps follow
+    std::fill(fill.begin(), fill.end(), 0);
+    for (int j = 0; j < n; ++j) out[at + (size_t)step[j] * G + fill[step[j]]++] = j;
+    made[k] = {G, steps, (int64_t)at};
+  }
+}
+
+// Sets every instance's schedule for `sites` (4, 8 or 16) sites per step and
+// builds the scheduled kernel's work items, longest first.
+void sched_items(CsrBatch &b, int sites) {
+  if (b.items_s_sites == sites && b.items_s_Rp == b.Rp) return;
+  const int k = sites == 4 ? 0 : sites == 8 ? 1 : 2;
+  std::vector<int> order(b.I);
+  std::iota(order.begin(), order.end(), 0);
+  int lds = 0;
+  for (int i = 0; i < b.I; ++i) {
+    CsrInst &d = b.inst[i];
+    d.isites = b.h_sched[k][i].isites;
+    d.steps = b.h_sched[k][i].steps;
+    d.sched_off = b.h_sched[k][i].off;
+    lds = std::max(lds, csr_sched_lds_bytes(d.n, d.isites));
+  }
+  auto work = [&](int i) { return (int64_t)b.inst[i].steps * (b.inst[i].width + 8); };
+  std::stable_sort(order.begin(), order.end(), [&](int a, int c) { return work(a) > work(c); });
+  std::vector<int2> items;
+  for (int i : order)
+    for (int g = 0; g < b.Rp / (64 / b.inst[i].isites); ++g) items.push_back(make_int2(i, g));
+  hipStream_t s = b.ctx->stream;
+  OS_HIP_CHECK(hipMemcpyAsync(b.d_inst.ptr, b.inst.data(), sizeof(CsrInst) * b.I,
+                              hipMemcpyHostToDevice, s));
+  b.items_s.ensure(sizeof(int2) * std::max<size_t>(items.size(), 1));
+  OS_HIP_CHECK(hipMemcpyAsync(b.items_s.ptr, items.data(), sizeof(int2) * items.size(),
+                              hipMemcpyHostToDevice, s));
+  OS_HIP_CHECK(hipStreamSynchronize(s));
+  b.num_items_s = (int)items.size();
+  b.s_lds = lds;
+  b.items_s_sites = sites;
+  b.items_s_Rp = b.Rp;
+}
+
+// Work-groups of the scheduled kernel at `sites` sites per step, 0 where an
+// instance does not fit the LDS (the items are then not built).
+int sched_groups(CsrBatch &b, int sites) {
+  const int k = sites == 4 ? 0 : sites == 8 ? 1 : 2;
+  for (int i = 0; i < b.I; ++i)
+    if (csr_sched_lds_bytes(b.inst[i].n, b.h_sched[k][i].isites) > 160 * 1024) return 0;
+  sched_items(b, sites);
+  return std::min(b.ctx->num_cus * csr_sched_max_groups_per_cu(b.s_lds), b.num_items_s);
+}
+
 // The run parameters in device memory for the launch enqueue() makes.
-void put_run(CsrBatch &b, CsrRun r) {
-  r.num_items = b.mode == 1 ? b.num_items_c : b.num_items;
+void put_run(CsrBatch &b, CsrRun r, int sq) {
+  r.num_items = b.mode == 1               ? b.num_items_c
+                : sq == CsrBatch::kSched ? b.num_items_s
+                                          : b.num_items;
   OS_HIP_CHECK(hipMemcpyAsync(b.run.ptr, &r, sizeof(CsrRun), hipMemcpyHostToDevice,
                               b.ctx->stream));
 }
 
-float time_launch(CsrBatch &b, bool rg, int w, int g) {
+float time_launch(CsrBatch &b, int sq, int w, int g) {
   Ctx &c = *b.ctx;
-  b.enqueue(rg, w, g, false);  // warm-up
+  b.enqueue(sq, w, g, false);  // warm-up
   OS_HIP_CHECK(hipEventRecord(c.ev_start, c.stream));
-  b.enqueue(rg, w, g, false);
+  b.enqueue(sq, w, g, false);
   OS_HIP_CHECK(hipEventRecord(c.ev_stop, c.stream));
   OS_HIP_CHECK(hipEventSynchronize(c.ev_stop));
   float ms = 0.f;
@@ -287,7 +392,7 @@ void tune_col(CsrBatch &b, const CsrRun &full) {
   float best_ms = 0.f;
   for (int limit : {1 << 30, 512, 256, 128, 64, 0}) {
     col_items(b, 0, limit);
-    put_run(b, probe);
+    put_run(b, probe, CsrBatch::kPlain);
     for (int w : {1, 2, 4}) {
       const int maxb = csr_col_max_groups_per_cu(w, b.c_plane_words);
       if (maxb < 1) continue;
@@ -295,7 +400,7 @@ void tune_col(CsrBatch &b, const CsrRun &full) {
       if (maxb > 1) gpcs.push_back(std::max(1, maxb / 2));
       for (int gpc : gpcs) {
         const int g = std::max(1, std::min(c.num_cus * gpc, (b.num_items_c + w - 1) / w));
-        const float ms = time_launch(b, false, w, g);
+        const float ms = time_launch(b, CsrBatch::kPlain, w, g);
         if (b.c_waves == 0 || ms < best_ms) {
           best_ms = ms;
           b.c_waves = w;
@@ -309,30 +414,39 @@ void tune_col(CsrBatch &b, const CsrRun &full) {
   OS_REQUIRE(b.c_waves > 0, "csr batch: no colour-kernel shape fits");
 }
 
-// Times the candidate launch shapes on a short run of the batch itself.
+// Times the candidate kernels and launch shapes on a short run of the batch
+// itself.
 void tune(CsrBatch &b, const CsrRun &full) {
   Ctx &c = *b.ctx;
   CsrRun probe = full;
   probe.num_sweeps = std::min(full.num_sweeps, 2);
-  put_run(b, probe);
   float best_ms = 0.f;
-  for (const bool rg : {false, true}) {
+  auto take = [&](int sq, int w, int g, int sites) {
+    const float ms = time_launch(b, sq, w, g);
+    if (b.waves == 0 || ms < best_ms) {
+      best_ms = ms;
+      b.seq = sq;
+      b.waves = w;
+      b.groups = g;
+      b.s_sites = sites;
+    }
+  };
+  for (int sites : {4, 8, 16}) {
+    const int g = sched_groups(b, sites);
+    if (g < 1) continue;
+    put_run(b, probe, CsrBatch::kSched);
+    take(CsrBatch::kSched, 1, g, sites);
+  }
+  put_run(b, probe, CsrBatch::kPlain);
+  for (const int sq : {CsrBatch::kPlain, CsrBatch::kPrefetch}) {
+    const bool rg = sq == CsrBatch::kPrefetch;
     if (rg && !csr_pf_eligible(b.max_width)) continue;
     for (int w : {1, 2, 4}) {
       const int maxb = csr_max_groups_per_cu(rg, w, b.max_words);
       if (maxb < 1) continue;
       std::vector<int> gpcs{maxb};
       if (maxb > 1) gpcs.push_back(std::max(1, maxb / 2));
-      for (int gpc : gpcs) {
-        const int g = std::max(1, std::min(c.num_cus * gpc, (b.num_items + w - 1) / w));
-        const float ms = time_launch(b, rg, w, g);
-        if (b.waves == 0 || ms < best_ms) {
-          best_ms = ms;
-          b.reg = rg;
-          b.waves = w;
-          b.groups = g;
-        }
-      }
+      for (int gpc : gpcs) take(sq, w, std::max(1, std::min(c.num_cus * gpc, (b.num_items + w - 1) / w)), 0);
     }
   }
   OS_REQUIRE(b.waves > 0, "csr batch: no launch shape fits (instance too large for LDS)");
@@ -349,9 +463,10 @@ void put_tscale(CsrBatch &b, const float *ts, int S) {
 }
 
 struct Shape {
-  bool rg;
+  int seq;
   int waves, groups;
   int uniform, limit;  // colour-class policy (mode 1)
+  int s_sites;         // sites per step of the scheduled kernel (mode 0)
 };
 
 // The launch shape of a run in `site_order` (tuned on first use when `tune`).
@@ -362,10 +477,11 @@ Shape select_shape(CsrBatch &b, const CsrRun &run, int site_order, bool tune_it)
     if (tune_it) {
       tune(b, run);
     } else {
-      b.reg = csr_pf_eligible(b.max_width);
+      b.seq = csr_pf_eligible(b.max_width) ? CsrBatch::kPrefetch : CsrBatch::kPlain;
       b.waves = 1;
-      b.groups = std::max(1, std::min(c.num_cus * csr_max_groups_per_cu(b.reg, 1, b.max_words),
-                                      b.num_items));
+      b.groups = std::max(
+          1, std::min(c.num_cus * csr_max_groups_per_cu(b.seq == CsrBatch::kPrefetch, 1, b.max_words),
+                      b.num_items));
     }
   }
   // OS_CSR_COLOUR_SITES (4, 8 or 16) fixes the colour kernel's sites per step
@@ -402,8 +518,13 @@ Shape select_shape(CsrBatch &b, const CsrRun &run, int site_order, bool tune_it)
     }
   }
   if (b.mode == 1) col_items(b, b.c_uniform, b.c_limit);
+  if (b.mode == 0 && b.seq == CsrBatch::kSched) {
+    // another replica count leaves other items, not another kernel
+    b.groups = std::max(1, sched_groups(b, b.s_sites));
+  }
   Shape sh;
-  sh.rg = b.mode == 0 && b.reg;
+  sh.seq = b.mode == 0 ? b.seq : CsrBatch::kPlain;
+  sh.s_sites = sh.seq == CsrBatch::kSched ? b.s_sites : 0;
   sh.waves = b.mode == 1 ? b.c_waves : b.waves;
   sh.groups = b.mode == 1 ? b.c_groups : b.groups;
   sh.uniform = b.mode == 1 ? b.c_uniform : 0;
@@ -415,14 +536,14 @@ Shape select_shape(CsrBatch &b, const CsrRun &run, int site_order, bool tune_it)
 // the graph already holds that shape.
 void ensure_graph(CsrBatch &b, const Shape &sh, bool energy) {
   hipStream_t s = b.ctx->stream;
-  if (b.gexec && b.g_mode == b.mode && b.g_reg == sh.rg && b.g_waves == sh.waves &&
+  if (b.gexec && b.g_mode == b.mode && b.g_seq == sh.seq && b.g_s_sites == sh.s_sites && b.g_waves == sh.waves &&
       b.g_groups == sh.groups && b.g_uniform == sh.uniform && b.g_limit == sh.limit &&
-      b.g_items_c == b.items_c.ptr && b.g_Rp == b.Rp && b.g_energy == energy)
+      b.g_items_c == b.items_c.ptr && b.g_items_s == b.items_s.ptr && b.g_Rp == b.Rp && b.g_energy == energy)
     return;
   b.drop_graph();
   OS_HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
   try {
-    b.enqueue(sh.rg, sh.waves, sh.groups, energy);
+    b.enqueue(sh.seq, sh.waves, sh.groups, energy);
   } catch (...) {
     hipGraph_t g = nullptr;
     (void)hipStreamEndCapture(s, &g);
@@ -432,12 +553,14 @@ void ensure_graph(CsrBatch &b, const Shape &sh, bool energy) {
   OS_HIP_CHECK(hipStreamEndCapture(s, &b.graph));
   OS_HIP_CHECK(hipGraphInstantiate(&b.gexec, b.graph, nullptr, nullptr, 0));
   b.g_mode = b.mode;
-  b.g_reg = sh.rg;
+  b.g_seq = sh.seq;
+  b.g_s_sites = sh.s_sites;
   b.g_waves = sh.waves;
   b.g_groups = sh.groups;
   b.g_uniform = sh.uniform;
   b.g_limit = sh.limit;
   b.g_items_c = b.items_c.ptr;
+  b.g_items_s = b.items_s.ptr;
   b.g_Rp = b.Rp;
   b.g_energy = energy;
   b.g_tscale = b.tscale.ptr;
@@ -598,7 +721,8 @@ int os_csr_batch_create(os_ctx *ctx_, int32_t num_instances, const int32_t *n,
     const int nd = (int)ds.size();
     std::vector<int32_t> ell_c((size_t)ell);
     std::vector<float> ell_v((size_t)ell, 0.0f), dg((size_t)spins);
-    std::vector<std::vector<int32_t>> cst(nd), cord(nd);
+    std::vector<std::vector<int32_t>> cst(nd), cord(nd), sch(nd);
+    for (auto &h : b->h_sched) h.resize(nd);
     std::vector<const char *> err(nd, nullptr);
     os::host_parallel_for(nd, [&](int i) {
       os::CsrInst &d = ds[i];
@@ -644,16 +768,22 @@ int os_csr_batch_create(os_ctx *ctx_, int32_t num_instances, const int32_t *n,
       std::vector<int32_t> fill(start.begin(), start.end() - 1);
       cord[i].resize(ni);
       for (int j = 0; j < ni; ++j) cord[i][fill[colour[j]]++] = j;
+      CsrBatch::Sched made[3];
+      os::build_schedules(d, rp, cl, sch[i], made);
+      for (int k = 0; k < 3; ++k) b->h_sched[k][i] = made[k];
     });
     // the first failing instance in order, as a serial pass reports it
     for (int i = 0; i < nd; ++i) OS_REQUIRE(!err[i], err[i]);
     OS_REQUIRE(!bad_msg, bad_msg);
-    // Pass 3 (serial): class offsets and the concatenated class arrays
+    // Pass 3 (serial): class and schedule offsets and the concatenated arrays
+    std::vector<int32_t> h_sched;
     for (int i = 0; i < nd; ++i) {
       os::CsrInst &d = ds[i];
       d.class_off = (int64_t)b->h_cstart.size();
       b->h_cstart.insert(b->h_cstart.end(), cst[i].begin(), cst[i].end());
       b->h_order.insert(b->h_order.end(), cord[i].begin(), cord[i].end());
+      for (auto &h : b->h_sched) h[i].off += (int64_t)h_sched.size();
+      h_sched.insert(h_sched.end(), sch[i].begin(), sch[i].end());
       b->max_words = std::max(b->max_words, d.words);
       b->max_width = std::max(b->max_width, d.width);
       b->total_words += d.words;
@@ -712,6 +842,9 @@ int os_csr_batch_create(os_ctx *ctx_, int32_t num_instances, const int32_t *n,
                                   hipMemcpyHostToDevice, s));
       OS_HIP_CHECK(hipStreamSynchronize(s));
     }
+    b->sched.ensure(sizeof(int32_t) * h_sched.size());
+    OS_HIP_CHECK(hipMemcpyAsync(b->sched.ptr, h_sched.data(), sizeof(int32_t) * h_sched.size(),
+                                hipMemcpyHostToDevice, s));
     b->corder.ensure(sizeof(int32_t) * b->h_order.size());
     b->cstart.ensure(sizeof(int32_t) * b->h_cstart.size());
     OS_HIP_CHECK(hipMemcpyAsync(b->corder.ptr, b->h_order.data(),
@@ -787,13 +920,13 @@ int os_csr_batch_anneal(os_csr_batch *b_, const os_csr_params *p, double *best_e
       OS_HIP_CHECK(hipStreamSynchronize(s));
     }
     const os::Shape sh = os::select_shape(b, run, p->site_order, p->tune != 0);
-    os::put_run(b, run);
+    os::put_run(b, run, sh.seq);
     if (p->use_graph) os::ensure_graph(b, sh, true);
     OS_HIP_CHECK(hipEventRecord(c.ev_start, s));
     if (p->use_graph)
       OS_HIP_CHECK(hipGraphLaunch(b.gexec, s));
     else
-      b.enqueue(sh.rg, sh.waves, sh.groups, true);
+      b.enqueue(sh.seq, sh.waves, sh.groups, true);
     OS_HIP_CHECK(hipEventRecord(c.ev_stop, s));
     os::collect(b, R, b.best, b.fin, run_best_energies ? &b.eb : nullptr, best_energies,
                 run_best_energies, best_states, final_states, inst_best_energy,
@@ -863,11 +996,11 @@ int os_csr_batch_population(os_csr_batch *b_, const os_csr_population_params *p,
     for (int k = 0; k < K; ++k) {
       run.sweep_base = k * theta;
       run.init_mode = k > 0 ? 1 : 0;
-      os::put_run(b, run);
+      os::put_run(b, run, sh.seq);
       if (p->use_graph)
         OS_HIP_CHECK(hipGraphLaunch(b.gexec, s));
       else
-        b.enqueue(sh.rg, sh.waves, sh.groups, false);
+        b.enqueue(sh.seq, sh.waves, sh.groups, false);
       // best of every replica index: the step's best where it is lower
       os::launch_csr_pop_best(s, b.d_inst.as<os::CsrInst>(), b.items.as<int2>(), b.num_items, Rp,
                               k == 0, b.eb.as<double>(), b.best.as<uint32_t>(),
@@ -989,11 +1122,11 @@ int os_csr_batch_tempering(os_csr_batch *b_, const os_csr_tempering_params *p,
       run.num_sweeps = ns;
       run.init_mode = s0 > 0 ? 1 : 0;
       run.use_tsr = 1;
-      os::put_run(b, run);
+      os::put_run(b, run, sh.seq);
       if (p->use_graph)
         OS_HIP_CHECK(hipGraphLaunch(b.gexec, s));
       else
-        b.enqueue(sh.rg, sh.waves, sh.groups, false);
+        b.enqueue(sh.seq, sh.waves, sh.groups, false);
       ++segments;
       os::launch_csr_pop_best(s, b.d_inst.as<os::CsrInst>(), b.items.as<int2>(), b.num_items, Rp,
                               s0 == 0, b.eb.as<double>(), b.best.as<uint32_t>(),
@@ -1068,7 +1201,7 @@ int os_csr_batch_launch_shape(os_csr_batch *b_, int32_t *waves_per_group, int32_
     const CsrBatch &b = *reinterpret_cast<CsrBatch *>(b_);
     if (waves_per_group) *waves_per_group = b.waves;
     if (groups) *groups = b.groups;
-    if (prefetch) *prefetch = b.reg ? 1 : 0;
+    if (prefetch) *prefetch = b.seq;
   });
 }
 

@@ -120,6 +120,9 @@ struct CsrInst {
   int64_t rep_off;    // first replica in per-replica arrays (Rp per instance)
   int64_t class_off;  // first entry in the class starts (ncol + 1 per instance)
   int32_t sites;      // colour-class kernel: sites per wave step (4, 8 or 16)
+  int32_t isites;     // scheduled index-order kernel: sites per wave step (4, 8 or 16)
+  int64_t sched_off;  // its schedule: isites slots a step, slot n idle
+  int32_t steps;      // steps in it (even; two idle steps follow)
   int32_t pad_;
 };
 // The device arrays of a sparse batch, for kernels outside the annealer (the
@@ -150,6 +153,16 @@ struct CsrRun {
 };
 int csr_lds_bytes(int waves, int max_words);
 // pf: the row-prefetching kernel (batches within csr_pf_eligible)
+// Scheduled index-order kernel: LDS bytes of a wave for an n-spin instance at G
+// sites per step, and its launch (one wave a work-group).
+int csr_sched_lds_bytes(int n, int G);
+int csr_sched_max_groups_per_cu(int lds);
+void launch_csr_sched_sweeps(hipStream_t st, int groups, int lds, const CsrInst *inst,
+                             const int2 *items, const CsrRun *run, const int4 *ell_col,
+                             const float4 *ell_val, const float *diag, const int32_t *sched,
+                             const float *tscale, const float *tsr, const uint32_t *init_bits,
+                             uint32_t *best_bits, uint32_t *final_bits, double *e_best,
+                             double *e_final, int *queue);
 bool csr_pf_eligible(int max_width);
 int csr_max_groups_per_cu(bool pf, int waves, int max_words);
 void launch_csr_queue_reset(hipStream_t st, int *queue);

@@ -126,6 +126,37 @@ def test_csr_prefetch_kernel_matches_oracle(ctx, tune):
     b.close()
 
 
+def _ring(n, seed):
+    """A cycle with real weights: index order leaves no two neighbours of it for
+    the same step."""
+    rng = np.random.default_rng(seed)
+    w = np.float32(rng.normal(size=n)).astype(np.float64)
+    cl = np.stack([(np.arange(n) - 1) % n, (np.arange(n) + 1) % n], 1)
+    vl = np.stack([w[(np.arange(n) - 1) % n], w], 1)
+    return (np.arange(0, 2 * n + 1, 2, dtype=np.int32), cl.astype(np.int32).ravel(), vl.ravel(),
+            np.float32(rng.normal(size=n)).astype(np.float64))
+
+
+@pytest.mark.parametrize("sizes", [
+    [(4, 3)], [(15, 4), (16, 5), (17, 4)], [(31, 4), (32, 3), (33, 4)], [(64, 12), (65, 16)],
+    [(1024, 8), (127, 6), (8, 3)], [(2048, 9)], [(3000, 3)]])
+def test_csr_tuned_index_order_matches_oracle(ctx, sizes):
+    """The kernel a tuned index-order run picks for few waves updates up to 16
+    uncoupled sites together: edges of its steps and words, rows of one, two and
+    more chunks, chains it cannot pack, isolated spins, and a run that goes on
+    with another number of replicas."""
+    insts = [instances.regular_csr(n, d, seed=5, instance=i) for i, (n, d) in enumerate(sizes)]
+    insts += [_ring(50, 9), _partly_isolated(45, 20, 3)]
+    S = 7
+    ts = _tscale(S)
+    b = onesolver_amd.CsrBatch(ctx, insts)
+    for R, seed in ((100, 3), (200, 4)):
+        out = b.anneal(R, ts, seed=seed, instance_base=1, final_states=True, tune=True)
+        print(f"[gpu] csr tuned index order {sizes} R={R} shape={b.launch_shape()}", flush=True)
+        _check_against_oracle(out, insts, ts, R, seed, 1)
+    b.close()
+
+
 def test_csr_graph_replays_with_new_parameters(ctx):
     insts = _batch()
     R, S = 64, 12
