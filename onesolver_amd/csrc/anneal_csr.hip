@@ -324,6 +324,65 @@ __global__ __launch_bounds__(64 * kW) void csr_sweep_pf_kernel(
   }
 }
 
+namespace {
+
+// Spins of a replica one byte each, replica by replica: bytes from one replica's
+// to the next's.
+__host__ __device__ inline int spin_stride(int words) { return words * 32 + 16; }
+
+// Order of this wave's LDS accesses as written (the LDS serves a wave's accesses
+// in order; only the compiler has to keep it).
+__device__ __forceinline__ void lds_order() {
+  __builtin_amdgcn_wave_barrier();
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+
+// Spins 32 wd .. 32 wd + 31 between bytes and a word.
+__device__ __forceinline__ void put_word(uint8_t *xb, int wd, uint32_t v) {
+  uint32_t *b = reinterpret_cast<uint32_t *>(xb + 32 * wd);
+#pragma unroll
+  for (int m = 0; m < 8; ++m) b[m] = (((v >> (4 * m)) & 15u) * 0x00204081u) & 0x01010101u;
+}
+__device__ __forceinline__ uint32_t get_word(const uint8_t *xb, int wd) {
+  const uint32_t *b = reinterpret_cast<const uint32_t *>(xb + 32 * wd);
+  uint32_t v = 0u;
+#pragma unroll
+  for (int m = 0; m < 8; ++m) v |= ((b[m] * 0x01020408u) >> 24) << (4 * m);
+  return v;
+}
+
+constexpr int kColThresholdBytes = 8 * 64 * 4;
+
+// Spins of the colour-class kernel's 64/G replicas in LDS, either a byte each
+// (replica by replica) or bit-packed (word by word, replicas side by side).
+template <int G>
+struct ByteSpins {
+  uint8_t *p;
+  __device__ ByteSpins(char *at, int rr, int words)
+      : p(reinterpret_cast<uint8_t *>(at) + rr * spin_stride(words)) {}
+  __device__ __forceinline__ uint32_t operator()(int j) const { return p[j]; }
+  __device__ __forceinline__ void flip(int j, uint32_t x) const { p[j] = (uint8_t)(x ^ 1u); }
+  __device__ __forceinline__ void put(int wd, uint32_t v) const { put_word(p, wd, v); }
+  __device__ __forceinline__ uint32_t word(int wd) const { return get_word(p, wd); }
+};
+template <int G>
+struct BitSpins {
+  uint32_t *p;
+  __device__ BitSpins(char *at, int rr, int) : p(reinterpret_cast<uint32_t *>(at) + rr) {}
+  // the bit-field extract reads only the low 5 bits of its offset
+  __device__ __forceinline__ uint32_t operator()(int j) const {
+    return __builtin_amdgcn_ubfe(p[(j >> 5) * (64 / G)], (uint32_t)j, 1u);
+  }
+  // sites of one class can share a word
+  __device__ __forceinline__ void flip(int j, uint32_t) const {
+    atomicXor(&p[(j >> 5) * (64 / G)], 1u << (j & 31));
+  }
+  __device__ __forceinline__ void put(int wd, uint32_t v) const { p[wd * (64 / G)] = v; }
+  __device__ __forceinline__ uint32_t word(int wd) const { return p[wd * (64 / G)]; }
+};
+
+}  // namespace
+
 // Colour-class variant.  The sites of an instance are visited class by class
 // (greedy colouring: no two sites of a class are coupled), every class in
 // ascending index order; within a class the updates are independent, so a
@@ -334,22 +393,27 @@ __global__ __launch_bounds__(64 * kW) void csr_sweep_pf_kernel(
 // field order and dE; the FP64 running energy adds the dE of a sweep per
 // lane and then over the G lanes of a replica (and the start energy, per
 // site as the oracle computes it, sums sites s, s+G, ... in lane s, then over
-// the G lanes).  Thresholds are computed for
-// windows of 4G positions (one Philox call per lane, four logarithms) into
-// LDS.  Flips are atomic XORs on the LDS planes, since sites of one class
-// can share a word.
+// the G lanes).  Thresholds are drawn 4G positions at a time (one Philox call
+// per lane, four logarithms) into an LDS ring of 8G.
+//
+// A step's latency bounds it (1024 waves hold the largest instances' chains, 40 %
+// of the vector issue slots used), so the host lists the steps (no class
+// bookkeeping in the kernel), all of a row's neighbours are read before the
+// first is used (rows of one chunk have their own code) and a spin is a byte
+// where that fits.  Measured: 96 instances of 64 .. 2048 spins, degrees 3 .. 8,
+// 256 replicas, 512 sweeps 46.9 -> 36.4 ms; with bit-packed spins 42.3.
 
 // One work item of the colour-class kernel: replicas [wi.y * 64/G, +64/G) of
-// instance d, G sites per step; xs: this wave's LDS planes, then the
-// threshold window.
-template <int G>
+// instance d, G sites per step; lds: this wave's thresholds, then its spins.
+// NCH: 1 for rows of at most 4 couplings, else 2.
+template <int G, int NCH, class Spins>
 __device__ __forceinline__ void col_item(
-    const CsrInst &d, int2 wi, uint32_t *xs, int plane_words, int lane, int S, int Rp,
+    const CsrInst &d, int2 wi, char *lds, int lane, int S, int Rp,
     uint32_t k0, uint32_t k1, uint32_t base, int init_mode, int tb, int use_tsr,
     const float *__restrict__ tsr,
     const int4 *__restrict__ ell_col, const float4 *__restrict__ ell_val,
     const float *__restrict__ diag, const int32_t *__restrict__ corder,
-    const int32_t *__restrict__ cstart, const int4 *__restrict__ pell_col,
+    const int32_t *__restrict__ csteps, const int4 *__restrict__ pell_col,
     const float4 *__restrict__ pell_val, const float *__restrict__ pdiag,
     const float *__restrict__ tscale, const uint32_t *__restrict__ init_bits,
     uint32_t *__restrict__ best_bits, uint32_t *__restrict__ final_bits,
@@ -357,19 +421,17 @@ __device__ __forceinline__ void col_item(
   static_assert(G == 4 || G == 8 || G == 16, "sites per step");
   constexpr int RW = 64 / G;  // replicas per wave
   const int rr = lane / G, s = lane % G;
-  // thresholds of the positions [win, win + 4G) for the RW replicas
-  float *thw = reinterpret_cast<float *>(xs + plane_words);
-  // bit j of this lane's replica (the bit-field extract reads only the low 5
-  // bits of its offset)
-  auto bit = [&](int j) { return __builtin_amdgcn_ubfe(xs[(j >> 5) * RW + rr], (uint32_t)j, 1u); };
-  const int n = d.n, words = d.words, chunks = d.width >> 2, ncol = d.ncol;
+  // thresholds, position pos at pos mod 8G, then the spins
+  float *thw = reinterpret_cast<float *>(lds) + rr;
+  const Spins x(lds + kColThresholdBytes, rr, d.words);
+  const int n = d.n, words = d.words, chunks = NCH == 1 ? 1 : d.width >> 2;
   const uint32_t r = (uint32_t)(wi.y * RW + rr);
   const uint32_t id = (base + (uint32_t)wi.x) << 8;
   const int4 *ecol = ell_col + (d.ell_off >> 2);
   const float4 *eval = ell_val + (d.ell_off >> 2);
   const float *dg = diag + d.spin_off;
   const int32_t *ord = corder + d.spin_off;
-  const int32_t *cs = cstart + d.class_off;
+  const int32_t *sc = csteps + d.csteps_off + s;
   // the rows and diagonal in visiting order (position pos: site ord[pos])
   const int4 *pcol = pell_col + (d.ell_off >> 2);
   const float4 *pval = pell_val + (d.ell_off >> 2);
@@ -388,9 +450,9 @@ __device__ __forceinline__ void col_item(
     }
     const int valid = n - 32 * wd;
     if (valid < 32) v = valid <= 0 ? 0u : (v & ((1u << valid) - 1u));
-    xs[wd * RW + rr] = v;
+    x.put(wd, v);
   }
-  wave_sync();
+  lds_order();
   // FP64 energy: lane s of a replica sums sites s, s + G, ... (each site as
   // the oracle does: diag + half its set couplings), then the G partial
   // sums are added
@@ -400,28 +462,27 @@ __device__ __forceinline__ void col_item(
     for (int c = 0; c < chunks; ++c) {
       const int4 cc = ecol[(size_t)j * chunks + c];
       const float4 vv = eval[(size_t)j * chunks + c];
-      off = bit(cc.x) ? off + (double)vv.x : off;
-      off = bit(cc.y) ? off + (double)vv.y : off;
-      off = bit(cc.z) ? off + (double)vv.z : off;
-      off = bit(cc.w) ? off + (double)vv.w : off;
+      off = x(cc.x) ? off + (double)vv.x : off;
+      off = x(cc.y) ? off + (double)vv.y : off;
+      off = x(cc.z) ? off + (double)vv.z : off;
+      off = x(cc.w) ? off + (double)vv.w : off;
     }
-    if (bit(j)) e += (double)dg[j] + 0.5 * off;
+    if (x(j)) e += (double)dg[j] + 0.5 * off;
   }
 #pragma unroll
   for (int o = 1; o < G; o <<= 1) e += __shfl_xor(e, o, 64);
   double eb = e;
-  for (int wd = s; wd < words; wd += G) bb[(size_t)wd * Rp] = xs[wd * RW + rr];
+  for (int wd = s; wd < words; wd += G) bb[(size_t)wd * Rp] = x.word(wd);
   for (int t = 0; t < S; ++t) {
     const float ts = use_tsr ? tsr[d.rep_off + r] : tscale[tb + t];
     double de_sum = 0.0;
-    int win = -4 * G;  // no window yet
-    // steps of the sweep: positions [p0, p0 + G) of class c (ending at
-    // c1); the rows of the next step are requested before this one runs
-    int c = 0, p0 = cs[0], c1 = cs[1];
+    int drawn = 0;  // thresholds drawn so far
+    // steps of the sweep: positions p0 .. p0 + G - 1 of one class; a step's
+    // rows are requested a step ahead, its positions two steps ahead
     // the first two chunks of a row travel with the step; rows of more
     // than 8 couplings read the rest when the step runs
     struct Step {
-      int j, pos;
+      int j, v;
       float dj;
       int4 c0, c1;
       float4 v0, v1;
@@ -430,129 +491,126 @@ __device__ __forceinline__ void col_item(
     auto at16 = [](const void *base, uint32_t off) {
       return reinterpret_cast<const char *>(base) + off;
     };
-    auto fetch = [&](int q0) {
+    auto fetch = [&](int v) {
       Step st;
-      const int pos = min(q0 + s, n - 1);
+      const int pos = v & 0x7FFFFFFF;
       const uint32_t ro = (uint32_t)pos * (uint32_t)chunks * 16u;  // row's byte offset
-      st.pos = pos;
+      st.v = v;
       st.j = *reinterpret_cast<const int32_t *>(at16(ord, (uint32_t)pos * 4u));
       st.dj = *reinterpret_cast<const float *>(at16(pdg, (uint32_t)pos * 4u));
       st.c0 = *reinterpret_cast<const int4 *>(at16(pcol, ro));
       st.v0 = *reinterpret_cast<const float4 *>(at16(pval, ro));
-      st.c1 = make_int4(n, n, n, n);
-      st.v1 = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (chunks > 1) {
+      if constexpr (NCH > 1) {
         st.c1 = *reinterpret_cast<const int4 *>(at16(pcol, ro + 16u));
         st.v1 = *reinterpret_cast<const float4 *>(at16(pval, ro + 16u));
       }
       return st;
     };
-    // one step: decides the sites of `cur` after requesting the next
-    // step's rows into `nxt`; false after the sweep's last step.  Two
-    // buffers in turn (no copies between steps).
-    auto step = [&](const Step &cur, Step &nxt) -> bool {
-      int np0 = p0 + G, nc = c, nc1 = c1;
-      if (np0 >= c1) {
-        nc = c + 1;
-        if (nc < ncol) {
-          np0 = cs[nc];
-          nc1 = cs[nc + 1];
-        }
-      }
-      const bool more = nc < ncol;
-      if (more) nxt = fetch(np0);
-      if (p0 + G > win + 4 * G) {
-        // next window: lane (rr, s) draws positions win + 4s .. +3
-        win = p0 & ~3;
-        const uint4 o = philox4x32_10(make_uint4((uint32_t)((win >> 2) + s), r,
+    auto step = [&](const Step &cur) {
+      const int pos = cur.v & 0x7FFFFFFF;
+      if (__builtin_amdgcn_readfirstlane(pos) + G > drawn) {
+        // the next 4G thresholds: lane (rr, s) draws positions drawn + 4s .. +3
+        const uint4 o = philox4x32_10(make_uint4((uint32_t)((drawn >> 2) + s), r,
                                                  (uint32_t)(tb + t), id | TAG_SWEEP_THR),
                                       k0, k1);
+        float *to = thw + ((drawn & (4 * G)) + 4 * s) * RW;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) thw[(4 * s + q) * RW + rr] = neg_ln_u(pick(o, (uint32_t)q)) * ts;
-        wave_sync();
+        for (int q = 0; q < 4; ++q) to[q * RW] = neg_ln_u(pick(o, (uint32_t)q)) * ts;
+        drawn += 4 * G;
+        lds_order();
       }
-      const int pos = p0 + s;
-      const bool active = pos < c1;
-      const float thr = thw[(pos - win) * RW + rr];
+      const float thr = thw[(pos & (8 * G - 1)) * RW];
+      const int j = cur.j;
+      const uint32_t xj = x(j);
       // h + w for a set neighbour bit, h for a clear one: fma(1, w, h) is the
       // rounded sum, fma(0, w, h) is h (up to the sign of a zero h, which no
       // comparison or later sum sees)
       float h = cur.dj;
-      h = fmaf((float)bit(cur.c0.x), cur.v0.x, h);
-      h = fmaf((float)bit(cur.c0.y), cur.v0.y, h);
-      h = fmaf((float)bit(cur.c0.z), cur.v0.z, h);
-      h = fmaf((float)bit(cur.c0.w), cur.v0.w, h);
-      if (chunks > 1) {
-        h = fmaf((float)bit(cur.c1.x), cur.v1.x, h);
-        h = fmaf((float)bit(cur.c1.y), cur.v1.y, h);
-        h = fmaf((float)bit(cur.c1.z), cur.v1.z, h);
-        h = fmaf((float)bit(cur.c1.w), cur.v1.w, h);
+      const float x0 = (float)x(cur.c0.x), x1 = (float)x(cur.c0.y), x2 = (float)x(cur.c0.z),
+                  x3 = (float)x(cur.c0.w);
+      float x4, x5, x6, x7;
+      if constexpr (NCH > 1) {
+        x4 = (float)x(cur.c1.x);
+        x5 = (float)x(cur.c1.y);
+        x6 = (float)x(cur.c1.z);
+        x7 = (float)x(cur.c1.w);
       }
-      for (int cc = 2; cc < chunks; ++cc) {
-        const uint32_t ro = ((uint32_t)cur.pos * (uint32_t)chunks + (uint32_t)cc) * 16u;
-        const int4 ci = *reinterpret_cast<const int4 *>(at16(pcol, ro));
-        const float4 vi = *reinterpret_cast<const float4 *>(at16(pval, ro));
-        h = fmaf((float)bit(ci.x), vi.x, h);
-        h = fmaf((float)bit(ci.y), vi.y, h);
-        h = fmaf((float)bit(ci.z), vi.z, h);
-        h = fmaf((float)bit(ci.w), vi.w, h);
+      h = fmaf(x0, cur.v0.x, h);
+      h = fmaf(x1, cur.v0.y, h);
+      h = fmaf(x2, cur.v0.z, h);
+      h = fmaf(x3, cur.v0.w, h);
+      if constexpr (NCH > 1) {
+        h = fmaf(x4, cur.v1.x, h);
+        h = fmaf(x5, cur.v1.y, h);
+        h = fmaf(x6, cur.v1.z, h);
+        h = fmaf(x7, cur.v1.w, h);
+        for (int cc = 2; cc < chunks; ++cc) {
+          const uint32_t ro = ((uint32_t)pos * (uint32_t)chunks + (uint32_t)cc) * 16u;
+          const int4 ci = *reinterpret_cast<const int4 *>(at16(pcol, ro));
+          const float4 vi = *reinterpret_cast<const float4 *>(at16(pval, ro));
+          h = fmaf((float)x(ci.x), vi.x, h);
+          h = fmaf((float)x(ci.y), vi.y, h);
+          h = fmaf((float)x(ci.z), vi.z, h);
+          h = fmaf((float)x(ci.w), vi.w, h);
+        }
       }
-      const int j = cur.j;
-      const float de = bit(j) ? -h : h;
-      if (active && de < thr) {
-        atomicXor(&xs[(j >> 5) * RW + rr], 1u << (j & 31));
+      const float de = xj ? -h : h;
+      lds_order();
+      if (cur.v >= 0 && de < thr) {
+        x.flip(j, xj);
         de_sum += (double)de;
       }
-      if (!more) return false;
-      // a new class reads this class's flips
-      if (nc != c) wave_sync();
-      p0 = np0;
-      c1 = nc1;
-      c = nc;
-      return true;
+      lds_order();
     };
-    Step sa = fetch(p0), sb = sa;
-    while (step(sa, sb) && step(sb, sa)) {
+    Step sa = fetch(sc[0]), sb;
+    int vn = sc[G];
+    const int32_t *sp = sc + 2 * G;
+    for (int k = 0; k < d.csteps; k += 2, sp += 2 * G) {
+      sb = fetch(vn);
+      vn = sp[0];
+      step(sa);
+      sa = fetch(vn);
+      vn = sp[G];
+      step(sb);
     }
-    wave_sync();
+    lds_order();
 #pragma unroll
     for (int off = 1; off < G; off <<= 1) de_sum += __shfl_xor(de_sum, off, 64);
     e += de_sum;
     if (e < eb) {
       eb = e;
-      for (int wd = s; wd < words; wd += G) bb[(size_t)wd * Rp] = xs[wd * RW + rr];
+      for (int wd = s; wd < words; wd += G) bb[(size_t)wd * Rp] = x.word(wd);
     }
   }
   uint32_t *fb = final_bits + d.state_off + r;
-  for (int wd = s; wd < words; wd += G) fb[(size_t)wd * Rp] = xs[wd * RW + rr];
+  for (int wd = s; wd < words; wd += G) fb[(size_t)wd * Rp] = x.word(wd);
   if (s == 0) {
     e_best[d.rep_off + r] = eb;
     e_final[d.rep_off + r] = e;
   }
   // the next item's start state overwrites these planes
-  wave_sync();
+  lds_order();
 }
 
 // Colour-class sweeps over a batch whose instances each have their own sites
-// per step (CsrInst::sites: 4, 8 or 16).  plane_words: LDS words per wave for
-// the state planes (the largest words * 64/sites of the batch), followed by
-// 4*64 threshold words.
-template <int kW>
-__global__ __launch_bounds__(64 * kW) void csr_sweep_col_kernel(
+// per step (CsrInst::sites: 4, 8 or 16).  spin_bytes: LDS bytes per wave for the
+// spins (csr_col_spin_bytes, the largest of the batch), behind 4*64 thresholds.
+template <template <int> class Spins>
+__global__ __launch_bounds__(256) void csr_sweep_col_kernel(
     const CsrInst *__restrict__ inst, const int2 *__restrict__ items,
     const CsrRun *__restrict__ run, const int4 *__restrict__ ell_col,
     const float4 *__restrict__ ell_val, const float *__restrict__ diag,
-    const int32_t *__restrict__ corder, const int32_t *__restrict__ cstart,
+    const int32_t *__restrict__ corder, const int32_t *__restrict__ csteps,
     const int4 *__restrict__ pell_col, const float4 *__restrict__ pell_val,
     const float *__restrict__ pdiag, const float *__restrict__ tscale,
     const float *__restrict__ tsr, const uint32_t *__restrict__ init_bits,
     uint32_t *__restrict__ best_bits, uint32_t *__restrict__ final_bits,
     double *__restrict__ e_best, double *__restrict__ e_final, int *__restrict__ queue,
-    int plane_words) {
-  extern __shared__ uint32_t lds[];
+    int spin_bytes) {
+  extern __shared__ __attribute__((aligned(16))) char clds[];
   const int w = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
-  uint32_t *xs = lds + (size_t)w * (plane_words + 4 * 64);
+  char *wl = clds + (size_t)w * (spin_bytes + kColThresholdBytes);  // this wave's
   const int num_items = run->num_items, S = run->num_sweeps, Rp = run->Rp;
   const uint32_t k0 = run->k0, k1 = run->k1;
   const uint32_t base = run->instance_base;
@@ -588,10 +646,18 @@ __global__ __launch_bounds__(64 * kW) void csr_sweep_col_kernel(
     const CsrInst d = inst[wi.x];
     const int g = __builtin_amdgcn_readfirstlane(d.sites);
 #define OS_COL_ITEM(GG)                                                                         \
-  col_item<GG>(d, wi, xs, plane_words, lane, S, Rp, k0, k1, base, init_mode, tb, use_tsr, tsr, \
-               ell_col,                                                                        \
-               ell_val, diag, corder, cstart, pell_col, pell_val, pdiag, tscale, init_bits,    \
-               best_bits, final_bits, e_best, e_final)
+  do {                                                                                          \
+    if (d.width == 4)                                                                           \
+      col_item<GG, 1, Spins<GG>>(d, wi, wl, lane, S, Rp, k0, k1, base, init_mode, tb, use_tsr,  \
+                                 tsr, ell_col, ell_val, diag, corder, csteps, pell_col,         \
+                                 pell_val, pdiag, tscale, init_bits, best_bits, final_bits,     \
+                                 e_best, e_final);                                              \
+    else                                                                                        \
+      col_item<GG, 2, Spins<GG>>(d, wi, wl, lane, S, Rp, k0, k1, base, init_mode, tb, use_tsr,  \
+                                 tsr, ell_col, ell_val, diag, corder, csteps, pell_col,         \
+                                 pell_val, pdiag, tscale, init_bits, best_bits, final_bits,     \
+                                 e_best, e_final);                                              \
+  } while (0)
     if (g == 4)
       OS_COL_ITEM(4);
     else if (g == 8)
@@ -618,7 +684,7 @@ __global__ __launch_bounds__(64 * kW) void csr_sweep_col_kernel(
 // replicas and 1/G of the steps.
 //
 // Measured: 32 instances of 64 .. 1024 spins, degrees 3 .. 8, 128 replicas, 192
-// sweeps 67.3 -> 5.8 ms, the largest instance's chain of 1020 sites (340 ns
+// sweeps 67.3 -> 5.2 ms, the largest instance's chain of 1020 sites (340 ns
 // each) now ~70 steps.  The other kernels remain for batches with enough
 // replicas to fill the chip at 64 a wave, where each site's row is read once
 // for all of them, and for states too large for these LDS arrays: the tuner
@@ -632,31 +698,10 @@ __global__ __launch_bounds__(64 * kW) void csr_sweep_col_kernel(
 // two instructions).
 namespace {
 
+// Thresholds of a replica, one per site: floats from one replica's to the next's.
 __host__ __device__ inline int sched_tstride(int n) { return ((n + 16) & ~15) + 4; }
-__host__ __device__ inline int sched_bstride(int words) { return words * 32 + 16; }
 
-// Order of this wave's LDS accesses as written (the LDS serves a wave's accesses
-// in order; only the compiler has to keep it).
-__device__ __forceinline__ void lds_order() {
-  __builtin_amdgcn_wave_barrier();
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-}
-
-// Spins 32 wd .. 32 wd + 31 between bytes and a word.
-__device__ __forceinline__ void put_word(uint8_t *xb, int wd, uint32_t v) {
-  uint32_t *b = reinterpret_cast<uint32_t *>(xb + 32 * wd);
-#pragma unroll
-  for (int m = 0; m < 8; ++m) b[m] = (((v >> (4 * m)) & 15u) * 0x00204081u) & 0x01010101u;
-}
-__device__ __forceinline__ uint32_t get_word(const uint8_t *xb, int wd) {
-  const uint32_t *b = reinterpret_cast<const uint32_t *>(xb + 32 * wd);
-  uint32_t v = 0u;
-#pragma unroll
-  for (int m = 0; m < 8; ++m) v |= ((b[m] * 0x01020408u) >> 24) << (4 * m);
-  return v;
-}
-
-template <int G>
+template <int G, int NCH>
 __device__ __forceinline__ void sched_item(
     const CsrInst &d, int2 wi, char *lds, int lane, int S, int Rp, uint32_t k0, uint32_t k1,
     uint32_t base, int init_mode, int tb, int use_tsr, const float *__restrict__ tsr,
@@ -667,10 +712,11 @@ __device__ __forceinline__ void sched_item(
     double *__restrict__ e_best, double *__restrict__ e_final) {
   constexpr int RW = 64 / G;  // replicas per wave
   const int rr = lane / G, s = lane % G;
-  const int n = d.n, words = d.words, chunks = d.width >> 2, steps = d.steps;
+  const int n = d.n, words = d.words, chunks = NCH == 1 ? 1 : d.width >> 2,
+            steps = d.steps;
   float *td = reinterpret_cast<float *>(lds) + rr * sched_tstride(n);
   uint8_t *xb = reinterpret_cast<uint8_t *>(lds) + 4 * RW * sched_tstride(n) +
-                rr * sched_bstride(words);
+                rr * spin_stride(words);
   const uint32_t r = (uint32_t)(wi.y * RW + rr);
   const uint32_t id = (base + (uint32_t)wi.x) << 8;
   const int4 *ecol = ell_col + (d.ell_off >> 2);
@@ -729,9 +775,7 @@ __device__ __forceinline__ void sched_item(
     st.dj = *reinterpret_cast<const float *>(at(dg, (uint32_t)jr * 4u));
     st.c0 = *reinterpret_cast<const int4 *>(at(ecol, ro));
     st.v0 = *reinterpret_cast<const float4 *>(at(eval, ro));
-    st.c1 = make_int4(n, n, n, n);
-    st.v1 = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (chunks > 1) {
+    if constexpr (NCH > 1) {
       st.c1 = *reinterpret_cast<const int4 *>(at(ecol, ro + 16u));
       st.v1 = *reinterpret_cast<const float4 *>(at(eval, ro + 16u));
     }
@@ -742,25 +786,33 @@ __device__ __forceinline__ void sched_item(
     float h = c.dj;
     const float xj = (float)xb[c.j];
     // h + w for a set neighbour, h for a clear one: see add_if_set
-    h = fmaf((float)xb[c.c0.x], c.v0.x, h);
-    h = fmaf((float)xb[c.c0.y], c.v0.y, h);
-    h = fmaf((float)xb[c.c0.z], c.v0.z, h);
-    h = fmaf((float)xb[c.c0.w], c.v0.w, h);
-    if (chunks > 1) {
-      h = fmaf((float)xb[c.c1.x], c.v1.x, h);
-      h = fmaf((float)xb[c.c1.y], c.v1.y, h);
-      h = fmaf((float)xb[c.c1.z], c.v1.z, h);
-      h = fmaf((float)xb[c.c1.w], c.v1.w, h);
+    const float x0 = (float)xb[c.c0.x], x1 = (float)xb[c.c0.y], x2 = (float)xb[c.c0.z],
+                x3 = (float)xb[c.c0.w];
+    float x4, x5, x6, x7;
+    if constexpr (NCH > 1) {
+      x4 = (float)xb[c.c1.x];
+      x5 = (float)xb[c.c1.y];
+      x6 = (float)xb[c.c1.z];
+      x7 = (float)xb[c.c1.w];
     }
-    for (int cc = 2; cc < chunks; ++cc) {
-      const uint32_t ro =
-          ((uint32_t)min(c.j, n - 1) * (uint32_t)chunks + (uint32_t)cc) * 16u;
-      const int4 ci = *reinterpret_cast<const int4 *>(at(ecol, ro));
-      const float4 vi = *reinterpret_cast<const float4 *>(at(eval, ro));
-      h = fmaf((float)xb[ci.x], vi.x, h);
-      h = fmaf((float)xb[ci.y], vi.y, h);
-      h = fmaf((float)xb[ci.z], vi.z, h);
-      h = fmaf((float)xb[ci.w], vi.w, h);
+    h = fmaf(x0, c.v0.x, h);
+    h = fmaf(x1, c.v0.y, h);
+    h = fmaf(x2, c.v0.z, h);
+    h = fmaf(x3, c.v0.w, h);
+    if constexpr (NCH > 1) {
+      h = fmaf(x4, c.v1.x, h);
+      h = fmaf(x5, c.v1.y, h);
+      h = fmaf(x6, c.v1.z, h);
+      h = fmaf(x7, c.v1.w, h);
+      for (int cc = 2; cc < chunks; ++cc) {
+        const uint32_t ro = ((uint32_t)min(c.j, n - 1) * (uint32_t)chunks + (uint32_t)cc) * 16u;
+        const int4 ci = *reinterpret_cast<const int4 *>(at(ecol, ro));
+        const float4 vi = *reinterpret_cast<const float4 *>(at(eval, ro));
+        h = fmaf((float)xb[ci.x], vi.x, h);
+        h = fmaf((float)xb[ci.y], vi.y, h);
+        h = fmaf((float)xb[ci.z], vi.z, h);
+        h = fmaf((float)xb[ci.w], vi.w, h);
+      }
     }
     const float de = xj != 0.0f ? -h : h;
     const bool acc = de < thr && c.j < n;
@@ -840,9 +892,17 @@ __global__ __launch_bounds__(64) void csr_sweep_sched_kernel(
     const int2 wi = items[it];
     const CsrInst d = inst[wi.x];
     const int g = __builtin_amdgcn_readfirstlane(d.isites);
-#define OS_SCHED_ITEM(GG)                                                                      \
-  sched_item<GG>(d, wi, slds, lane, S, Rp, k0, k1, base, init_mode, tb, use_tsr, tsr, ell_col, \
-                 ell_val, diag, sched, tscale, init_bits, best_bits, final_bits, e_best, e_final)
+#define OS_SCHED_ITEM(GG)                                                                       \
+  do {                                                                                          \
+    if (d.width == 4)                                                                           \
+      sched_item<GG, 1>(d, wi, slds, lane, S, Rp, k0, k1, base, init_mode, tb, use_tsr, tsr,    \
+                        ell_col, ell_val, diag, sched, tscale, init_bits, best_bits,            \
+                        final_bits, e_best, e_final);                                           \
+    else                                                                                        \
+      sched_item<GG, 2>(d, wi, slds, lane, S, Rp, k0, k1, base, init_mode, tb, use_tsr, tsr,    \
+                        ell_col, ell_val, diag, sched, tscale, init_bits, best_bits,            \
+                        final_bits, e_best, e_final);                                           \
+  } while (0)
     if (g == 4)
       OS_SCHED_ITEM(4);
     else if (g == 8)
@@ -980,7 +1040,7 @@ void launch_csr_queue_reset(hipStream_t st, int *queue) {
 
 int csr_sched_lds_bytes(int n, int G) {
   const int words = (n + 1 + 31) / 32;
-  return 64 / G * (4 * sched_tstride(n) + sched_bstride(words));
+  return 64 / G * (4 * sched_tstride(n) + spin_stride(words));
 }
 
 int csr_sched_max_groups_per_cu(int lds) {
@@ -1085,54 +1145,44 @@ int csr_max_groups_per_cu(bool pf, int waves, int max_words) {
   return blocks;
 }
 
-int csr_col_lds_bytes(int waves, int plane_words) { return waves * (plane_words + 4 * 64) * 4; }
+int csr_col_spin_bytes(int words, int G, bool bytes) {
+  return 64 / G * (bytes ? spin_stride(words) : 4 * words);
+}
+int csr_col_lds_bytes(int waves, int spin_bytes) { return waves * (spin_bytes + kColThresholdBytes); }
 
 namespace {
 
-const void *col_kernel_for(int waves) {
-  switch (waves) {
-    case 1: return (const void *)csr_sweep_col_kernel<1>;
-    case 2: return (const void *)csr_sweep_col_kernel<2>;
-    case 4: return (const void *)csr_sweep_col_kernel<4>;
-    default: throw Error(-3, "csr colour sweep kernel: unsupported waves per group");
-  }
+const void *col_kernel_for(bool bytes) {
+  return bytes ? (const void *)csr_sweep_col_kernel<ByteSpins>
+               : (const void *)csr_sweep_col_kernel<BitSpins>;
 }
 
 }  // namespace
 
-int csr_col_max_groups_per_cu(int waves, int plane_words) {
-  const size_t lds = (size_t)csr_col_lds_bytes(waves, plane_words);
+int csr_col_max_groups_per_cu(int waves, int spin_bytes, bool bytes) {
+  const size_t lds = (size_t)csr_col_lds_bytes(waves, spin_bytes);
   int blocks = 0;
-  OS_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, col_kernel_for(waves),
+  OS_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, col_kernel_for(bytes),
                                                            64 * waves, lds));
   return blocks;
 }
 
-void launch_csr_col_sweeps(hipStream_t st, int waves, int groups, int plane_words,
+void launch_csr_col_sweeps(hipStream_t st, int waves, int groups, int spin_bytes, bool bytes,
                            const CsrInst *inst, const int2 *items, const CsrRun *run,
                            const int4 *ell_col, const float4 *ell_val, const float *diag,
-                           const int32_t *corder, const int32_t *cstart, const int4 *pell_col,
+                           const int32_t *corder, const int32_t *csteps, const int4 *pell_col,
                            const float4 *pell_val, const float *pdiag, const float *tscale,
                            const float *tsr, const uint32_t *init_bits, uint32_t *best_bits,
                            uint32_t *final_bits, double *e_best, double *e_final, int *queue) {
-  const size_t lds = (size_t)csr_col_lds_bytes(waves, plane_words);
-  const void *k = col_kernel_for(waves);
+  const size_t lds = (size_t)csr_col_lds_bytes(waves, spin_bytes);
+  const void *k = col_kernel_for(bytes);
   if (lds > 65536)
     OS_HIP_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-#define OS_COL_CASE(W)                                                                          \
-  case W:                                                                                       \
-    csr_sweep_col_kernel<W><<<groups, 64 * W, lds, st>>>(                                       \
-        inst, items, run, ell_col, ell_val, diag, corder, cstart, pell_col, pell_val, pdiag,    \
-        tscale, tsr, init_bits, best_bits, final_bits, e_best, e_final, queue, plane_words);   \
-    break;
-  switch (waves) {
-    OS_COL_CASE(1)
-    OS_COL_CASE(2)
-    OS_COL_CASE(4)
-    default:
-      throw Error(-3, "csr colour sweep kernel: unsupported waves per group");
-  }
-#undef OS_COL_CASE
+  auto run_kernel = bytes ? csr_sweep_col_kernel<ByteSpins> : csr_sweep_col_kernel<BitSpins>;
+  run_kernel<<<groups, 64 * waves, lds, st>>>(inst, items, run, ell_col, ell_val, diag, corder,
+                                              csteps, pell_col, pell_val, pdiag, tscale, tsr,
+                                              init_bits, best_bits, final_bits, e_best, e_final,
+                                              queue, spin_bytes);
   OS_HIP_CHECK(hipGetLastError());
 }
 

@@ -37,9 +37,15 @@ struct CsrBatch {
   int64_t total_spins = 0;
   std::vector<CsrInst> inst;
   DevBuf d_inst, ell_col, ell_val, diag, diag64, row_ptr, col, val64;
+  // steps of a sweep in the batch's array of them
+  struct Steps {
+    int32_t sites, steps;
+    int64_t off;
+  };
   // colour classes: sites class by class (offset spin_off), class starts
-  // (offset class_off)
-  DevBuf corder, cstart;
+  // (offset class_off), and the positions of each step
+  DevBuf corder, csteps;
+  std::vector<Steps> h_csteps[3];  // at 4, 8 and 16 sites per step
   std::vector<int32_t> h_order, h_cstart;
   // ELL rows and diagonal in that visiting order
   DevBuf pell_col, pell_val, pdiag;
@@ -63,11 +69,7 @@ struct CsrBatch {
   // scheduled kernel: every instance's schedules at 4, 8 and 16 sites per step,
   // the policy in use (s_sites; 0: none tried) and its work items ((instance,
   // group of 64/isites replicas)), built for (items_s_sites, items_s_Rp)
-  struct Sched {
-    int32_t isites, steps;
-    int64_t off;
-  };
-  std::vector<Sched> h_sched[3];
+  std::vector<Steps> h_sched[3];
   DevBuf sched, items_s;
   int num_items_s = 0, s_sites = 0, items_s_sites = 0, items_s_Rp = 0;
   int s_lds = 0;  // LDS of a wave: the largest of the batch
@@ -80,7 +82,8 @@ struct CsrBatch {
   int c_waves = 0, c_groups = 0, c_uniform = 0, c_limit = 0;
   DevBuf items_c;
   int num_items_c = 0, items_uniform = -1, items_limit = -1, items_c_Rp = 0;
-  int c_plane_words = 0;  // LDS state words per wave: max of words_i * 64/sites_i
+  bool c_bytes = false;  // spins a byte each in LDS, else bit-packed
+  int c_spin_bytes = 0;  // LDS bytes of the spins per wave: the largest of the batch
   std::vector<int> order_by_work;  // instances, largest first
   // the run that enqueue() launches: 0 sequential, 1 colour classes
   int mode = 0;
@@ -102,7 +105,7 @@ struct CsrBatch {
     drop_graph();
     for (auto *b : {&d_inst, &ell_col, &ell_val, &diag, &diag64, &row_ptr, &col, &val64, &items,
                     &run, &tscale, &init, &best, &fin, &eb, &ef, &e64, &queue, &marg, &corder,
-                    &cstart, &items_c, &pell_col, &pell_val, &pdiag, &pop_best, &pop_eb,
+                    &csteps, &items_c, &pell_col, &pell_val, &pdiag, &pop_best, &pop_eb,
                     &pop_anc, &tsr, &pt_slots, &sched, &items_s})
       b->release();
   }
@@ -113,9 +116,9 @@ struct CsrBatch {
     hipStream_t st = ctx->stream;
     launch_csr_queue_reset(st, queue.as<int>());
     if (mode == 1)
-      launch_csr_col_sweeps(st, w, g, c_plane_words, d_inst.as<CsrInst>(), items_c.as<int2>(),
+      launch_csr_col_sweeps(st, w, g, c_spin_bytes, c_bytes, d_inst.as<CsrInst>(), items_c.as<int2>(),
                             run.as<CsrRun>(), ell_col.as<int4>(), ell_val.as<float4>(),
-                            diag.as<float>(), corder.as<int32_t>(), cstart.as<int32_t>(),
+                            diag.as<float>(), corder.as<int32_t>(), csteps.as<int32_t>(),
                             pell_col.as<int4>(), pell_val.as<float4>(), pdiag.as<float>(),
                             tscale.as<float>(), tsr.as<float>(), init.as<uint32_t>(),
                             best.as<uint32_t>(),
@@ -218,6 +221,11 @@ int sites_for(int n, int uniform, int limit) {
   return 16;
 }
 
+// Colour kernel: LDS of a wave up to which its spins take a byte each.  A mixed
+// batch of up to 2048 spins runs 42.3 ms bit-packed, 36.6 with bytes under this
+// limit and the same under 40 and 80 KB; n = 40000 only fits as bits.
+constexpr int kByteSpinLimit = 16 * 1024;
+
 // Sets every instance's sites per step for the policy (uniform, limit) and
 // builds the colour kernel's work items: (instance, group of 64/sites_i
 // replicas), the items of longer estimated runtime first (steps per sweep
@@ -227,12 +235,16 @@ void col_items(CsrBatch &b, int uniform, int limit) {
   std::vector<int> order(b.I);
   std::iota(order.begin(), order.end(), 0);
   std::vector<int64_t> est(b.I);
-  int plane = 0;
+  int spins[2] = {0, 0};
   for (int i = 0; i < b.I; ++i) {
     CsrInst &d = b.inst[i];
     d.sites = sites_for(d.n, uniform, limit);
-    est[i] = ((int64_t)(d.n + d.sites - 1) / d.sites + d.ncol) * (d.width + 8);
-    plane = std::max(plane, d.words * (64 / d.sites));
+    const CsrBatch::Steps &cs = b.h_csteps[d.sites == 4 ? 0 : d.sites == 8 ? 1 : 2][i];
+    d.csteps = cs.steps;
+    d.csteps_off = cs.off;
+    est[i] = (int64_t)d.csteps * (d.width + 8);
+    for (bool bytes : {false, true})
+      spins[bytes] = std::max(spins[bytes], csr_col_spin_bytes(d.words, d.sites, bytes));
   }
   std::stable_sort(order.begin(), order.end(), [&](int a, int c) { return est[a] > est[c]; });
   // whole instances to the 8 XCD lists, largest total work first onto the
@@ -270,7 +282,8 @@ void col_items(CsrBatch &b, int uniform, int limit) {
                               s));
   OS_HIP_CHECK(hipStreamSynchronize(s));
   b.num_items_c = (int)items.size();
-  b.c_plane_words = plane;
+  b.c_bytes = spins[1] <= kByteSpinLimit;
+  b.c_spin_bytes = spins[b.c_bytes];
   b.items_uniform = uniform;
   b.items_limit = limit;
   b.items_c_Rp = b.Rp;
@@ -281,7 +294,7 @@ void col_items(CsrBatch &b, int uniform, int limit) {
 // lower-index site that it reads or that reads it.  A schedule that fills less
 // than half of its slots is left out and the next smaller G stands in for it.
 void build_schedules(const CsrInst &d, const int32_t *rp, const int32_t *cl,
-                     std::vector<int32_t> &out, CsrBatch::Sched (&made)[3]) {
+                     std::vector<int32_t> &out, CsrBatch::Steps (&made)[3]) {
   const int n = d.n;
   std::vector<int32_t> earliest(n), fill, next, step(n);
   for (int k = 0; k < 3; ++k) {
@@ -316,6 +329,29 @@ void build_schedules(const CsrInst &d, const int32_t *rp, const int32_t *cl,
   }
 }
 
+// Steps of the colour-class order at G = 4, 8 and 16 sites per step: the
+// positions of each class by G; an idle slot repeats its step's first position
+// with bit 31 set.
+void class_steps(const std::vector<int32_t> &start, std::vector<int32_t> &out,
+                 CsrBatch::Steps (&made)[3]) {
+  constexpr int32_t kIdle = INT32_MIN;
+  for (int k = 0; k < 3; ++k) {
+    const int G = 4 << k;
+    const size_t at = out.size();
+    for (size_t c = 0; c + 1 < start.size(); ++c)
+      for (int p0 = start[c]; p0 < start[c + 1]; p0 += G)
+        for (int s = 0; s < G; ++s)
+          out.push_back(p0 + s < start[c + 1] ? p0 + s : p0 | kIdle);
+    int steps = (int)((out.size() - at) / G);
+    // an even number, and two more for the requests made ahead: the last
+    // position again, idle
+    const int32_t last = start.back() - 1;
+    const int extra = (steps & 1) + 2;
+    out.insert(out.end(), (size_t)extra * G, last | kIdle);
+    made[k] = {G, steps + (steps & 1), (int64_t)at};
+  }
+}
+
 // Sets every instance's schedule for `sites` (4, 8 or 16) sites per step and
 // builds the scheduled kernel's work items, longest first.
 void sched_items(CsrBatch &b, int sites) {
@@ -326,7 +362,7 @@ void sched_items(CsrBatch &b, int sites) {
   int lds = 0;
   for (int i = 0; i < b.I; ++i) {
     CsrInst &d = b.inst[i];
-    d.isites = b.h_sched[k][i].isites;
+    d.isites = b.h_sched[k][i].sites;
     d.steps = b.h_sched[k][i].steps;
     d.sched_off = b.h_sched[k][i].off;
     lds = std::max(lds, csr_sched_lds_bytes(d.n, d.isites));
@@ -354,7 +390,7 @@ void sched_items(CsrBatch &b, int sites) {
 int sched_groups(CsrBatch &b, int sites) {
   const int k = sites == 4 ? 0 : sites == 8 ? 1 : 2;
   for (int i = 0; i < b.I; ++i)
-    if (csr_sched_lds_bytes(b.inst[i].n, b.h_sched[k][i].isites) > 160 * 1024) return 0;
+    if (csr_sched_lds_bytes(b.inst[i].n, b.h_sched[k][i].sites) > 160 * 1024) return 0;
   sched_items(b, sites);
   return std::min(b.ctx->num_cus * csr_sched_max_groups_per_cu(b.s_lds), b.num_items_s);
 }
@@ -394,7 +430,7 @@ void tune_col(CsrBatch &b, const CsrRun &full) {
     col_items(b, 0, limit);
     put_run(b, probe, CsrBatch::kPlain);
     for (int w : {1, 2, 4}) {
-      const int maxb = csr_col_max_groups_per_cu(w, b.c_plane_words);
+      const int maxb = csr_col_max_groups_per_cu(w, b.c_spin_bytes, b.c_bytes);
       if (maxb < 1) continue;
       std::vector<int> gpcs{maxb};
       if (maxb > 1) gpcs.push_back(std::max(1, maxb / 2));
@@ -496,7 +532,7 @@ Shape select_shape(CsrBatch &b, const CsrRun &run, int site_order, bool tune_it)
       b.c_waves = 1;
       col_items(b, b.c_uniform, b.c_limit);
       b.c_groups = std::max(
-          1, std::min(c.num_cus * csr_col_max_groups_per_cu(1, b.c_plane_words), b.num_items_c));
+          1, std::min(c.num_cus * csr_col_max_groups_per_cu(1, b.c_spin_bytes, b.c_bytes), b.num_items_c));
     }
   }
   if (b.mode == 1 && b.c_waves == 0) {
@@ -514,7 +550,7 @@ Shape select_shape(CsrBatch &b, const CsrRun &run, int site_order, bool tune_it)
       b.c_waves = 2;
       col_items(b, b.c_uniform, b.c_limit);
       b.c_groups = std::max(
-          1, std::min(c.num_cus * csr_col_max_groups_per_cu(2, b.c_plane_words), b.num_items_c));
+          1, std::min(c.num_cus * csr_col_max_groups_per_cu(2, b.c_spin_bytes, b.c_bytes), b.num_items_c));
     }
   }
   if (b.mode == 1) col_items(b, b.c_uniform, b.c_limit);
@@ -721,7 +757,8 @@ int os_csr_batch_create(os_ctx *ctx_, int32_t num_instances, const int32_t *n,
     const int nd = (int)ds.size();
     std::vector<int32_t> ell_c((size_t)ell);
     std::vector<float> ell_v((size_t)ell, 0.0f), dg((size_t)spins);
-    std::vector<std::vector<int32_t>> cst(nd), cord(nd), sch(nd);
+    std::vector<std::vector<int32_t>> cst(nd), cord(nd), sch(nd), cls(nd);
+    for (auto &h : b->h_csteps) h.resize(nd);
     for (auto &h : b->h_sched) h.resize(nd);
     std::vector<const char *> err(nd, nullptr);
     os::host_parallel_for(nd, [&](int i) {
@@ -768,15 +805,17 @@ int os_csr_batch_create(os_ctx *ctx_, int32_t num_instances, const int32_t *n,
       std::vector<int32_t> fill(start.begin(), start.end() - 1);
       cord[i].resize(ni);
       for (int j = 0; j < ni; ++j) cord[i][fill[colour[j]]++] = j;
-      CsrBatch::Sched made[3];
+      CsrBatch::Steps made[3];
       os::build_schedules(d, rp, cl, sch[i], made);
       for (int k = 0; k < 3; ++k) b->h_sched[k][i] = made[k];
+      os::class_steps(start, cls[i], made);
+      for (int k = 0; k < 3; ++k) b->h_csteps[k][i] = made[k];
     });
     // the first failing instance in order, as a serial pass reports it
     for (int i = 0; i < nd; ++i) OS_REQUIRE(!err[i], err[i]);
     OS_REQUIRE(!bad_msg, bad_msg);
     // Pass 3 (serial): class and schedule offsets and the concatenated arrays
-    std::vector<int32_t> h_sched;
+    std::vector<int32_t> h_sched, h_csteps;
     for (int i = 0; i < nd; ++i) {
       os::CsrInst &d = ds[i];
       d.class_off = (int64_t)b->h_cstart.size();
@@ -784,6 +823,8 @@ int os_csr_batch_create(os_ctx *ctx_, int32_t num_instances, const int32_t *n,
       b->h_order.insert(b->h_order.end(), cord[i].begin(), cord[i].end());
       for (auto &h : b->h_sched) h[i].off += (int64_t)h_sched.size();
       h_sched.insert(h_sched.end(), sch[i].begin(), sch[i].end());
+      for (auto &h : b->h_csteps) h[i].off += (int64_t)h_csteps.size();
+      h_csteps.insert(h_csteps.end(), cls[i].begin(), cls[i].end());
       b->max_words = std::max(b->max_words, d.words);
       b->max_width = std::max(b->max_width, d.width);
       b->total_words += d.words;
@@ -846,11 +887,11 @@ int os_csr_batch_create(os_ctx *ctx_, int32_t num_instances, const int32_t *n,
     OS_HIP_CHECK(hipMemcpyAsync(b->sched.ptr, h_sched.data(), sizeof(int32_t) * h_sched.size(),
                                 hipMemcpyHostToDevice, s));
     b->corder.ensure(sizeof(int32_t) * b->h_order.size());
-    b->cstart.ensure(sizeof(int32_t) * b->h_cstart.size());
     OS_HIP_CHECK(hipMemcpyAsync(b->corder.ptr, b->h_order.data(),
                                 sizeof(int32_t) * b->h_order.size(), hipMemcpyHostToDevice, s));
-    OS_HIP_CHECK(hipMemcpyAsync(b->cstart.ptr, b->h_cstart.data(),
-                                sizeof(int32_t) * b->h_cstart.size(), hipMemcpyHostToDevice, s));
+    b->csteps.ensure(sizeof(int32_t) * h_csteps.size());
+    OS_HIP_CHECK(hipMemcpyAsync(b->csteps.ptr, h_csteps.data(), sizeof(int32_t) * h_csteps.size(),
+                                hipMemcpyHostToDevice, s));
     OS_HIP_CHECK(hipStreamSynchronize(s));
     *out = reinterpret_cast<os_csr_batch *>(b.release());
   });

@@ -122,8 +122,9 @@ struct CsrInst {
   int32_t sites;      // colour-class kernel: sites per wave step (4, 8 or 16)
   int32_t isites;     // scheduled index-order kernel: sites per wave step (4, 8 or 16)
   int64_t sched_off;  // its schedule: isites slots a step, slot n idle
-  int32_t steps;      // steps in it (even; two idle steps follow)
-  int32_t pad_;
+  int64_t csteps_off; // colour-class steps: `sites` positions a step, bit 31: idle
+  int32_t steps;      // steps of the schedule (even; two idle steps follow)
+  int32_t csteps;     // colour-class steps (likewise)
 };
 // The device arrays of a sparse batch, for kernels outside the annealer (the
 // warm-start network): instance descriptors, CSR (both directions, no
@@ -175,16 +176,17 @@ void launch_csr_sweeps(hipStream_t st, bool pf, int waves, int groups, int max_w
 // colour-class sweeps: instance i updates G_i = CsrInst::sites (4, 8 or 16)
 // sites of 64/G_i replicas per wave step; items are (instance, group of
 // 64/G_i replicas); corder lists the sites of each instance class by class
-// (offset spin_off), cstart the class starts (offset class_off); pell_col /
-// pell_val / pdiag hold the ELL rows and the diagonal in that visiting order
-// (offsets ell_off, spin_off).  plane_words: LDS words per wave for the
-// state planes, the batch's largest words_i * 64/G_i.
-int csr_col_lds_bytes(int waves, int plane_words);
-int csr_col_max_groups_per_cu(int waves, int plane_words);
-void launch_csr_col_sweeps(hipStream_t st, int waves, int groups, int plane_words,
+// (offset spin_off), csteps the positions of each step (offset csteps_off);
+// pell_col / pell_val / pdiag hold the ELL rows and the diagonal in that
+// visiting order (offsets ell_off, spin_off).  spin_bytes: LDS bytes per wave
+// for the spins (csr_col_spin_bytes, the batch's largest).
+int csr_col_spin_bytes(int words, int G, bool bytes);
+int csr_col_lds_bytes(int waves, int spin_bytes);
+int csr_col_max_groups_per_cu(int waves, int spin_bytes, bool bytes);
+void launch_csr_col_sweeps(hipStream_t st, int waves, int groups, int spin_bytes, bool bytes,
                            const CsrInst *inst, const int2 *items, const CsrRun *run,
                            const int4 *ell_col, const float4 *ell_val, const float *diag,
-                           const int32_t *corder, const int32_t *cstart, const int4 *pell_col,
+                           const int32_t *corder, const int32_t *csteps, const int4 *pell_col,
                            const float4 *pell_val, const float *pdiag, const float *tscale,
                            const float *tsr, const uint32_t *init_bits, uint32_t *best_bits,
                            uint32_t *final_bits, double *e_best, double *e_final, int *queue);
