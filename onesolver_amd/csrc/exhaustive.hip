@@ -11,17 +11,14 @@
 // n <= 20: one thread per state computes that literal energy; a minimum over
 // (energy, index) pairs follows.
 //
-// 20 < n <= 40: thread t owns the states whose top n-L bits equal t.  It walks
-// them in Gray-code order in segments of 2^S states, starting each segment
-// from its literal energy.  The low kLow bits flip in an unrolled order with
-// their local fields h_j = q_jj + sum_{i != j} q_ij x_i in registers, so a
-// state costs kLow FMAs; a higher bit B flips once per 2^kLow states, with
-// its field summed from the LDS copy of q.
-//   pass 1: every thread's minimum of its walk energies, and their minimum
-//           E_w;
+// 20 < n <= 40: thread t owns the states whose top n-L bits equal t and walks
+// them in Gray-code order in segments of 2^S states, each from its literal
+// energy.
+//   pass 1: every thread's minimum energy, and the minimum E_w of them (below);
 //   pass 2: only the threads whose minimum is within tol = 1e-9 (|E_w| + 1)
-//           of E_w walk again; every state whose walk energy is within tol of
-//           E_w gets its literal energy, and the (literal energy, index)
+//           of E_w walk again, their states split over 2^K threads each where
+//           few blocks hold them; every state whose walk energy is within tol
+//           of E_w gets its literal energy, and the (literal energy, index)
 //           minimum of those is the answer.
 // A walk energy differs from the literal one by the rounding of at most 2^S
 // steps, far below tol, so the literal minimum is always among the
@@ -40,8 +37,10 @@ namespace {
 
 constexpr int kMaxN = 40;
 constexpr int kLiteralMaxN = 20;
-constexpr int kLow = 5;      // bits flipped in the unrolled order
+constexpr int kLow = 5;       // pass 2: bits flipped in the unrolled order
+constexpr int kMinLow = 7;    // pass 1: bits of an unrolled block
 constexpr int kSegBits = 12;  // literal restart every 2^kSegBits states
+constexpr int kMaxActive = 16;  // blocks with candidates that pass 2 splits
 constexpr int kMaxTopBits = 20;
 constexpr int kThreads = 256;
 
@@ -124,29 +123,135 @@ __global__ __launch_bounds__(kThreads) void exh_literal_kernel(int n, const doub
   block_min(e, bx, out_e, out_x);
 }
 
-// Gray-code walks, 20 < n <= 40; L = n - P bits per thread, 2^P threads.
-// PASS 1 writes every thread's minimum walk energy to tmin and per-block
-// minima of them (out_x unused); PASS 2 walks the threads with tmin <= thr
-// and writes per-block (literal energy, index) minima of the candidates
-// e_walk <= thr.
-template <int PASS>
-__global__ __launch_bounds__(kThreads) void exh_gray_kernel(int n, int L, const double *__restrict__ q,
-                                                            double thr, double *__restrict__ tmin,
-                                                            double *__restrict__ out_e,
-                                                            uint64_t *__restrict__ out_x) {
+// Pass 1, 20 < n <= 40; L = n - P bits per thread, 2^P threads: writes every
+// thread's minimum energy to tmin and per-block minima of them.
+//
+// FP64 issue bounds it, so a state costs few instructions.  The fields
+// h_j = q_jj + sum_{i != j} q_ij x_i of the low kSegBits bits are kept in
+// registers.  Bits 0, 1 and 2 are not walked: with them clear and energy e,
+//   min over x0, x1, x2 = e + min(g(h0, h1), h2 + g(h0 + q02, h1 + q12)),
+//   g(a, b) = min(min(0, a), b + min(0, a + q01)),
+// 16 instructions for 8 states.  Bits 3 .. 6 go once round the Gray cycle in an
+// unrolled block whose signs are constants and whose couplings are scalars; a
+// higher bit flips once per 128 states.  About 3 instructions a state instead
+// of 11 (5 FMAs and a minimum, and a field summed from LDS every 32 states).
+// Measured: n = 32 2174 -> 579 us; whole calls n = 31 1459 -> 489 us, n = 25
+// 281 -> 153, n = 21 127 -> 117.
+template <int B>
+__device__ __forceinline__ void flip_high(const double *qs, bool set, double &e,
+                                          double (&h)[kSegBits]) {
+  const double sb = set ? -1.0 : 1.0;
+  int row = B * kMaxN;
+  asm volatile("" : "+v"(row));  // or every row is kept in registers
+  e = fma(sb, h[B], e);
+#pragma unroll
+  for (int j = 0; j < kSegBits; ++j)
+    if (j != B) h[j] = fma(sb, qs[row + j], h[j]);
+}
+
+__global__ __launch_bounds__(kThreads) void exh_min_kernel(int n, int L, const double *__restrict__ q,
+                                                           double *__restrict__ tmin,
+                                                           double *__restrict__ out_e,
+                                                           uint64_t *__restrict__ out_x) {
   __shared__ double qs[kMaxN * kMaxN];
   const int S = min(L, kSegBits);
   const uint64_t t = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
-  bool active = t < (1ull << (n - L));
-  if (PASS == 2) {
-    if (active) active = tmin[t] <= thr;
-    if (!__syncthreads_or(active)) {  // no candidate in this block
-      if (threadIdx.x == 0) {
-        out_e[blockIdx.x] = DBL_MAX;
-        out_x[blockIdx.x] = 0;
-      }
-      return;
+  load_q(n, q, qs);
+  __syncthreads();
+  auto uniform = [](double v) {
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(v)));
+  };
+  double ql[kMinLow][kMinLow];  // q_ij, i < j
+#pragma unroll
+  for (int i = 0; i < kMinLow; ++i)
+#pragma unroll
+    for (int j = i + 1; j < kMinLow; ++j) ql[i][j] = uniform(qs[i * kMaxN + j]);
+  double emin = DBL_MAX;
+  const bool active = t < (1ull << (n - L));
+  const int segs = active ? 1 << (L - S) : 0;
+  const int blocks = 1 << (S - kMinLow);
+  for (int seg = 0; seg < segs; ++seg) {
+    const uint64_t x0 = (t << L) | ((uint64_t)seg << S);  // low S bits zero
+    double e = literal_energy(n, qs, x0);
+    double h[kSegBits];
+#pragma unroll
+    for (int j = 0; j < kSegBits; ++j) h[j] = qs[j * kMaxN + j];
+    for (int i = S; i < n; ++i) {  // (fields of bits from S on are not used)
+      const double xi = (x0 >> i) & 1u ? 1.0 : 0.0;
+#pragma unroll
+      for (int j = 0; j < kSegBits; ++j) h[j] = fma(xi, qs[i * kMaxN + j], h[j]);
     }
+    for (int blk = 0;;) {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        const double a = fmin(fmin(0.0, h[0]), h[1] + fmin(0.0, h[0] + ql[0][1]));
+        const double h0 = h[0] + ql[0][2], h1 = h[1] + ql[1][2];
+        const double b = fmin(fmin(0.0, h0), h1 + fmin(0.0, h0 + ql[0][1]));
+        emin = fmin(emin, e + fmin(a, h[2] + b));
+        // the next bit of the cycle: state k ^ (k >> 1) of bits 3 .. 6 so far
+        const int f = k < 15 ? 3 + __builtin_ctz(k + 1) : 6;
+        const bool set = ((k ^ (k >> 1)) >> (f - 3)) & 1;
+        e = set ? e - h[f] : e + h[f];
+#pragma unroll
+        for (int j = 0; j < kMinLow; ++j)
+          if (j != f) {
+            const double c = j < f ? ql[j][f] : ql[f][j];
+            h[j] = set ? h[j] - c : h[j] + c;
+          }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // the fields of the bits above followed none of it: the cycle ends where
+      // it began
+      if (++blk == blocks) break;
+      const int B = kMinLow + __builtin_ctz((unsigned)blk);
+      // bit B of the Gray code of blk - 1
+      const bool set = (((blk - 1) ^ ((blk - 1) >> 1)) >> (B - kMinLow)) & 1;
+      switch (B) {
+        case 7: flip_high<7>(qs, set, e, h); break;
+        case 8: flip_high<8>(qs, set, e, h); break;
+        case 9: flip_high<9>(qs, set, e, h); break;
+        case 10: flip_high<10>(qs, set, e, h); break;
+        default: flip_high<11>(qs, set, e, h); break;
+      }
+    }
+  }
+  static_assert(kSegBits == 12 && kMinLow == 7, "the flips above");
+  if (active) tmin[t] = emin;
+  block_min(emin, 0, out_e, out_x);
+}
+
+// Blocks of pass 1 that hold a candidate.
+struct ActiveBlocks {
+  int count;
+  int id[kMaxActive];
+};
+
+// Pass 2: walks the states of the threads of pass 1 with tmin <= thr and writes
+// per-block (literal energy, index) minima of the candidates e_walk <= thr.  A
+// thread takes 2^(L-K) of a pass-1 thread's 2^L states; blocks are those of
+// `act`, 2^K each, or all of them (K = 0, act.count 0).
+__global__ __launch_bounds__(kThreads) void exh_gray_kernel(int n, int L, int K, ActiveBlocks act,
+                                                            const double *__restrict__ q,
+                                                            double thr,
+                                                            const double *__restrict__ tmin,
+                                                            double *__restrict__ out_e,
+                                                            uint64_t *__restrict__ out_x) {
+  __shared__ double qs[kMaxN * kMaxN];
+  const uint64_t block =
+      act.count ? ((uint64_t)act.id[blockIdx.x >> K] << K) + (blockIdx.x & ((1u << K) - 1u))
+                : blockIdx.x;
+  const uint64_t t = block * kThreads + threadIdx.x;
+  L -= K;
+  const int S = min(L, kSegBits);
+  bool active = t < (1ull << (n - L));
+  if (active) active = tmin[t >> K] <= thr;
+  if (!__syncthreads_or(active)) {  // no candidate in this block
+    if (threadIdx.x == 0) {
+      out_e[blockIdx.x] = DBL_MAX;
+      out_x[blockIdx.x] = 0;
+    }
+    return;
   }
   load_q(n, q, qs);
   __syncthreads();
@@ -159,7 +264,6 @@ __global__ __launch_bounds__(kThreads) void exh_gray_kernel(int n, int L, const 
     for (int j = i + 1; j < kLow; ++j) ql[i][j] = qs[i * kMaxN + j];
   double emin = DBL_MAX;
   uint64_t xmin = 0;
-  double eg[8];  // PASS 1: the energies of 8 consecutive states
   const int segs = active ? 1 << (L - S) : 0;
   const int blocks = 1 << (S - kLow);
   for (int seg = 0; seg < segs; ++seg) {
@@ -185,18 +289,7 @@ __global__ __launch_bounds__(kThreads) void exh_gray_kernel(int n, int L, const 
             if (j != b) h[j] = fma(s[b], j < b ? ql[j][b] : ql[b][j], h[j]);
           s[b] = -s[b];
         }
-        if (PASS == 1) {
-          // minimum of each 8 states as a tree, then into emin; the barrier
-          // keeps the compiler from holding a whole block of energies
-          // (register pressure, occupancy)
-          eg[pos & 7] = e;
-          if ((pos & 7) == 7) {
-            const double m = fmin(fmin(fmin(eg[0], eg[1]), fmin(eg[2], eg[3])),
-                                  fmin(fmin(eg[4], eg[5]), fmin(eg[6], eg[7])));
-            emin = fmin(emin, m);
-            __builtin_amdgcn_sched_barrier(0);
-          }
-        } else if (e <= thr) {
+        if (e <= thr) {
           const uint64_t x = xhi | (low0 ^ (uint32_t)(pos ^ (pos >> 1)));
           const double v = literal_energy(n, qs, x);
           if (better(v, x, emin, xmin)) {
@@ -217,7 +310,6 @@ __global__ __launch_bounds__(kThreads) void exh_gray_kernel(int n, int L, const 
       }
     }
   }
-  if (PASS == 1 && t < (1ull << (n - L))) tmin[t] = emin;
   block_min(emin, xmin, out_e, out_x);
 }
 
@@ -225,14 +317,14 @@ int exhaustive_max_n() { return kMaxN; }
 
 // Threads and per-thread bits of the Gray walk for n (20 < n <= 40).
 static void gray_shape(int n, int *P, int *L) {
-  *P = std::min(n - kLow, kMaxTopBits);
+  *P = std::min(n - kMinLow, kMaxTopBits);
   *L = n - *P;
 }
 
 void exhaustive_solve(hipStream_t st, int n, const double *q_dev, bool finite, double *tmin,
                       double *part_e, uint64_t *part_x, size_t part_cap, double *best_e,
                       uint64_t *best_x) {
-  auto reduce = [&](int nb) {
+  auto reduce = [&](int nb, std::vector<double> *minima) {
     std::vector<double> e(nb);
     std::vector<uint64_t> x(nb);
     OS_HIP_CHECK(hipMemcpyAsync(e.data(), part_e, sizeof(double) * nb, hipMemcpyDeviceToHost, st));
@@ -247,13 +339,14 @@ void exhaustive_solve(hipStream_t st, int n, const double *q_dev, bool finite, d
       }
     *best_e = be;
     *best_x = bx;
+    if (minima) minima->swap(e);
   };
   if (n <= kLiteralMaxN || (!finite && n <= 30)) {
     const int nb = (int)(((1ull << n) + kThreads - 1) / kThreads);
     OS_REQUIRE((size_t)nb <= part_cap, "partials buffer too small");
     exh_literal_kernel<<<nb, kThreads, 0, st>>>(n, q_dev, part_e, part_x);
     OS_HIP_CHECK(hipGetLastError());
-    reduce(nb);
+    reduce(nb, nullptr);
     return;
   }
   if (!finite)
@@ -263,14 +356,25 @@ void exhaustive_solve(hipStream_t st, int n, const double *q_dev, bool finite, d
   gray_shape(n, &P, &L);
   const int nb = (int)(((1ull << P) + kThreads - 1) / kThreads);
   OS_REQUIRE((size_t)nb <= part_cap, "partials buffer too small");
-  exh_gray_kernel<1><<<nb, kThreads, 0, st>>>(n, L, q_dev, 0.0, tmin, part_e, part_x);
+  exh_min_kernel<<<nb, kThreads, 0, st>>>(n, L, q_dev, tmin, part_e, part_x);
   OS_HIP_CHECK(hipGetLastError());
-  reduce(nb);
+  std::vector<double> minima;
+  reduce(nb, &minima);
   const double ew = *best_e;
   const double thr = ew + 1e-9 * (std::fabs(ew) + 1.0);
-  exh_gray_kernel<2><<<nb, kThreads, 0, st>>>(n, L, q_dev, thr, tmin, part_e, part_x);
+  // One thread's walk is a serial chain, so its states go to 2^K threads where
+  // few blocks hold candidates (most instances: one; n = 32 441 -> 53 us).
+  // Instances with many take the undivided walk, which fills the chip by itself.
+  ActiveBlocks act{0, {}};
+  int found = 0;
+  for (int i = 0; i < nb; ++i)
+    if (minima[i] <= thr && found++ < kMaxActive) act.id[act.count++] = i;
+  int K = std::min(8, L - kLow);
+  if (found < 1 || found > kMaxActive || ((size_t)found << K) > part_cap) K = act.count = 0;
+  const int nb2 = act.count ? found << K : nb;
+  exh_gray_kernel<<<nb2, kThreads, 0, st>>>(n, L, K, act, q_dev, thr, tmin, part_e, part_x);
   OS_HIP_CHECK(hipGetLastError());
-  reduce(nb);
+  reduce(nb2, nullptr);
 }
 
 size_t exhaustive_thread_slots(int n) {

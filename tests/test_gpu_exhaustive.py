@@ -93,6 +93,29 @@ def test_exhaustive_ties_go_to_the_lowest_index(ctx, n, a, b):
     assert (st == want).all()
 
 
+@pytest.mark.parametrize("n", [21, 22, 27, 28, 32, 33])
+def test_exhaustive_finds_planted_minimum(ctx, n):
+    """E = sum a_i y_i + sum b_ij y_i y_j with y = x XOR s and positive whole
+    a, b has its one minimum at x = s (all sums exact): s at the edges of the
+    walks' blocks (3, 7 and 12 low bits), with one segment a thread or two."""
+    rng = np.random.default_rng(n)
+    low = [0, 7, 8, 0x7F, 0x80, 0xFFF, 0xA55]
+    for k, bits in enumerate(low):
+        s = bits | (int(rng.integers(0, 1 << 20)) << 12)
+        s = np.array([(s >> i) & 1 for i in range(n)])
+        a = rng.integers(1, 1 << 20, n).astype(np.float64)
+        b = np.triu(rng.integers(1, 1 << 10, (n, n)), 1).astype(np.float64)
+        # y = s + (1 - 2 s) x
+        f = 1.0 - 2.0 * s
+        q = b * np.outer(f, f)
+        bs = b + b.T
+        q[np.diag_indices(n)] = f * (a + bs @ s)
+        const = a @ s + s @ b @ s
+        print(f"[gpu] exhaustive planted n={n} low bits {bits:#x}", flush=True)
+        x, e = ctx.exhaustive(q)
+        assert np.array_equal(x, s) and e == -const, (n, k)
+
+
 def test_exhaustive_all_zero_instance(ctx):
     for n in (5, 22):
         st, e = ctx.exhaustive(np.zeros((n, n)))
