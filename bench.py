@@ -371,7 +371,8 @@ def run_csr_c3(args):
                      "frac": achieved / PEAK_HBM_GBS,
                      "traffic": (TRAFFIC_CSR_C3_COLOUR if order else TRAFFIC_CSR_C3)
                      if S == 2048 else None,
-                     "kernel": "csr_sweep_col_kernel" if order else "csr_sweep_pf_kernel",
+                     "kernel": "csr_sweep_col_kernel" if order else
+                               "csr_sweep_sched_kernel" if shape()[2] == 2 else "csr_sweep_pf_kernel",
                      "avg_launch_ms": avg_launch_s * 1e3,
                      "algorithmic_bytes_per_launch": bytes_alg},
     }
@@ -805,11 +806,11 @@ def run_exhaustive(args):
     elapsed = time.perf_counter() - t0
     ctx.close()
     states = float(2 ** n) * args.steps
-    # per state: one FP64 add for the energy and kLow - 1 = 4 for the low
-    # fields of the Gray-code walk (the second pass re-walks only the threads
-    # whose minimum is within the re-ranking tolerance)
-    flops = 5.0 * states
-    achieved = flops / elapsed / 1e12
+    # FP64 adds and minima of pass 1 (the second pass re-walks only the threads
+    # whose minimum is within the re-ranking tolerance): per 128 states 16 times
+    # 16 for the minimum over three bits and 7 for a flip
+    flops = 16 * 23 / 128 * 2.0 ** n  # of one search
+    achieved = flops * args.steps / elapsed / 1e12
     res = {
         "metric": "exhaustive states/s", "value": states / elapsed, "unit": "states/s",
         "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
@@ -819,9 +820,9 @@ def run_exhaustive(args):
                                f"on ties", "n": n},
         "roofline": {"bound": "fp64", "achieved": achieved, "peak": PEAK_FP64_TFLOPS,
                      "unit": "TFLOP/s", "frac": achieved / PEAK_FP64_TFLOPS, "traffic": None,
-                     "kernel": "exh_gray_kernel, both passes (whole os_exhaustive call)",
+                     "kernel": "exh_min_kernel and exh_gray_kernel (whole os_exhaustive call)",
                      "avg_launch_ms": elapsed / args.steps * 1e3,
-                     "algorithmic_flops_per_launch": 5.0 * 2 ** n},
+                     "algorithmic_flops_per_launch": flops},
         "best_energy": e,
     }
     if not args.no_cpu_baseline:
