@@ -24,14 +24,6 @@ namespace os {
 
 namespace {
 
-// This wave's LDS writes are done before its later LDS reads (other lanes
-// read what a lane wrote).
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-  __builtin_amdgcn_wave_barrier();
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-}
-
 // Bit j of replica lane in a wave's transposed planes (the bit-field extract
 // reads only the low 5 bits of its offset).
 __device__ __forceinline__ uint32_t plane_bit(const uint32_t *xs, int j, int lane) {

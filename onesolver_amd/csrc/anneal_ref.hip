@@ -100,8 +100,9 @@ __global__ __launch_bounds__(64) void ref_anneal_kernel(int n, const double *__r
 // later lanes keep, with the chain's own fma; then the tests of the lanes
 // behind it are taken again.  So a rejection costs a 64th of a step and an
 // acceptance some forty instructions.  The n fields themselves take the
-// window's accepted rows of Q at its end, in order, several requested at once.  The couplings between the window's sites come from
-// Q staged in LDS (kQLds, n <= 64) or are gathered into LDS at its start.
+// window's accepted rows of Q at its end, in order, several requested at once.
+// The couplings between the window's sites come from Q staged in LDS (kQLds,
+// n <= 64) or are gathered into LDS at its start.
 // The state and the best state are bit words, word w in lane w.
 //
 // The test exp(-dE / b) > u is decided by dE against -b ln u, made once per

@@ -572,7 +572,8 @@ Shape select_shape(CsrBatch &b, const CsrRun &run, int site_order, bool tune_it)
 // the graph already holds that shape.
 void ensure_graph(CsrBatch &b, const Shape &sh, bool energy) {
   hipStream_t s = b.ctx->stream;
-  if (b.gexec && b.g_mode == b.mode && b.g_seq == sh.seq && b.g_s_sites == sh.s_sites && b.g_waves == sh.waves &&
+  if (b.gexec && b.g_mode == b.mode && b.g_seq == sh.seq && b.g_s_sites == sh.s_sites &&
+      b.g_waves == sh.waves &&
       b.g_groups == sh.groups && b.g_uniform == sh.uniform && b.g_limit == sh.limit &&
       b.g_items_c == b.items_c.ptr && b.g_items_s == b.items_s.ptr && b.g_Rp == b.Rp && b.g_energy == energy)
     return;

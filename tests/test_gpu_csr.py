@@ -157,6 +157,27 @@ def test_csr_tuned_index_order_matches_oracle(ctx, sizes):
     b.close()
 
 
+@pytest.mark.parametrize("upper", [True, False])
+def test_csr_tuned_index_order_with_one_sided_rows(ctx, upper):
+    """Rows that list only their higher-index (or only their lower-index)
+    neighbours: index order still decides which state an update reads."""
+    rng = np.random.default_rng(4)
+    n, S, R = 300, 6, 100
+    rows = [np.sort(rng.choice(np.arange(j + 1, n) if upper else np.arange(j), size=min(
+        5, n - 1 - j if upper else j), replace=False)) for j in range(n)]
+    rp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    cl = np.concatenate(rows).astype(np.int32)
+    inst = (rp, cl, np.float32(rng.normal(size=len(cl))).astype(np.float64),
+            np.float32(rng.normal(size=n)).astype(np.float64))
+    ts = _tscale(S)
+    print(f"[gpu] csr one-sided rows upper={upper}", flush=True)
+    b = onesolver_amd.CsrBatch(ctx, [inst])
+    out = b.anneal(R, ts, seed=6, final_states=True, tune=True)
+    fin, bs, _ = oracle.sweep_csr(*inst, ts, R, seed=6, instance=0)
+    assert (out["final_states"][0] == fin).all()
+    b.close()
+
+
 def test_csr_graph_replays_with_new_parameters(ctx):
     insts = _batch()
     R, S = 64, 12
