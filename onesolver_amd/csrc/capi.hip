@@ -168,9 +168,6 @@ int os_exhaustive(os_ctx *ctx_, int n, const double *q_upper, uint8_t *best_stat
                       "exhaustive search supports n <= " + std::to_string(os::exhaustive_max_n()));
     Ctx &c = *reinterpret_cast<Ctx *>(ctx_);
     c.activate();
-    bool finite = true;
-    for (int i = 0; i < n; ++i)
-      for (int j = i; j < n; ++j) finite = finite && std::isfinite(q_upper[(size_t)i * n + j]);
     const size_t qbytes = sizeof(double) * (size_t)n * n;
     const size_t parts = os::exhaustive_partials(n);
     c.b_q.ensure(qbytes);
@@ -180,7 +177,7 @@ int os_exhaustive(os_ctx *ctx_, int n, const double *q_upper, uint8_t *best_stat
     OS_HIP_CHECK(hipMemcpyAsync(c.b_q.ptr, q_upper, qbytes, hipMemcpyHostToDevice, c.stream));
     double e = 0.0;
     uint64_t x = 0;
-    os::exhaustive_solve(c.stream, n, c.b_q.as<double>(), finite, c.b_fields.as<double>(),
+    os::exhaustive_solve(c.stream, n, q_upper, c.b_q.as<double>(), c.b_fields.as<double>(),
                          c.b_energy.as<double>(), c.b_scratch.as<uint64_t>(), parts, &e, &x);
     for (int i = 0; i < n; ++i) best_state[i] = (uint8_t)((x >> i) & 1u);
     *best_energy = e;

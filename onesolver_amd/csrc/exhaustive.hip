@@ -15,14 +15,18 @@
 // them in Gray-code order in segments of 2^S states, each from its literal
 // energy.
 //   pass 1: every thread's minimum energy, and the minimum E_w of them (below);
-//   pass 2: only the threads whose minimum is within tol = 1e-9 (|E_w| + 1)
-//           of E_w walk again, their states split over 2^K threads each where
-//           few blocks hold them; every state whose walk energy is within tol
-//           of E_w gets its literal energy, and the (literal energy, index)
-//           minimum of those is the answer.
-// A walk energy differs from the literal one by the rounding of at most 2^S
-// steps, far below tol, so the literal minimum is always among the
-// candidates and the result equals the reference's.
+//   pass 2: only the threads whose minimum is near E_w walk again, their states
+//           split over 2^K threads each where few blocks hold them; every state
+//           whose walk energy is near E_w gets its literal energy, and the
+//           (literal energy, index) minimum of those is the answer.
+// "Near" is what rounding can make of the walks, which scales with the
+// coefficients and not with E_w (large penalties cancel in the minimum).  With
+// exact energies E, let e1, e2 and el bound the rounding of pass 1, pass 2 and
+// the literal sums, and x a state of lowest literal energy: where E_w is pass
+// 1's energy of y, E(x) <= E(y) + 2 el <= E_w + e1 + 2 el, so pass 1 finds x's
+// thread within 2 e1 + 2 el of E_w and pass 2 finds x within e1 + e2 + 2 el:
+// the literal minimum is always among the candidates and the result equals the
+// reference's.  The bounds are walk_bound()'s.
 #include <algorithm>
 #include <cfloat>
 #include <cmath>
@@ -227,13 +231,14 @@ struct ActiveBlocks {
   int id[kMaxActive];
 };
 
-// Pass 2: walks the states of the threads of pass 1 with tmin <= thr and writes
-// per-block (literal energy, index) minima of the candidates e_walk <= thr.  A
-// thread takes 2^(L-K) of a pass-1 thread's 2^L states; blocks are those of
-// `act`, 2^K each, or all of them (K = 0, act.count 0).
+// Pass 2: walks the states of the threads of pass 1 with tmin <= thr1 and writes
+// per-block (literal energy, index) minima of the candidates e_walk <= thr2.  A
+// walk energy that is NaN (sums beyond FP64) is a candidate.  A thread takes
+// 2^(L-K) of a pass-1 thread's 2^L states; blocks are those of `act`, 2^K each,
+// or all of them (K = 0, act.count 0).
 __global__ __launch_bounds__(kThreads) void exh_gray_kernel(int n, int L, int K, ActiveBlocks act,
                                                             const double *__restrict__ q,
-                                                            double thr,
+                                                            double thr1, double thr2,
                                                             const double *__restrict__ tmin,
                                                             double *__restrict__ out_e,
                                                             uint64_t *__restrict__ out_x) {
@@ -245,7 +250,7 @@ __global__ __launch_bounds__(kThreads) void exh_gray_kernel(int n, int L, int K,
   L -= K;
   const int S = min(L, kSegBits);
   bool active = t < (1ull << (n - L));
-  if (active) active = tmin[t >> K] <= thr;
+  if (active) active = !(tmin[t >> K] > thr1);
   if (!__syncthreads_or(active)) {  // no candidate in this block
     if (threadIdx.x == 0) {
       out_e[blockIdx.x] = DBL_MAX;
@@ -289,7 +294,7 @@ __global__ __launch_bounds__(kThreads) void exh_gray_kernel(int n, int L, int K,
             if (j != b) h[j] = fma(s[b], j < b ? ql[j][b] : ql[b][j], h[j]);
           s[b] = -s[b];
         }
-        if (e <= thr) {
+        if (!(e > thr2)) {
           const uint64_t x = xhi | (low0 ^ (uint32_t)(pos ^ (pos >> 1)));
           const double v = literal_energy(n, qs, x);
           if (better(v, x, emin, xmin)) {
@@ -321,9 +326,50 @@ static void gray_shape(int n, int *P, int *L) {
   *L = n - *P;
 }
 
-void exhaustive_solve(hipStream_t st, int n, const double *q_dev, bool finite, double *tmin,
-                      double *part_e, uint64_t *part_x, size_t part_cap, double *best_e,
-                      uint64_t *best_x) {
+namespace {
+
+// What bounds the rounding of energies of the upper triangle of q.
+struct Size {
+  double sum = 0.0;    // sum of all |q_ij|: no exact energy is larger
+  double field = 0.0;  // largest |q_jj| + sum of |q_ij| of a bit: no exact field is
+};
+
+Size coefficient_size(int n, const double *q) {
+  Size s;
+  std::vector<double> f(n, 0.0);
+  for (int i = 0; i < n; ++i)
+    for (int j = i; j < n; ++j) {
+      const double a = std::fabs(q[(size_t)i * n + j]);
+      s.sum += a;
+      f[i] += a;
+      if (j != i) f[j] += a;
+    }
+  for (double v : f) s.field = std::max(s.field, v);
+  return s;
+}
+
+// Bound of |walk energy - exact energy| over a segment of `flips` flips, to
+// first order in u = 2^-53 and a quarter more for the rest.  The segment starts
+// from a literal energy (at most n (n + 1) / 2 additions) and fields of at most
+// n additions; each flip adds one rounding to the energy and one to every field,
+// and the flipped field's error so far to the energy.  The closed form of pass 1
+// adds three fields and a few roundings.  flips = 0: a literal energy.
+double walk_bound(int n, int flips, const Size &s) {
+  const double fields = (flips * (n + 0.5 * flips) + 3.0 * (n + flips)) * s.field;
+  return 1.25 * 0x1p-53 * ((0.5 * n * (n + 1) + flips + 8.0) * s.sum + fields);
+}
+
+}  // namespace
+
+void exhaustive_solve(hipStream_t st, int n, const double *q_host, const double *q_dev,
+                      double *tmin, double *part_e, uint64_t *part_x, size_t part_cap,
+                      double *best_e, uint64_t *best_x) {
+  bool finite = true;
+  for (int i = 0; i < n; ++i)
+    for (int j = i; j < n; ++j) finite = finite && std::isfinite(q_host[(size_t)i * n + j]);
+  const Size size = coefficient_size(n, q_host);
+  // beyond this, a sum of a walk may leave FP64, which no bound covers
+  const bool bounded = size.sum <= 1e300;
   auto reduce = [&](int nb, std::vector<double> *minima) {
     std::vector<double> e(nb);
     std::vector<uint64_t> x(nb);
@@ -341,7 +387,7 @@ void exhaustive_solve(hipStream_t st, int n, const double *q_dev, bool finite, d
     *best_x = bx;
     if (minima) minima->swap(e);
   };
-  if (n <= kLiteralMaxN || (!finite && n <= 30)) {
+  if (n <= kLiteralMaxN || (!bounded && n <= 30)) {
     const int nb = (int)(((1ull << n) + kThreads - 1) / kThreads);
     OS_REQUIRE((size_t)nb <= part_cap, "partials buffer too small");
     exh_literal_kernel<<<nb, kThreads, 0, st>>>(n, q_dev, part_e, part_x);
@@ -360,21 +406,31 @@ void exhaustive_solve(hipStream_t st, int n, const double *q_dev, bool finite, d
   OS_HIP_CHECK(hipGetLastError());
   std::vector<double> minima;
   reduce(nb, &minima);
+  // candidates of pass 1 and, for walks of 2^(L-K) states a thread, of pass 2;
+  // every state where nothing is bounded
   const double ew = *best_e;
-  const double thr = ew + 1e-9 * (std::fabs(ew) + 1.0);
+  const double e1 = walk_bound(n, 17 << (std::min(L, kSegBits) - kMinLow), size);
+  const double el = walk_bound(n, 0, size);
+  const double thr1 = bounded ? ew + 2.0 * (e1 + el) : INFINITY;
+  auto thr2 = [&](int split) {
+    const double e2 = walk_bound(n, 1 << std::min(L - split, kSegBits), size);
+    return bounded ? ew + e1 + e2 + 2.0 * el : INFINITY;
+  };
   // One thread's walk is a serial chain, so its states go to 2^K threads where
   // few blocks hold candidates (most instances: one; n = 32 441 -> 53 us).
   // Instances with many take the undivided walk, which fills the chip by itself.
   ActiveBlocks act{0, {}};
   int found = 0;
   for (int i = 0; i < nb; ++i)
-    if (minima[i] <= thr && found++ < kMaxActive) act.id[act.count++] = i;
+    if (!(minima[i] > thr1) && found++ < kMaxActive) act.id[act.count++] = i;
   int K = std::min(8, L - kLow);
   if (found < 1 || found > kMaxActive || ((size_t)found << K) > part_cap) K = act.count = 0;
   const int nb2 = act.count ? found << K : nb;
-  exh_gray_kernel<<<nb2, kThreads, 0, st>>>(n, L, K, act, q_dev, thr, tmin, part_e, part_x);
+  exh_gray_kernel<<<nb2, kThreads, 0, st>>>(n, L, K, act, q_dev, thr1, thr2(K), tmin, part_e,
+                                            part_x);
   OS_HIP_CHECK(hipGetLastError());
   reduce(nb2, nullptr);
+  if (*best_e == DBL_MAX) throw Error(OS_ERR_INTERNAL, "exhaustive search found no candidate");
 }
 
 size_t exhaustive_thread_slots(int n) {

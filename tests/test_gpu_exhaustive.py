@@ -116,6 +116,54 @@ def test_exhaustive_finds_planted_minimum(ctx, n):
         assert np.array_equal(x, s) and e == -const, (n, k)
 
 
+def _penalised(n, edges, penalty, seed):
+    """Maximum-weight independent set as a QUBO, weights U(0, 1) and a penalty on
+    every edge, and its answer: the lowest literal energy over the independent
+    sets (a penalty above 1 keeps every other state above one of them)."""
+    rng = np.random.default_rng(seed)
+    adj = np.triu(rng.random((n, n)) < edges, 1)
+    w = rng.uniform(0, 1, n)
+    sets = [(0, 0.0)]  # in ascending order of the state index
+    for v in range(n):
+        nbr = sum(1 << int(i) for i in np.nonzero(adj[:, v])[0])
+        sets += [(x | 1 << v, e - float(w[v])) for x, e in sets if not x & nbr]
+    x, e = min(sets, key=lambda t: (t[1], t[0]))
+    return adj * penalty - np.diag(w), x, e
+
+
+@pytest.mark.parametrize("n,edges", [(21, 0.5), (28, 0.5), (32, 0.5), (33, 0.5), (32, 0.3)])
+@pytest.mark.parametrize("penalty", [1e3, 1e6, 1e7, 1e9, 1e13])
+def test_exhaustive_penalties_far_above_the_minimum(ctx, n, edges, penalty):
+    """The walks pass through energies of the size of the penalties, so their
+    rounding scales with those and not with the minimum."""
+    for seed in range(4):
+        q, x, e = _penalised(n, edges, penalty, 10 * n + seed)
+        print(f"[gpu] exhaustive penalties {penalty:g} n={n} edges={edges} seed {seed}", flush=True)
+        st, got = ctx.exhaustive(q)
+        assert got == e, (got, e)
+        assert sum(int(b) << i for i, b in enumerate(st)) == x
+
+
+@pytest.mark.parametrize("n", [21, 22, 31])
+def test_exhaustive_sums_beyond_fp64(ctx, n):
+    """Finite coefficients whose sums overflow in some states: the others still
+    have the reference's energies."""
+    q = np.diag(np.full(n, -1.0))
+    q[0, 0] = q[n - 1, n - 1] = q[0, n - 1] = 1.5e308
+    q[3, 4] = 0.25
+    print(f"[gpu] exhaustive overflow n={n}", flush=True)
+    st, e = ctx.exhaustive(q)
+    want = np.ones(n, dtype=np.uint8)
+    want[[0, n - 1]] = 0
+    assert (st == want).all() and e == -(n - 2) + 0.25
+    if n <= 22:
+        rng = np.random.default_rng(n)
+        q = np.triu(rng.uniform(-1, 1, (n, n)) * 10.0 ** rng.integers(-3, 309, (n, n)))
+        st, e = ctx.exhaustive(q)
+        ref_st, ref_e = oracle.exhaustive(_sym(q), n, literal=True)
+        assert e == ref_e and (st == ref_st).all()
+
+
 def test_exhaustive_all_zero_instance(ctx):
     for n in (5, 22):
         st, e = ctx.exhaustive(np.zeros((n, n)))
