@@ -235,7 +235,7 @@ struct ActiveBlocks {
 // per-block (literal energy, index) minima of the candidates e_walk <= thr2.  A
 // walk energy that is NaN (sums beyond FP64) is a candidate.  A thread takes
 // 2^(L-K) of a pass-1 thread's 2^L states; blocks are those of `act`, 2^K each,
-// or all of them (K = 0, act.count 0).
+// or all of them where act.count is 0.
 __global__ __launch_bounds__(kThreads) void exh_gray_kernel(int n, int L, int K, ActiveBlocks act,
                                                             const double *__restrict__ q,
                                                             double thr1, double thr2,
@@ -418,14 +418,19 @@ void exhaustive_solve(hipStream_t st, int n, const double *q_host, const double 
   };
   // One thread's walk is a serial chain, so its states go to 2^K threads where
   // few blocks hold candidates (most instances: one; n = 32 441 -> 53 us).
-  // Instances with many take the undivided walk, which fills the chip by itself.
+  // Instances with many fill the chip by themselves; their threads are split as
+  // far as 2^20 threads and walks of 2^kLow states allow (all states tied, n = 26:
+  // 5.8 ms undivided, SPLITMS split in two).
   ActiveBlocks act{0, {}};
   int found = 0;
   for (int i = 0; i < nb; ++i)
     if (!(minima[i] > thr1) && found++ < kMaxActive) act.id[act.count++] = i;
   int K = std::min(8, L - kLow);
-  if (found < 1 || found > kMaxActive || ((size_t)found << K) > part_cap) K = act.count = 0;
-  const int nb2 = act.count ? found << K : nb;
+  if (found > kMaxActive || ((size_t)found << K) > part_cap) {
+    K = std::min(n - kLow, kMaxTopBits) - P;
+    act.count = 0;
+  }
+  const int nb2 = (act.count ? found : nb) << K;
   exh_gray_kernel<<<nb2, kThreads, 0, st>>>(n, L, K, act, q_dev, thr1, thr2(K), tmin, part_e,
                                             part_x);
   OS_HIP_CHECK(hipGetLastError());
