@@ -10,7 +10,8 @@
 //   - an accepted flip updates all fields with row s of Q (coalesced,
 //     Q is symmetric), E += dE;
 //   - best state copied whenever E < E_best (annealing.hpp:115-121).
-// ref_anneal_kernel (n > 1024) takes these steps one by one.
+// ref_anneal_kernel takes these steps one by one, ref_anneal_window_kernel 64 at
+// a time; launch_ref_anneal says which runs.
 #include "os_kernels.h"
 
 namespace os {
@@ -121,6 +122,21 @@ __global__ __launch_bounds__(64) void ref_anneal_kernel(int n, const double *__r
 // Above 1024 spins 32 fields, as many diagonal entries and two rows of a lane
 // no longer fit 256 registers; ref_anneal_kernel takes over there.
 constexpr int kRefWindowN = 1024;
+// For 64 < n the window's couplings (33 .. 40 KB of LDS) leave four tries a CU,
+// 1024 on the chip, where ref_anneal_kernel has up to 32 a CU.  Up to two rounds
+// of them the window kernel is never slower, however many attempts are accepted;
+// beyond, the other one catches up, first where the schedule is hot, and from 768
+// spins on it never does (its rows no longer hide behind one another).  Whole
+// calls of 300 attempts, all accepted, ms, ref_anneal_kernel | window: n = 65
+// 2048 tries 0.41 | 0.40, 4096 0.58 | 0.72; n = 128 2048 0.41 | 0.38, 4096 0.53 |
+// 0.69, 16384 1.46 | 2.53; n = 256 4096 0.85 | 0.87, 16384 2.24 | 3.25; n = 640
+// 2048 1.79 | 1.17, 4096 2.04 | 2.06, 16384 5.6 | 7.3; n = 768 2048 2.49 | 1.39,
+// 16384 9.5 | 9.0; n = 1024 16384 18.5 | 11.7.
+constexpr uint32_t kRefWindowTries = 2048;
+constexpr int kRefAlwaysWindowN = 768;
+static bool ref_window(int n, uint32_t tries) {
+  return n <= 64 || (n <= kRefWindowN && (tries <= kRefWindowTries || n >= kRefAlwaysWindowN));
+}
 
 __device__ __forceinline__ double readlane_f64(double v, int l) {
   const uint64_t b = (uint64_t)__double_as_longlong(v);
@@ -325,7 +341,7 @@ void launch_ref_anneal(hipStream_t st, int n, const double *q, const double *bet
   const uint64_t total = (uint64_t)num_iter * (uint64_t)spb;
   const int W = (n + 31) / 32;
   const size_t lds = (ref_lds_bytes(n) + 15) & ~(size_t)15;
-  if (n <= kRefWindowN) {
+  if (ref_window(n, num_tries)) {
     // fields per lane: the next power of two of n / 64
     const size_t wlds = sizeof(double) * (n <= 64 ? (size_t)n * n : (size_t)64 * 64 + n);
 #define OS_WINDOW(NC, QL)                                                           \

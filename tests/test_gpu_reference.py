@@ -118,6 +118,29 @@ def test_reference_anneal_windows_match_oracle_chain(ctx, n):
     assert be == e_or.min() and (best == s_or[int(np.argmin(e_or))]).all()
 
 
+@pytest.mark.parametrize("n", [64, 65, 640, 767, 768])
+def test_reference_anneal_many_tries_match_oracle_chain(ctx, n):
+    """Both sides of the numbers of tries and spins at which another kernel takes
+    the chains: a try's chain does not depend on the others, so the runs agree, and
+    with the oracle bit for bit (integer Q)."""
+    rng = np.random.default_rng(n)
+    q = np.triu(rng.integers(-3, 4, (n, n)).astype(np.float64))
+    q = q + np.triu(q, 1).T
+    beta = np.geomspace(0.5, 2.0, 70) * np.sqrt(n)
+    s_or, e_or = oracle.anneal(q, n, beta, 2049 if n < 100 else 64, seed=7)
+    last = None
+    for tries in (2048, 2049):
+        print(f"[gpu] reference n={n} tries={tries}", flush=True)
+        best, be, states, energies = ctx.anneal_reference(q, beta, tries, seed=7)
+        k = min(tries, len(e_or))
+        assert (states[:k] == s_or[:k]).all() and np.array_equal(energies[:k], e_or[:k])
+        i = int(np.argmin(energies))
+        assert be == energies[i] and (best == states[i]).all()
+        if last is not None:
+            assert (states[:2048] == last[0]).all() and np.array_equal(energies[:2048], last[1])
+        last = states, energies
+
+
 def test_reference_anneal_large_n_uses_global_fields(ctx):
     rng = np.random.default_rng(5)
     n = 4100  # above the LDS-resident field limit
