@@ -18,6 +18,8 @@
 // sweep's number (run->sweep_base + the launch's own sweep index); the
 // FP64 running energy adds dE.  At the end of every sweep a replica whose
 // running energy is below its best copies its state to the best-state planes.
+#include <algorithm>
+
 #include "os_kernels.h"
 
 namespace os {
@@ -921,8 +923,10 @@ __global__ __launch_bounds__(64 * kEnergyWaves) void csr_energy_kernel(
     const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col,
     const double *__restrict__ val, const double *__restrict__ diag64,
     const uint32_t *__restrict__ bits, double *__restrict__ out) {
-  __shared__ double part[kEnergyWaves][64];
-  extern __shared__ uint32_t eplanes[];  // [words][64]
+  // [words][64], then the waves' sums in their place: the largest instances
+  // leave no LDS beside their planes
+  extern __shared__ __attribute__((aligned(16))) uint32_t eplanes[];
+  double(*part)[64] = reinterpret_cast<double(*)[64]>(eplanes);
   const int it = blockIdx.x;  // < num_items: the grid has one work-group per item
   const int lane = threadIdx.x & 63;
   const int w = threadIdx.x >> 6;
@@ -965,6 +969,7 @@ __global__ __launch_bounds__(64 * kEnergyWaves) void csr_energy_kernel(
     }
     e += bit(j) ? s : 0.0;
   }
+  __syncthreads();  // the planes are read
   part[w][lane] = e;
   __syncthreads();
   if (w == 0) {
@@ -1227,7 +1232,11 @@ void launch_csr_energy(hipStream_t st, const CsrInst *inst, const int2 *items, i
                        const double *val, const double *diag64, const uint32_t *bits,
                        double *out) {
   if (num_items == 0) return;
-  const size_t lds = (size_t)max_words * 64 * sizeof(uint32_t);
+  const size_t lds = std::max((size_t)max_words * 64 * sizeof(uint32_t),
+                              sizeof(double) * kEnergyWaves * 64);
+  if (lds > 65536)
+    OS_HIP_CHECK(hipFuncSetAttribute((const void *)csr_energy_kernel,
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   csr_energy_kernel<<<num_items, 64 * kEnergyWaves, lds, st>>>(inst, items, num_items, Rp,
                                                                 row_ptr, col, val, diag64, bits,
                                                                 out);

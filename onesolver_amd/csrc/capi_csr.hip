@@ -834,7 +834,7 @@ int os_csr_batch_create(os_ctx *ctx_, int32_t num_instances, const int32_t *n,
     b->total_spins = spins;
 
     OS_REQUIRE(os::csr_lds_bytes(1, b->max_words) <= 160 * 1024,
-               "csr batch: instance too large for the LDS-resident state (n <= 40000)");
+               "csr batch: instance too large for the LDS-resident state (n <= 20479)");
     hipStream_t s = c.stream;
     b->ell_col.ensure(sizeof(int32_t) * std::max<size_t>(ell_c.size(), 4));
     b->ell_val.ensure(sizeof(float) * std::max<size_t>(ell_v.size(), 4));

@@ -126,6 +126,27 @@ def test_csr_prefetch_kernel_matches_oracle(ctx, tune):
     b.close()
 
 
+@pytest.mark.parametrize("n", [19967, 19968, 20479])
+def test_csr_largest_instances(ctx, n):
+    """Up to the largest instance whose bit planes fit the LDS, beside which no kernel of a run may need any."""
+    insts = [instances.regular_csr(n, 4, seed=7, instance=0)]
+    R, ts = 64, _tscale(2)
+    b = onesolver_amd.CsrBatch(ctx, insts)
+    for order in (0, 1):
+        print(f"[gpu] csr largest n={n} order={order}", flush=True)
+        out = b.anneal(R, ts, seed=2, final_states=True, site_order=order, tune=False)
+        if order:
+            _check_colour_against_oracle(b, out, insts, ts, R, 2, 0)
+        else:
+            _check_against_oracle(out, insts, ts, R, 2, 0)
+    b.close()
+
+
+def test_csr_rejects_instances_beyond_the_lds(ctx):
+    with pytest.raises(onesolver_amd.OneSolverError, match="20479"):
+        onesolver_amd.CsrBatch(ctx, [instances.regular_csr(20480, 4, seed=7, instance=0)])
+
+
 def _ring(n, seed):
     """A cycle with real weights: index order leaves no two neighbours of it for
     the same step."""
