@@ -39,13 +39,14 @@ struct CsrBatch {
   DevBuf d_inst, ell_col, ell_val, diag, diag64, row_ptr, col, val64;
   // steps of a sweep in the batch's array of them
   struct Steps {
-    int32_t sites, steps;
-    int64_t off;
+    int32_t sites = 0, steps = 0;
+    int64_t off = 0;
   };
   // colour classes: sites class by class (offset spin_off), class starts
   // (offset class_off), and the positions of each step
   DevBuf corder, csteps;
-  std::vector<Steps> h_csteps[3];  // at 4, 8 and 16 sites per step
+  std::vector<Steps> h_csteps[3];  // at 4, 8 and 16 sites per step; steps 0: not made yet
+  std::vector<int32_t> h_csteps_all;
   std::vector<int32_t> h_order, h_cstart;
   // ELL rows and diagonal in that visiting order
   DevBuf pell_col, pell_val, pdiag;
@@ -66,8 +67,8 @@ struct CsrBatch {
   enum Seq { kPlain = 0, kPrefetch = 1, kSched = 2 };
   int waves = 0, groups = 0;
   int seq = kPlain;
-  // scheduled kernel: every instance's schedules at 4, 8 and 16 sites per step,
-  // the policy in use (s_sites; 0: none tried) and its work items ((instance,
+  // scheduled kernel: every instance's schedules at 4, 8 and 16 sites per step
+  // (empty before the first run that may use them), the policy in use (s_sites; 0: none tried) and its work items ((instance,
   // group of 64/isites replicas)), built for (items_s_sites, items_s_Rp)
   std::vector<Steps> h_sched[3];
   DevBuf sched, items_s;
@@ -226,6 +227,137 @@ int sites_for(int n, int uniform, int limit) {
 // limit and the same under 40 and 80 KB; n = 40000 only fits as bits.
 constexpr int kByteSpinLimit = 16 * 1024;
 
+// Schedules of an instance for the scheduled index-order kernel at G = 4, 8 and
+// 16 sites per step: each site goes to the first step with room after every
+// lower-index site that it reads or that reads it.  A schedule that fills less
+// than half of its slots is left out and the next smaller G stands in for it.
+void build_schedules(const CsrInst &d, const int32_t *rp, const int32_t *cl,
+                     std::vector<int32_t> &out, CsrBatch::Steps (&made)[3]) {
+  const int n = d.n;
+  std::vector<int32_t> earliest(n), fill, next, step(n);
+  for (int k = 0; k < 3; ++k) {
+    const int G = 4 << k;
+    std::fill(earliest.begin(), earliest.end(), 0);
+    fill.assign((size_t)n + 1, 0);
+    next.resize((size_t)n + 1);  // union-find: the first step from here with room
+    std::iota(next.begin(), next.end(), 0);
+    int steps = 0;
+    for (int j = 0; j < n; ++j) {
+      int e = earliest[j];
+      for (int q = rp[j]; q < rp[j + 1]; ++q)
+        if (cl[q] < j) e = std::max(e, step[cl[q]] + 1);
+      int f = e;
+      while (next[f] != f) f = next[f] = next[next[f]];
+      step[j] = f;
+      if (++fill[f] == G) next[f] = f + 1;
+      steps = std::max(steps, f + 1);
+      for (int q = rp[j]; q < rp[j + 1]; ++q)
+        if (cl[q] > j) earliest[cl[q]] = std::max(earliest[cl[q]], f + 1);
+    }
+    steps += steps & 1;
+    if (k > 0 && (int64_t)steps * G > 2 * (int64_t)n + 64) {
+      made[k] = made[k - 1];
+      continue;
+    }
+    const size_t at = out.size();
+    out.resize(at + (size_t)(steps + 2) * G, n);  // two idle steps follow
+    std::fill(fill.begin(), fill.end(), 0);
+    for (int j = 0; j < n; ++j) out[at + (size_t)step[j] * G + fill[step[j]]++] = j;
+    made[k] = {G, steps, (int64_t)at};
+  }
+}
+
+// Steps of the colour-class order at G sites per step: the positions of each
+// class by G; an idle slot repeats its step's first position with bit 31 set.
+std::vector<int32_t> class_steps(const int32_t *start, int ncol, int G, CsrBatch::Steps &made) {
+  constexpr int32_t kIdle = INT32_MIN;
+  int steps = 0;
+  for (int c = 0; c < ncol; ++c) steps += (start[c + 1] - start[c] + G - 1) / G;
+  const int even = steps + (steps & 1);
+  // an even number, and two more for the requests made ahead: the last
+  // position again, idle
+  std::vector<int32_t> out((size_t)(even + 2) * G, (start[ncol] - 1) | kIdle);
+  int32_t *o = out.data();
+  for (int c = 0; c < ncol; ++c)
+    for (int p0 = start[c]; p0 < start[c + 1]; p0 += G, o += G)
+      for (int s = 0; s < G; ++s) o[s] = p0 + s < start[c + 1] ? p0 + s : p0 | kIdle;
+  made = {G, even, 0};
+  return out;
+}
+
+void upload_ints(CsrBatch &b, const std::vector<int32_t> &v, DevBuf &dev) {
+  hipStream_t s = b.ctx->stream;
+  dev.ensure(sizeof(int32_t) * v.size());
+  OS_HIP_CHECK(hipMemcpyAsync(dev.ptr, v.data(), sizeof(int32_t) * v.size(),
+                              hipMemcpyHostToDevice, s));
+  OS_HIP_CHECK(hipStreamSynchronize(s));
+}
+
+// Steps and schedules are made when a run first needs them, the steps at the
+// sites per step it uses: a batch of 512 instances of 64 .. 2048 spins is created
+// in 19 ms, with all of both in 25 .. 27.
+int sites_index(int sites) { return sites == 4 ? 0 : sites == 8 ? 1 : 2; }
+
+// The colour-class steps of every instance at its CsrInst::sites.
+void need_class_steps(CsrBatch &b) {
+  for (auto &h : b.h_csteps) h.resize(b.I);
+  std::vector<int> todo;
+  for (int i = 0; i < b.I; ++i)
+    if (b.h_csteps[sites_index(b.inst[i].sites)][i].steps == 0) todo.push_back(i);
+  if (todo.empty()) return;
+  std::vector<std::vector<int32_t>> part(todo.size());
+  std::vector<CsrBatch::Steps> made(todo.size());
+  host_parallel_for((int)todo.size(), [&](int t) {
+    const CsrInst &d = b.inst[todo[t]];
+    part[t] = class_steps(b.h_cstart.data() + d.class_off, d.ncol, d.sites, made[t]);
+  });
+  std::vector<int32_t> all(b.h_csteps_all);
+  for (size_t t = 0; t < todo.size(); ++t) {
+    made[t].off = (int64_t)all.size();
+    all.insert(all.end(), part[t].begin(), part[t].end());
+  }
+  b.drop_graph();  // it may hold the steps' former address
+  upload_ints(b, all, b.csteps);
+  b.h_csteps_all.swap(all);
+  for (size_t t = 0; t < todo.size(); ++t)
+    b.h_csteps[sites_index(b.inst[todo[t]].sites)][todo[t]] = made[t];
+}
+
+// The schedules of every instance at 4, 8 and 16 sites per step.
+void need_schedules(CsrBatch &b) {
+  if (!b.h_sched[0].empty()) return;
+  int64_t rows = 0, nnz = 0;  // the couplings are on the GPU only
+  std::vector<int32_t> rp, cl;
+  hipStream_t s = b.ctx->stream;
+  for (const CsrInst &d : b.inst) rows += d.n + 1;
+  rp.resize((size_t)rows);
+  OS_HIP_CHECK(hipMemcpyAsync(rp.data(), b.row_ptr.ptr, sizeof(int32_t) * rp.size(),
+                              hipMemcpyDeviceToHost, s));
+  OS_HIP_CHECK(hipStreamSynchronize(s));
+  for (const CsrInst &d : b.inst) nnz += rp[(size_t)d.row_off + d.n];
+  cl.resize((size_t)nnz);
+  if (nnz)
+    OS_HIP_CHECK(hipMemcpyAsync(cl.data(), b.col.ptr, sizeof(int32_t) * cl.size(),
+                                hipMemcpyDeviceToHost, s));
+  OS_HIP_CHECK(hipStreamSynchronize(s));
+  std::vector<std::vector<int32_t>> part(b.I);
+  std::vector<CsrBatch::Steps> made[3];
+  for (auto &h : made) h.resize(b.I);
+  host_parallel_for(b.I, [&](int i) {
+    const CsrInst &d = b.inst[i];
+    CsrBatch::Steps st[3];
+    build_schedules(d, rp.data() + d.row_off, cl.data() + d.csr_off, part[i], st);
+    for (int k = 0; k < 3; ++k) made[k][i] = st[k];
+  });
+  std::vector<int32_t> all;
+  for (int i = 0; i < b.I; ++i) {
+    for (auto &h : made) h[i].off += (int64_t)all.size();
+    all.insert(all.end(), part[i].begin(), part[i].end());
+  }
+  upload_ints(b, all, b.sched);
+  for (int k = 0; k < 3; ++k) b.h_sched[k].swap(made[k]);
+}
+
 // Sets every instance's sites per step for the policy (uniform, limit) and
 // builds the colour kernel's work items: (instance, group of 64/sites_i
 // replicas), the items of longer estimated runtime first (steps per sweep
@@ -236,10 +368,11 @@ void col_items(CsrBatch &b, int uniform, int limit) {
   std::iota(order.begin(), order.end(), 0);
   std::vector<int64_t> est(b.I);
   int spins[2] = {0, 0};
+  for (CsrInst &d : b.inst) d.sites = sites_for(d.n, uniform, limit);
+  need_class_steps(b);
   for (int i = 0; i < b.I; ++i) {
     CsrInst &d = b.inst[i];
-    d.sites = sites_for(d.n, uniform, limit);
-    const CsrBatch::Steps &cs = b.h_csteps[d.sites == 4 ? 0 : d.sites == 8 ? 1 : 2][i];
+    const CsrBatch::Steps &cs = b.h_csteps[sites_index(d.sites)][i];
     d.csteps = cs.steps;
     d.csteps_off = cs.off;
     est[i] = (int64_t)d.csteps * (d.width + 8);
@@ -289,74 +422,11 @@ void col_items(CsrBatch &b, int uniform, int limit) {
   b.items_c_Rp = b.Rp;
 }
 
-// Schedules of an instance for the scheduled index-order kernel at G = 4, 8 and
-// 16 sites per step: each site goes to the first step with room after every
-// lower-index site that it reads or that reads it.  A schedule that fills less
-// than half of its slots is left out and the next smaller G stands in for it.
-void build_schedules(const CsrInst &d, const int32_t *rp, const int32_t *cl,
-                     std::vector<int32_t> &out, CsrBatch::Steps (&made)[3]) {
-  const int n = d.n;
-  std::vector<int32_t> earliest(n), fill, next, step(n);
-  for (int k = 0; k < 3; ++k) {
-    const int G = 4 << k;
-    std::fill(earliest.begin(), earliest.end(), 0);
-    fill.assign((size_t)n + 1, 0);
-    next.resize((size_t)n + 1);  // union-find: the first step from here with room
-    std::iota(next.begin(), next.end(), 0);
-    int steps = 0;
-    for (int j = 0; j < n; ++j) {
-      int e = earliest[j];
-      for (int q = rp[j]; q < rp[j + 1]; ++q)
-        if (cl[q] < j) e = std::max(e, step[cl[q]] + 1);
-      int f = e;
-      while (next[f] != f) f = next[f] = next[next[f]];
-      step[j] = f;
-      if (++fill[f] == G) next[f] = f + 1;
-      steps = std::max(steps, f + 1);
-      for (int q = rp[j]; q < rp[j + 1]; ++q)
-        if (cl[q] > j) earliest[cl[q]] = std::max(earliest[cl[q]], f + 1);
-    }
-    steps += steps & 1;
-    if (k > 0 && (int64_t)steps * G > 2 * (int64_t)n + 64) {
-      made[k] = made[k - 1];
-      continue;
-    }
-    const size_t at = out.size();
-    out.resize(at + (size_t)(steps + 2) * G, n);  // two idle steps follow
-    std::fill(fill.begin(), fill.end(), 0);
-    for (int j = 0; j < n; ++j) out[at + (size_t)step[j] * G + fill[step[j]]++] = j;
-    made[k] = {G, steps, (int64_t)at};
-  }
-}
-
-// Steps of the colour-class order at G = 4, 8 and 16 sites per step: the
-// positions of each class by G; an idle slot repeats its step's first position
-// with bit 31 set.
-void class_steps(const std::vector<int32_t> &start, std::vector<int32_t> &out,
-                 CsrBatch::Steps (&made)[3]) {
-  constexpr int32_t kIdle = INT32_MIN;
-  for (int k = 0; k < 3; ++k) {
-    const int G = 4 << k;
-    const size_t at = out.size();
-    for (size_t c = 0; c + 1 < start.size(); ++c)
-      for (int p0 = start[c]; p0 < start[c + 1]; p0 += G)
-        for (int s = 0; s < G; ++s)
-          out.push_back(p0 + s < start[c + 1] ? p0 + s : p0 | kIdle);
-    int steps = (int)((out.size() - at) / G);
-    // an even number, and two more for the requests made ahead: the last
-    // position again, idle
-    const int32_t last = start.back() - 1;
-    const int extra = (steps & 1) + 2;
-    out.insert(out.end(), (size_t)extra * G, last | kIdle);
-    made[k] = {G, steps + (steps & 1), (int64_t)at};
-  }
-}
-
 // Sets every instance's schedule for `sites` (4, 8 or 16) sites per step and
 // builds the scheduled kernel's work items, longest first.
 void sched_items(CsrBatch &b, int sites) {
   if (b.items_s_sites == sites && b.items_s_Rp == b.Rp) return;
-  const int k = sites == 4 ? 0 : sites == 8 ? 1 : 2;
+  const int k = sites_index(sites);
   std::vector<int> order(b.I);
   std::iota(order.begin(), order.end(), 0);
   int lds = 0;
@@ -388,7 +458,7 @@ void sched_items(CsrBatch &b, int sites) {
 // Work-groups of the scheduled kernel at `sites` sites per step, 0 where an
 // instance does not fit the LDS (the items are then not built).
 int sched_groups(CsrBatch &b, int sites) {
-  const int k = sites == 4 ? 0 : sites == 8 ? 1 : 2;
+  const int k = sites_index(sites);
   for (int i = 0; i < b.I; ++i)
     if (csr_sched_lds_bytes(b.inst[i].n, b.h_sched[k][i].sites) > 160 * 1024) return 0;
   sched_items(b, sites);
@@ -467,6 +537,7 @@ void tune(CsrBatch &b, const CsrRun &full) {
       b.s_sites = sites;
     }
   };
+  need_schedules(b);
   for (int sites : {4, 8, 16}) {
     const int g = sched_groups(b, sites);
     if (g < 1) continue;
@@ -758,9 +829,7 @@ int os_csr_batch_create(os_ctx *ctx_, int32_t num_instances, const int32_t *n,
     const int nd = (int)ds.size();
     std::vector<int32_t> ell_c((size_t)ell);
     std::vector<float> ell_v((size_t)ell, 0.0f), dg((size_t)spins);
-    std::vector<std::vector<int32_t>> cst(nd), cord(nd), sch(nd), cls(nd);
-    for (auto &h : b->h_csteps) h.resize(nd);
-    for (auto &h : b->h_sched) h.resize(nd);
+    std::vector<std::vector<int32_t>> cst(nd), cord(nd);
     std::vector<const char *> err(nd, nullptr);
     os::host_parallel_for(nd, [&](int i) {
       os::CsrInst &d = ds[i];
@@ -806,26 +875,16 @@ int os_csr_batch_create(os_ctx *ctx_, int32_t num_instances, const int32_t *n,
       std::vector<int32_t> fill(start.begin(), start.end() - 1);
       cord[i].resize(ni);
       for (int j = 0; j < ni; ++j) cord[i][fill[colour[j]]++] = j;
-      CsrBatch::Steps made[3];
-      os::build_schedules(d, rp, cl, sch[i], made);
-      for (int k = 0; k < 3; ++k) b->h_sched[k][i] = made[k];
-      os::class_steps(start, cls[i], made);
-      for (int k = 0; k < 3; ++k) b->h_csteps[k][i] = made[k];
     });
     // the first failing instance in order, as a serial pass reports it
     for (int i = 0; i < nd; ++i) OS_REQUIRE(!err[i], err[i]);
     OS_REQUIRE(!bad_msg, bad_msg);
-    // Pass 3 (serial): class and schedule offsets and the concatenated arrays
-    std::vector<int32_t> h_sched, h_csteps;
+    // Pass 3 (serial): class offsets and the concatenated class arrays
     for (int i = 0; i < nd; ++i) {
       os::CsrInst &d = ds[i];
       d.class_off = (int64_t)b->h_cstart.size();
       b->h_cstart.insert(b->h_cstart.end(), cst[i].begin(), cst[i].end());
       b->h_order.insert(b->h_order.end(), cord[i].begin(), cord[i].end());
-      for (auto &h : b->h_sched) h[i].off += (int64_t)h_sched.size();
-      h_sched.insert(h_sched.end(), sch[i].begin(), sch[i].end());
-      for (auto &h : b->h_csteps) h[i].off += (int64_t)h_csteps.size();
-      h_csteps.insert(h_csteps.end(), cls[i].begin(), cls[i].end());
       b->max_words = std::max(b->max_words, d.words);
       b->max_width = std::max(b->max_width, d.width);
       b->total_words += d.words;
@@ -884,15 +943,9 @@ int os_csr_batch_create(os_ctx *ctx_, int32_t num_instances, const int32_t *n,
                                   hipMemcpyHostToDevice, s));
       OS_HIP_CHECK(hipStreamSynchronize(s));
     }
-    b->sched.ensure(sizeof(int32_t) * h_sched.size());
-    OS_HIP_CHECK(hipMemcpyAsync(b->sched.ptr, h_sched.data(), sizeof(int32_t) * h_sched.size(),
-                                hipMemcpyHostToDevice, s));
     b->corder.ensure(sizeof(int32_t) * b->h_order.size());
     OS_HIP_CHECK(hipMemcpyAsync(b->corder.ptr, b->h_order.data(),
                                 sizeof(int32_t) * b->h_order.size(), hipMemcpyHostToDevice, s));
-    b->csteps.ensure(sizeof(int32_t) * h_csteps.size());
-    OS_HIP_CHECK(hipMemcpyAsync(b->csteps.ptr, h_csteps.data(), sizeof(int32_t) * h_csteps.size(),
-                                hipMemcpyHostToDevice, s));
     OS_HIP_CHECK(hipStreamSynchronize(s));
     *out = reinterpret_cast<os_csr_batch *>(b.release());
   });

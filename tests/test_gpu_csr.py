@@ -126,6 +126,20 @@ def test_csr_prefetch_kernel_matches_oracle(ctx, tune):
     b.close()
 
 
+def test_csr_sites_per_step_change_between_runs(ctx, monkeypatch):
+    """Runs of one batch at other sites per step, with and without the graph in
+    between: each has its own steps."""
+    insts = _batch()
+    R, ts = 64, _tscale(5)
+    b = onesolver_amd.CsrBatch(ctx, insts)
+    for sites, graph in ((4, True), (16, False), (4, True), (8, True), (16, True), (8, False)):
+        monkeypatch.setenv("OS_CSR_COLOUR_SITES", str(sites))
+        print(f"[gpu] csr {sites} sites per step, graph={graph}", flush=True)
+        out = b.anneal(R, ts, seed=sites, final_states=True, site_order=1, use_graph=graph)
+        _check_colour_against_oracle(b, out, insts, ts, R, sites, 0)
+    b.close()
+
+
 @pytest.mark.parametrize("n", [19967, 19968, 20479])
 def test_csr_largest_instances(ctx, n):
     """Up to the largest instance whose bit planes fit the LDS, beside which no kernel of a run may need any."""
