@@ -399,8 +399,9 @@ struct BitSpins {
 
 // One work item of the colour-class kernel: replicas [wi.y * 64/G, +64/G) of
 // instance d, G sites per step; lds: this wave's thresholds, then its spins.
-// NCH: 1 for rows of at most 4 couplings, else 2.
-template <int G, int NCH, class Spins>
+// NCH: 1 for rows of at most 4 couplings, else 2.  Off: unsigned type of byte
+// offsets into an instance's rows, 32 bits unless these take 4 GiB.
+template <int G, int NCH, class Spins, class Off>
 __device__ __forceinline__ void col_item(
     const CsrInst &d, int2 wi, char *lds, int lane, int S, int Rp,
     uint32_t k0, uint32_t k1, uint32_t base, int init_mode, int tb, int use_tsr,
@@ -481,14 +482,14 @@ __device__ __forceinline__ void col_item(
       int4 c0, c1;
       float4 v0, v1;
     };
-    // loads at a uniform base plus a 32-bit byte offset
-    auto at16 = [](const void *base, uint32_t off) {
+    // loads at a uniform base plus a byte offset
+    auto at16 = [](const void *base, Off off) {
       return reinterpret_cast<const char *>(base) + off;
     };
     auto fetch = [&](int v) {
       Step st;
       const int pos = v & 0x7FFFFFFF;
-      const uint32_t ro = (uint32_t)pos * (uint32_t)chunks * 16u;  // row's byte offset
+      const Off ro = (Off)pos * (Off)chunks * 16u;  // row's byte offset
       st.v = v;
       st.j = *reinterpret_cast<const int32_t *>(at16(ord, (uint32_t)pos * 4u));
       st.dj = *reinterpret_cast<const float *>(at16(pdg, (uint32_t)pos * 4u));
@@ -539,7 +540,7 @@ __device__ __forceinline__ void col_item(
         h = fmaf(x6, cur.v1.z, h);
         h = fmaf(x7, cur.v1.w, h);
         for (int cc = 2; cc < chunks; ++cc) {
-          const uint32_t ro = ((uint32_t)pos * (uint32_t)chunks + (uint32_t)cc) * 16u;
+          const Off ro = ((Off)pos * (Off)chunks + (Off)cc) * 16u;
           const int4 ci = *reinterpret_cast<const int4 *>(at16(pcol, ro));
           const float4 vi = *reinterpret_cast<const float4 *>(at16(pval, ro));
           h = fmaf((float)x(ci.x), vi.x, h);
@@ -642,16 +643,17 @@ __global__ __launch_bounds__(256) void csr_sweep_col_kernel(
 #define OS_COL_ITEM(GG)                                                                         \
   do {                                                                                          \
     if (d.width == 4)                                                                           \
-      col_item<GG, 1, Spins<GG>>(d, wi, wl, lane, S, Rp, k0, k1, base, init_mode, tb, use_tsr,  \
-                                 tsr, ell_col, ell_val, diag, corder, csteps, pell_col,         \
-                                 pell_val, pdiag, tscale, init_bits, best_bits, final_bits,     \
-                                 e_best, e_final);                                              \
+      OS_COL_RUN(GG, 1, uint32_t);                                                              \
+    else if ((int64_t)d.n * d.width < (int64_t)1 << 30)                                         \
+      OS_COL_RUN(GG, 2, uint32_t);                                                              \
     else                                                                                        \
-      col_item<GG, 2, Spins<GG>>(d, wi, wl, lane, S, Rp, k0, k1, base, init_mode, tb, use_tsr,  \
-                                 tsr, ell_col, ell_val, diag, corder, csteps, pell_col,         \
-                                 pell_val, pdiag, tscale, init_bits, best_bits, final_bits,     \
-                                 e_best, e_final);                                              \
+      OS_COL_RUN(GG, 2, uint64_t);                                                              \
   } while (0)
+#define OS_COL_RUN(GG, NCH, OFF)                                                                \
+  col_item<GG, NCH, Spins<GG>, OFF>(d, wi, wl, lane, S, Rp, k0, k1, base, init_mode, tb,        \
+                                    use_tsr, tsr, ell_col, ell_val, diag, corder, csteps,       \
+                                    pell_col, pell_val, pdiag, tscale, init_bits, best_bits,    \
+                                    final_bits, e_best, e_final)
     if (g == 4)
       OS_COL_ITEM(4);
     else if (g == 8)
@@ -659,6 +661,7 @@ __global__ __launch_bounds__(256) void csr_sweep_col_kernel(
     else
       OS_COL_ITEM(16);
 #undef OS_COL_ITEM
+#undef OS_COL_RUN
   }
 }
 

@@ -456,11 +456,14 @@ void sched_items(CsrBatch &b, int sites) {
 }
 
 // Work-groups of the scheduled kernel at `sites` sites per step, 0 where an
-// instance does not fit the LDS (the items are then not built).
+// instance does not fit the LDS or the kernel's 32-bit offsets into its rows (the
+// items are then not built).
 int sched_groups(CsrBatch &b, int sites) {
   const int k = sites_index(sites);
   for (int i = 0; i < b.I; ++i)
-    if (csr_sched_lds_bytes(b.inst[i].n, b.h_sched[k][i].sites) > 160 * 1024) return 0;
+    if (csr_sched_lds_bytes(b.inst[i].n, b.h_sched[k][i].sites) > 160 * 1024 ||
+        (int64_t)b.inst[i].n * b.inst[i].width >= (int64_t)1 << 30)
+      return 0;
   sched_items(b, sites);
   return std::min(b.ctx->num_cus * csr_sched_max_groups_per_cu(b.s_lds), b.num_items_s);
 }

@@ -156,6 +156,29 @@ def test_csr_largest_instances(ctx, n):
     b.close()
 
 
+def test_csr_rows_beyond_4_gib(ctx):
+    """One row of 56000 entries (columns may repeat) pads the rows of an instance
+    to more than 2^32 bytes; the last rows are still their own."""
+    n, hub = 20479, 56000
+    rng = np.random.default_rng(3)
+    deg = np.ones(n, dtype=np.int64)
+    deg[0] = hub
+    rp = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    cl = np.concatenate([rng.integers(1, n, hub), (np.arange(1, n) + 1) % n]).astype(np.int32)
+    vl = rng.integers(-8, 9, len(cl)).astype(np.float64)
+    insts = [(rp, cl, vl, rng.integers(-4, 5, n).astype(np.float64))]
+    R, ts = 64, _tscale(1)
+    print("[gpu] csr rows beyond 4 GiB: create", flush=True)
+    b = onesolver_amd.CsrBatch(ctx, insts)
+    print("[gpu] csr rows beyond 4 GiB: class order", flush=True)
+    out = b.anneal(R, ts, seed=5, final_states=True, site_order=1, tune=False)
+    b.close()
+    order, _ = oracle.csr_colour_order(rp, cl)
+    fin, bs, _ = oracle.sweep_csr(*insts[0], ts, R, seed=5, instance=0, order=order)
+    assert (out["final_states"][0] == fin).all()
+    assert (out["best_states"][0] == bs).all()
+
+
 def test_csr_rejects_instances_beyond_the_lds(ctx):
     with pytest.raises(onesolver_amd.OneSolverError, match="20479"):
         onesolver_amd.CsrBatch(ctx, [instances.regular_csr(20480, 4, seed=7, instance=0)])
