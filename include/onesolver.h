@@ -411,7 +411,9 @@ int os_csr_batch_population(os_csr_batch *batch, const os_csr_population_params 
 /* The launch shape in use (0 before the first run); prefetch: 1 if the
  * kernel variant that requests the next site's row ahead runs (batches whose
  * rows have at most 8 couplings), 2 if the one that updates up to 16 uncoupled
- * sites of a replica together (a tuned batch only), 0 for the general one. */
+ * sites of a replica together (a tuned batch only), 0 for the general one.
+ * OS_CSR_INDEX_SITES (4, 8 or 16) in the environment takes that variant, with so
+ * many sites, tuned or not. */
 int os_csr_batch_launch_shape(os_csr_batch *batch, int32_t *waves_per_group, int32_t *groups,
                               int32_t *prefetch);
 /* The colour-class order's launch shape in use (0 before its first run).

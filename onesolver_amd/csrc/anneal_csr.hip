@@ -589,7 +589,8 @@ __device__ __forceinline__ void col_item(
 
 // Colour-class sweeps over a batch whose instances each have their own sites
 // per step (CsrInst::sites: 4, 8 or 16).  spin_bytes: LDS bytes per wave for the
-// spins (csr_col_spin_bytes, the largest of the batch), behind 4*64 thresholds.
+// spins (csr_col_spin_bytes, the largest of the batch), behind 8*64 thresholds
+// (kColThresholdBytes).
 template <template <int> class Spins>
 __global__ __launch_bounds__(256) void csr_sweep_col_kernel(
     const CsrInst *__restrict__ inst, const int2 *__restrict__ items,

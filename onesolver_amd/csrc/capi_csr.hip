@@ -583,7 +583,7 @@ struct Shape {
 Shape select_shape(CsrBatch &b, const CsrRun &run, int site_order, bool tune_it) {
   Ctx &c = *b.ctx;
   b.mode = site_order;
-  if (b.mode == 0 && b.waves == 0) {
+  if (b.mode == 0 && b.waves == 0 && !std::getenv("OS_CSR_INDEX_SITES")) {
     if (tune_it) {
       tune(b, run);
     } else {
@@ -592,6 +592,22 @@ Shape select_shape(CsrBatch &b, const CsrRun &run, int site_order, bool tune_it)
       b.groups = std::max(
           1, std::min(c.num_cus * csr_max_groups_per_cu(b.seq == CsrBatch::kPrefetch, 1, b.max_words),
                       b.num_items));
+    }
+  }
+  // OS_CSR_INDEX_SITES (4, 8 or 16): the scheduled kernel at that many sites per
+  // step, tuned or not
+  if (b.mode == 0) {
+    const char *senv = std::getenv("OS_CSR_INDEX_SITES");
+    const int forced = senv ? std::atoi(senv) : 0;
+    OS_REQUIRE(!senv || forced == 4 || forced == 8 || forced == 16,
+               "OS_CSR_INDEX_SITES must be 4, 8 or 16");
+    if (forced) {
+      need_schedules(b);
+      OS_REQUIRE(sched_groups(b, forced) > 0,
+                 "OS_CSR_INDEX_SITES: an instance is too large for the scheduled kernel");
+      b.seq = CsrBatch::kSched;
+      b.waves = 1;
+      b.s_sites = forced;
     }
   }
   // OS_CSR_COLOUR_SITES (4, 8 or 16) fixes the colour kernel's sites per step

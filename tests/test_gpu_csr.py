@@ -126,6 +126,20 @@ def test_csr_prefetch_kernel_matches_oracle(ctx, tune):
     b.close()
 
 
+@pytest.mark.parametrize("n", [4062, 4064])
+def test_csr_colour_classes_byte_and_bit_spins(ctx, monkeypatch, n):
+    """Both sides of the size at which a class-order wave of 16 sites per step
+    keeps its spins as bits (n = 4062 is the last even one with a byte each)."""
+    insts = [instances.regular_csr(n, 5, seed=7, instance=9), _irregular(70, 1)]
+    R, ts = 68, _tscale(4)
+    monkeypatch.setenv("OS_CSR_COLOUR_SITES", "16")
+    print(f"[gpu] csr colour classes n={n}, 16 sites per step", flush=True)
+    b = onesolver_amd.CsrBatch(ctx, insts)
+    out = b.anneal(R, ts, seed=13, final_states=True, site_order=1)
+    _check_colour_against_oracle(b, out, insts, ts, R, 13, 0)
+    b.close()
+
+
 def test_csr_sites_per_step_change_between_runs(ctx, monkeypatch):
     """Runs of one batch at other sites per step, with and without the graph in
     between: each has its own steps."""
@@ -198,27 +212,41 @@ def _ring(n, seed):
 @pytest.mark.parametrize("sizes", [
     [(4, 3)], [(15, 4), (16, 5), (17, 4)], [(31, 4), (32, 3), (33, 4)], [(64, 12), (65, 16)],
     [(1024, 8), (127, 6), (8, 3)], [(2048, 9)], [(3000, 3)]])
-def test_csr_tuned_index_order_matches_oracle(ctx, sizes):
-    """The kernel a tuned index-order run picks for few waves updates up to 16
-    uncoupled sites together: edges of its steps and words, rows of one, two and
-    more chunks, chains it cannot pack, isolated spins, and a run that goes on
-    with another number of replicas."""
+@pytest.mark.parametrize("sites", [None, 4, 8, 16])
+def test_csr_tuned_index_order_matches_oracle(ctx, monkeypatch, sizes, sites):
+    """The kernel that a tuned index-order run may pick updates up to 16 uncoupled
+    sites together: edges of its steps and words, rows of one, two and more
+    chunks, chains it cannot pack, isolated spins, and a run that goes on with
+    another number of replicas; with each number of sites, and as tuned."""
+    if sites:
+        monkeypatch.setenv("OS_CSR_INDEX_SITES", str(sites))
     insts = [instances.regular_csr(n, d, seed=5, instance=i) for i, (n, d) in enumerate(sizes)]
     insts += [_ring(50, 9), _partly_isolated(45, 20, 3)]
     S = 7
     ts = _tscale(S)
     b = onesolver_amd.CsrBatch(ctx, insts)
+    if sites == 4 and max(n for n, _ in sizes) > 2000:  # 80 bytes of LDS a spin
+        with pytest.raises(onesolver_amd.OneSolverError, match="too large"):
+            b.anneal(64, ts)
+        b.close()
+        return
     for R, seed in ((100, 3), (200, 4)):
         out = b.anneal(R, ts, seed=seed, instance_base=1, final_states=True, tune=True)
-        print(f"[gpu] csr tuned index order {sizes} R={R} shape={b.launch_shape()}", flush=True)
+        print(f"[gpu] csr tuned index order {sizes} R={R} sites={sites} shape={b.launch_shape()}",
+              flush=True)
+        if sites:
+            assert b.launch_shape()[2] == 2
         _check_against_oracle(out, insts, ts, R, seed, 1)
     b.close()
 
 
 @pytest.mark.parametrize("upper", [True, False])
-def test_csr_tuned_index_order_with_one_sided_rows(ctx, upper):
+@pytest.mark.parametrize("sites", [None, 4, 8, 16])
+def test_csr_tuned_index_order_with_one_sided_rows(ctx, monkeypatch, upper, sites):
     """Rows that list only their higher-index (or only their lower-index)
     neighbours: index order still decides which state an update reads."""
+    if sites:
+        monkeypatch.setenv("OS_CSR_INDEX_SITES", str(sites))
     rng = np.random.default_rng(4)
     n, S, R = 300, 6, 100
     rows = [np.sort(rng.choice(np.arange(j + 1, n) if upper else np.arange(j), size=min(
@@ -231,8 +259,11 @@ def test_csr_tuned_index_order_with_one_sided_rows(ctx, upper):
     print(f"[gpu] csr one-sided rows upper={upper}", flush=True)
     b = onesolver_amd.CsrBatch(ctx, [inst])
     out = b.anneal(R, ts, seed=6, final_states=True, tune=True)
+    if sites:
+        assert b.launch_shape()[2] == 2
     fin, bs, _ = oracle.sweep_csr(*inst, ts, R, seed=6, instance=0)
     assert (out["final_states"][0] == fin).all()
+    assert (out["best_states"][0] == bs).all()
     b.close()
 
 
