@@ -75,10 +75,13 @@ __global__ __launch_bounds__(256) void xq_mfma_kernel(
   const int lane = threadIdx.x & 63;
   const int wc = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int li = lane & 15, lk = lane >> 4;
-  // columns fastest; one grid dimension, whose limit no number of states meets
+  // columns fastest, then tiles of states, over two grid dimensions (xq_grid)
   const int cb = blockIdx.x % (unsigned)ncb;
   const int c0 = cb * kTN + 16 * CT * wc;
-  const int r0 = blockIdx.x / (unsigned)ncb * 16 * RT;
+  unsigned tile = blockIdx.x / (unsigned)ncb;
+  if (blockIdx.y) tile += blockIdx.y * (gridDim.x / (unsigned)ncb);
+  if ((int64_t)tile * (16 * RT) >= R) return;
+  const int r0 = (int)(tile * (16 * RT));
   // instance blockIdx.z: its matrix and its R rows of states / outputs
   q += (size_t)blockIdx.z * n * n;
   bits += (size_t)blockIdx.z * R * W;
@@ -317,6 +320,32 @@ __global__ __launch_bounds__(256) void energy_small_kernel(int n, int W, const d
   out[(size_t)s * count + r] = e;
 }
 
+namespace {
+
+// Grid of xq_mfma_kernel for `tiles` tiles of states by ncb blocks of columns:
+// work-items along a dimension stay below 2^32, so beyond 2^24 work-groups the
+// tiles go over a second one.
+struct XqGrid {
+  unsigned x, y;
+};
+constexpr XqGrid xq_grid(size_t ncb, size_t tiles) {
+  const size_t along = tiles < 0xFFFFFF / ncb ? tiles : 0xFFFFFF / ncb;
+  return {(unsigned)(ncb * along), (unsigned)((tiles + along - 1) / along)};
+}
+constexpr bool xq_grid_holds(size_t ncb, size_t states, size_t rt) {
+  const size_t tiles = (states + 16 * rt - 1) / (16 * rt);
+  const XqGrid g = xq_grid(ncb, tiles);
+  return (size_t)g.x * 256 < (size_t)1 << 32 && g.x % ncb == 0 && g.y <= 65535 &&
+         (size_t)g.x / ncb * g.y >= tiles && (size_t)g.x / ncb * (g.y - 1) < tiles;
+}
+static_assert(xq_grid_holds(1, 1, 1) && xq_grid_holds(128, 4096, 2), "one tile, and N = 16384");
+static_assert(xq_grid_holds(64, 65535 * 128, 2) && xq_grid_holds(65, 65535 * 128, 2) &&
+                  xq_grid_holds(65, 65535 * 128, 1) && xq_grid_holds(1024, 65535 * 128, 2) &&
+                  xq_grid_holds(8, 0x7FFFFFFF, 1),
+              "8.4 million states at any N, 2^31 - 1 at N = 1024");
+
+}  // namespace
+
 void launch_energy_fp64(hipStream_t st, int n, int W, const double *q, int count,
                         const uint32_t *bits, double *out, double *scratch, float *fields, int ldf,
                         unsigned int *drift_max, int num_instances) {
@@ -340,7 +369,8 @@ void launch_energy_fp64(hipStream_t st, int n, int W, const double *q, int count
   const size_t groups32 = (size_t)ncb * ((count + 31) / 32) * num_instances;
 #define OS_XQ(RT)                                                                                \
   do {                                                                                           \
-    const dim3 grid((unsigned)ncb * ((count + 16 * RT - 1) / (16 * RT)), 1, num_instances);      \
+    const XqGrid g = xq_grid(ncb, ((size_t)count + 16 * RT - 1) / (16 * RT));                    \
+    const dim3 grid(g.x, g.y, num_instances);                                                    \
     if (fields)                                                                                  \
       xq_mfma_kernel<true, RT><<<grid, 256, 0, st>>>(n, W, q, count, bits, part, ncb, fields,    \
                                                      ldf, drift_max);                            \
