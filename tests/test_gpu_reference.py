@@ -55,6 +55,57 @@ def test_energy_tiles_match_oracle(ctx, n, counts):
         assert np.array_equal(ctx.energy_fp64(q, st), oracle.energy(q, st)), count
 
 
+def _energy_in_the_kernels_order(q, x):
+    """0.5 sum_j x_j (Y_j + q_jj) with Y = x q summed over k ascending (products by
+    0 or 1 are exact), then columns 16 apart, the tree over 16, 128 columns at a
+    time: every addition the one that the energy kernel documents."""
+    n = q.shape[0]
+    y = np.zeros((len(x), n))
+    for k in range(n):
+        y += x[:, k, None] * q[k]
+    term = y + np.diag(q)
+    e = np.zeros(len(x))
+    for c0 in range(0, n, 128):
+        s = np.zeros((len(x), 16))
+        for c in range(c0, min(c0 + 128, n)):
+            s[:, c % 16] = np.where(x[:, c] > 0, s[:, c % 16] + term[:, c], s[:, c % 16])
+        for o in (1, 2, 4, 8):
+            s = s + s[:, np.arange(16) ^ o]
+        e = e + 0.5 * s[:, 0]
+    return e
+
+
+@pytest.mark.parametrize("n,count", [(65, 40), (127, 33), (128, 17), (129, 64), (300, 50),
+                                     (515, 20), (1024, 16), (200, 9000)])
+def test_energy_sums_are_in_the_documented_order(ctx, n, count):
+    """Coefficients of many magnitudes, where another order of the sums shows in
+    the last bits: equal bit for bit to the documented one."""
+    rng = np.random.default_rng(n)
+    q = np.triu(rng.normal(size=(n, n)) * 10.0 ** rng.uniform(-6, 6, (n, n)))
+    q = q + np.triu(q, 1).T
+    st = rng.integers(0, 2, (count, n)).astype(np.uint8)
+    print(f"[gpu] energy order n={n} count={count}", flush=True)
+    want = _energy_in_the_kernels_order(q, st.astype(np.float64))
+    assert np.array_equal(ctx.energy_fp64(q, st), want)
+    # the coefficients do tell orders apart
+    assert (want != 0.5 * ((st @ q + np.diag(q)) * st).sum(1)).any()
+
+
+@pytest.mark.parametrize("n,count", [(7, 100), (28, 300), (57, 257), (64, 65600)])
+def test_small_energies_are_the_references_sum(ctx, n, count):
+    """n <= 64: the reference's loop over i, then j >= i, bit for bit."""
+    rng = np.random.default_rng(n)
+    q = np.triu(rng.normal(size=(n, n)) * 10.0 ** rng.uniform(-6, 6, (n, n)))
+    q = q + np.triu(q, 1).T
+    st = rng.integers(0, 2, (count, n)).astype(np.uint8)
+    print(f"[gpu] small energies n={n} count={count}", flush=True)
+    e, x = np.zeros(count), st.astype(np.float64)
+    for i in range(n):
+        for j in range(i, n):
+            e += q[i, j] * (x[:, i] * x[:, j])
+    assert np.array_equal(ctx.energy_fp64(q, st), e)
+
+
 @pytest.mark.parametrize("path,ground", _kats())
 def test_reference_anneal_matches_oracle_chain_on_kats(ctx, path, ground):
     q = load_qubo(path)
