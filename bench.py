@@ -40,14 +40,14 @@ PEAK_FP64_TFLOPS = 78.6    # MI355X FP64 vector
 # (FETCH_SIZE, WRITE_SIZE; KiB per dispatch) on the default configurations,
 # calibrated on a 1 GiB device copy (read bytes = 2 x FETCH_SIZE, written
 # bytes = WRITE_SIZE).  Only reported when the run uses that configuration.
-TRAFFIC_DENSE_512 = (2 * 2967756.3 + 252689.6) * 1024   # dense_sweep_kernel, 512 sweeps
+TRAFFIC_DENSE_512 = (2 * 3143382.4 + 297723.1) * 1024   # dense_sweep_kernel, 512 sweeps
 TRAFFIC_CSR_C3 = (2 * 9356018.9 + 7374460.7) * 1024     # csr_sweep_pf_kernel, 2048 sweeps
-TRAFFIC_CSR_C3_COLOUR = (2 * 20880.6 + 4838077.6) * 1024  # csr_sweep_col_kernel, 2048 sweeps
+TRAFFIC_CSR_C3_COLOUR = (2 * 31425.6 + 6311013.2) * 1024  # csr_sweep_col_kernel, 2048 sweeps
 # csr_sweep_col_kernel, one 2048-sweep launch of the config-3 batch (PMC passes): L2 requests and
 # hits, LDS instructions (wave level), LDS bank-conflict and active cycles, VALU instructions
-COUNTERS_CSR_C3_COLOUR = {"tcc_req": 6640911323.0, "tcc_hit": 6640351949.0,
-                          "sq_insts_lds": 25849097501.0, "sq_lds_bank_conflict": 88772708309.0,
-                          "sq_lds_idx_active": 143560519727.0, "sq_insts_valu": 274166665953.0}
+COUNTERS_CSR_C3_COLOUR = {"tcc_req": 7731934802.0, "tcc_hit": 7731066568.0,
+                          "sq_insts_lds": 25738079517.0, "sq_lds_bank_conflict": 83761800224.0,
+                          "sq_lds_idx_active": 137914961018.0, "sq_insts_valu": 215819107793.0}
 TRAFFIC_PASS_C5 = (2 * 107418.5 + 131072.0) * 1024      # stream_pass_kernel, 5 blocks
 TRAFFIC_INGEST_8192 = (2 * 643639.7 + 558661.2) * 1024   # parse_lines_kernel<true>, N=8192 text
 
@@ -366,13 +366,15 @@ def run_csr_c3(args):
                    "instances": 512, "replicas": R, "sweeps": S, "sum_n": int(ns.sum()),
                    "site_order": args.c3_order, "launch_shape": list(shape()),
                    "launch_shape_fields": ["waves per group", "groups",
-                                           "sites per step" if order else "kernel (1: row prefetch, 2: scheduled)"]},
+                                           "sites per step" if order else
+                                           "kernel (1: row prefetch, 2: scheduled)"]},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": PEAK_HBM_GBS, "unit": "GB/s",
                      "frac": achieved / PEAK_HBM_GBS,
-                     "traffic": (TRAFFIC_CSR_C3_COLOUR if order else TRAFFIC_CSR_C3)
-                     if S == 2048 else None,
+                     "traffic": None if S != 2048 else TRAFFIC_CSR_C3_COLOUR if order else
+                                TRAFFIC_CSR_C3 if shape()[2] == 1 else None,
                      "kernel": "csr_sweep_col_kernel" if order else
-                               "csr_sweep_sched_kernel" if shape()[2] == 2 else "csr_sweep_pf_kernel",
+                               ("csr_sweep_kernel", "csr_sweep_pf_kernel",
+                                "csr_sweep_sched_kernel")[shape()[2]],
                      "avg_launch_ms": avg_launch_s * 1e3,
                      "algorithmic_bytes_per_launch": bytes_alg},
     }
@@ -389,8 +391,8 @@ def run_csr_c3(args):
             "valu_lane_instructions_per_attempt": k["sq_insts_valu"] * 64 / (attempts / args.steps),
             "valu_wave_instructions_per_simd_cycle":
                 k["sq_insts_valu"] / avg_launch_s / (256 * 4 * 2.4e9),
-            "bound": "LDS latency per wave step (neighbour-bit gathers, 62% bank-conflict "
-                     "cycles), see profiles/csr_sweep_col_kernel_sparse512.md"}
+            "bound": "LDS latency per wave step (neighbour-bit gathers, 61% bank-conflict "
+                     "cycles), see profiles/kernel_counters.md"}
     if order:
         sites = b.colour_sites()
         res["config"]["instances_by_sites_per_step"] = {

@@ -394,8 +394,9 @@ struct BitSpins {
 // of the vector issue slots used), so the host lists the steps (no class
 // bookkeeping in the kernel), all of a row's neighbours are read before the
 // first is used (rows of one chunk have their own code) and a spin is a byte
-// where that fits.  Measured: 96 instances of 64 .. 2048 spins, degrees 3 .. 8,
-// 256 replicas, 512 sweeps 46.9 -> 36.4 ms; with bit-packed spins 42.3.
+// where that fits (kByteSpinLimit).  Measured: 96 instances of 64 .. 2048 spins,
+// degrees 3 .. 8, 256 replicas, 512 sweeps 46.9 -> 36.4 ms; with bit-packed spins
+// 42.3.  512 such instances, bit-packed, 2048 sweeps 473 -> 345 ms.
 
 // One work item of the colour-class kernel: replicas [wi.y * 64/G, +64/G) of
 // instance d, G sites per step; lds: this wave's thresholds, then its spins.

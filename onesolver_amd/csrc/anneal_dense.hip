@@ -45,7 +45,7 @@
 // lookup table for the bf16 rows: n = 60, 64 replicas, 64 sweeps 786 -> 190
 // us; 16 x n = 300, 256 sweeps 9.0 -> 4.4 ms; 4 x n = 512 replica exchange,
 // 256 sweeps 11.9 -> 7.2 ms; n = 1024, 16384 replicas, 512 sweeps 52.7 ->
-// 41.5 ms.
+// 41.5 ms (40.8 .. 45 in longer runs, depending on the card).
 //
 // Acceptance: flip iff dE < neg_ln_u(w) * tscale[t] with w the Philox word of
 // counter (j>>2, replica, sweep, tag), i.e. with probability

@@ -222,9 +222,11 @@ int sites_for(int n, int uniform, int limit) {
   return 16;
 }
 
-// Colour kernel: LDS of a wave up to which its spins take a byte each.  A mixed
-// batch of up to 2048 spins runs 42.3 ms bit-packed, 36.6 with bytes under this
-// limit and the same under 40 and 80 KB; n = 40000 only fits as bits.
+// Colour kernel: LDS of a wave up to which its spins take a byte each.  Beyond, the
+// instructions that bytes save cost more waves on a CU than they are worth: 96
+// instances whose spins take at most 16 KB a wave as bytes run 512 sweeps in 36.6
+// ms with them and 42.3 bit-packed; 512 whose largest take 17 KB run 2048 sweeps
+// in 345 ms bit-packed and 369 with bytes.
 constexpr int kByteSpinLimit = 16 * 1024;
 
 // Schedules of an instance for the scheduled index-order kernel at G = 4, 8 and
@@ -629,9 +631,10 @@ Shape select_shape(CsrBatch &b, const CsrRun &run, int site_order, bool tune_it)
     if (tune_it) {
       tune_col(b, run);
     } else {
-      // untuned: the shape the tuner picks for the mixed config-3 batch
-      // (at most 256 steps per class sweep, 2 waves per group);
-      // OS_CSR_COLOUR_LIMIT overrides the step limit
+      // untuned: a shape that the tuner picks for a batch of 512 instances of 64
+      // .. 2048 spins (at most 256 steps per class sweep, 2 waves per group: 345
+      // ms for 2048 sweeps, 345 .. 347 tuned); OS_CSR_COLOUR_LIMIT overrides the
+      // step limit
       const char *lenv = std::getenv("OS_CSR_COLOUR_LIMIT");
       const int lim = lenv ? std::atoi(lenv) : 256;
       OS_REQUIRE(!lenv || lim > 0, "OS_CSR_COLOUR_LIMIT must be a positive step count");
@@ -645,7 +648,9 @@ Shape select_shape(CsrBatch &b, const CsrRun &run, int site_order, bool tune_it)
   }
   if (b.mode == 1) col_items(b, b.c_uniform, b.c_limit);
   if (b.mode == 0 && b.seq == CsrBatch::kSched) {
-    // another replica count leaves other items, not another kernel
+    // another replica count leaves other items, not another kernel (64 instances
+    // of 500 spins, 256 sweeps, tuned at 64 replicas, run at 1024: 26 ms; the
+    // prefetching kernel in the shape tuned there takes 47)
     b.groups = std::max(1, sched_groups(b, b.s_sites));
   }
   Shape sh;
