@@ -216,12 +216,15 @@ def _ring(n, seed):
 def test_csr_tuned_index_order_matches_oracle(ctx, monkeypatch, sizes, sites):
     """The kernel that a tuned index-order run may pick updates up to 16 uncoupled
     sites together: edges of its steps and words, rows of one, two and more
-    chunks, chains it cannot pack, isolated spins, and a run that goes on with
-    another number of replicas; with each number of sites, and as tuned."""
+    chunks, chains it cannot pack, isolated spins, one and two spins, and a run
+    that goes on with another number of replicas; with each number of sites, and as tuned."""
     if sites:
         monkeypatch.setenv("OS_CSR_INDEX_SITES", str(sites))
     insts = [instances.regular_csr(n, d, seed=5, instance=i) for i, (n, d) in enumerate(sizes)]
-    insts += [_ring(50, 9), _partly_isolated(45, 20, 3)]
+    insts += [_ring(50, 9), _partly_isolated(45, 20, 3),
+              (np.zeros(2, np.int32), np.zeros(0, np.int32), np.zeros(0), np.array([-0.5])),
+              (np.array([0, 1, 2], np.int32), np.array([1, 0], np.int32), np.array([0.75, 0.75]),
+               np.array([-0.5, 0.25]))]
     S = 7
     ts = _tscale(S)
     b = onesolver_amd.CsrBatch(ctx, insts)

@@ -131,7 +131,8 @@ def _penalised(n, edges, penalty, seed):
     return adj * penalty - np.diag(w), x, e
 
 
-@pytest.mark.parametrize("n,edges", [(21, 0.5), (28, 0.5), (32, 0.5), (33, 0.5), (32, 0.3)])
+@pytest.mark.parametrize("n,edges", [(21, 0.5), (28, 0.5), (32, 0.5), (33, 0.5), (32, 0.3),
+                                     (38, 0.5)])
 @pytest.mark.parametrize("penalty", [1e3, 1e6, 1e7, 1e9, 1e13])
 def test_exhaustive_penalties_far_above_the_minimum(ctx, n, edges, penalty):
     """The walks pass through energies of the size of the penalties, so their
