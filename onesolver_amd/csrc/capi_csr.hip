@@ -10,9 +10,9 @@
 // launch shape (waves per work-group, resident work-groups, the index order's
 // kernel and sites per wave step) is picked by timing short runs of the
 // candidates on the batch itself; an untuned index-order run keeps 64 replicas
-// a wave.  Every instance is coloured
-// greedily when the batch is created (index order, smallest colour free of
-// lower-index neighbours) for the colour-class site order.
+// a wave.  Every instance is coloured greedily when the batch is created (index
+// order, smallest colour free of lower-index neighbours) for the colour-class
+// site order.
 #include <algorithm>
 #include <atomic>
 #include <cmath>
@@ -68,8 +68,9 @@ struct CsrBatch {
   int waves = 0, groups = 0;
   int seq = kPlain;
   // scheduled kernel: every instance's schedules at 4, 8 and 16 sites per step
-  // (empty before the first run that may use them), the policy in use (s_sites; 0: none tried) and its work items ((instance,
-  // group of 64/isites replicas)), built for (items_s_sites, items_s_Rp)
+  // (empty before the first run that may use them), the policy in use (s_sites; 0:
+  // none tried) and its work items ((instance, group of 64/isites replicas)),
+  // built for (items_s_sites, items_s_Rp)
   std::vector<Steps> h_sched[3];
   DevBuf sched, items_s;
   int num_items_s = 0, s_sites = 0, items_s_sites = 0, items_s_Rp = 0;
@@ -558,7 +559,8 @@ void tune(CsrBatch &b, const CsrRun &full) {
       if (maxb < 1) continue;
       std::vector<int> gpcs{maxb};
       if (maxb > 1) gpcs.push_back(std::max(1, maxb / 2));
-      for (int gpc : gpcs) take(sq, w, std::max(1, std::min(c.num_cus * gpc, (b.num_items + w - 1) / w)), 0);
+      for (int gpc : gpcs)
+        take(sq, w, std::max(1, std::min(c.num_cus * gpc, (b.num_items + w - 1) / w)), 0);
     }
   }
   OS_REQUIRE(b.waves > 0, "csr batch: no launch shape fits (instance too large for LDS)");

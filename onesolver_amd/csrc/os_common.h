@@ -83,8 +83,8 @@ __host__ __device__ __forceinline__ uint32_t pick(const uint4 &v, uint32_t i) {
 // fp32 operation, so host and device results agree bit for bit.  The bits of
 // w that make u, converted in place, are 2^32 u exactly; taking the bits of
 // 2^32 sqrt(1/2) off leaves e above the 23 mantissa bits and the offset of m
-// from sqrt(1/2) in them, so m and e cost five integer operations (the argument
-// reduction of the logarithms in FreeBSD's msun).
+// from sqrt(1/2) in them, so m and e cost five integer operations (an argument
+// reduction known from the single-precision logarithms of musl).
 __host__ __device__ __forceinline__ float neg_ln_u(uint32_t w) {
   constexpr uint32_t kSqrtHalf = 0x3F3504F3u;
   const float v = (float)((w & 0xFFFFFE00u) | 0x100u);
